@@ -29,6 +29,8 @@ CXXFLAGS = [
     "-fPIC",
     "-Wall",
     "-Wno-unused-result",
+    # mfma_tables.h computes its tables at compile time
+    "-fconstexpr-steps=100000000",
     # keep the compiler from forming packed-FP32 VALU ops
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I", os.path.join(ROOT, "include"),

@@ -37,6 +37,8 @@
 // launches over consecutive ranges of b (nothing waits across work-groups,
 // and the arrival counters work across launches).
 #pragma once
+#include <type_traits>
+
 #include "gmem.h"
 #include "hash.h"
 #include "merkle_types.h"
@@ -44,14 +46,15 @@
 
 namespace zkx {
 
-// Occupancy hint per hash type: four waves per SIMD (128 VGPRs) for Poseidon,
-// whose matrix-core leaf path keeps 36 VGPRs of coefficient operands and 48
-// of MFMA accumulators (measured on the 4 x 135 x 2^18 leaf launch: the
-// operands read from LDS inside the round loop, at five or six waves, 9%
-// slower); six waves (80 VGPRs) for Poseidon2 (8 VGPRs spilled outside the
-// round loop, and as fast as five waves without the spill); the others would
-// spill more, and keep the compiler's choice.
-constexpr int merkle_waves_per_eu(int ht) { return ht == kPoseidon ? 4 : ht == kPoseidon2 ? 6 : 1; }
+// Hashes whose whole waves run on the matrix cores, and what a work-group
+// keeps in LDS for them.
+constexpr bool has_mfma(int ht) { return ht == kPoseidon || ht == kPoseidon2; }
+template <int HT>
+using MerkleTables = std::conditional_t<has_mfma(HT), MfmaLds, uint32_t>;
+
+// Occupancy hint per hash type: four waves per SIMD (128 VGPRs) for the
+// matrix-core hashes; the others would spill, and keep the compiler's choice.
+constexpr int merkle_waves_per_eu(int ht) { return has_mfma(ht) ? 4 : 1; }
 
 // Digest slot of node `idx` of the level of width 2^lg_w in subtree `sub`.
 __device__ __forceinline__ gptr<uint64_t> node_ptr(const MerkleArgs &a, uint64_t sub, uint32_t lg_w, uint64_t idx)
@@ -70,21 +73,20 @@ __device__ __forceinline__ const MerkleArgs *find_job(const MerkleArgs *jobs, ui
     return jobs + lo;
 }
 
-// Poseidon leaf hashing by whole waves with the MDS on the matrix cores
-// (poseidon_mfma.h): wave w hashes leaves first + 64w + [0, 64), leaf
-// 32 t + j of the wave in group t, column j.  Needs whole waves (cur >= 64)
-// and leaf_size > 4; leaves are absorbed as in hash_one.  The digests land in
-// lds[leaf - first]; kt receives the round-constant table.  Every lane of the
-// work-group calls it.
-template <int TPB>
+// Poseidon and Poseidon2 leaf hashing by whole waves with the linear maps on
+// the matrix cores (poseidon_mfma.h): wave w hashes leaves first + 64w +
+// [0, 64), leaf 32 q + j of the wave in group q, column j.  Needs whole waves
+// (cur >= 64) and leaf_size > 4; leaves are absorbed as in hash_one.  The
+// digests land in lds[leaf - first]; m receives the tables.  Every lane of
+// the work-group calls it.
+template <int HT, int TPB>
 __device__ __forceinline__ void leaf_hash_mfma(const MerkleArgs &a, uint64_t first, uint32_t cur, uint64_t (*lds)[4],
-                                               uint64_t *kt)
+                                               MfmaLds &m)
 {
     const uint32_t t = threadIdx.x, w = t >> 6, j = t & 31, h = (t >> 5) & 1;
-    mfma_fill_rc(kt, t, TPB);
+    mfma_fill<HT>(m, t, TPB);
     __syncthreads();
     if (64 * w < cur) {
-        const MfmaOps o = mfma_setup();
         const uint32_t ls = a.leaf_size;
         const uint64_t cs = a.col_stride;
         uint64_t s[2][6];
@@ -101,28 +103,26 @@ __device__ __forceinline__ void leaf_hash_mfma(const MerkleArgs &a, uint64_t fir
 #pragma unroll
             for (int q = 0; q < 2; q++) {
                 const uint64_t leaf = first + 64 * w + 32 * q + j;
-                const uint32_t el0 = 6 * ((h + q) & 1);  // this lane's first element of group q
                 const gptr<const uint64_t> row = gmem(a.leaves) + leaf * a.leaf_stride;
 #pragma unroll
                 for (int e = 0; e < 6; e++) {
-                    const uint32_t k = kb + el0 + e;
-                    if (el0 + e < 8 && k < ls) {
+                    const uint32_t k = kb + 6 * h + e;
+                    if (6 * h + e < 8 && k < ls) {
                         const uint64_t v = row[(uint64_t)k * cs];
                         if (a.leaves_out) gmem(a.leaves_out)[leaf * ls + k] = v;
                         s[q][e] = v;
                     }
                 }
             }
-            poseidon_permute_mfma(s, o, kt);
+            permute_mfma<HT>(s, m);
         }
-        // elements 0-3 of group q sit in slots 0-3 of half q
+        // elements 0-3 sit on half 0: lane 32 q + j takes those of group q
 #pragma unroll
-        for (int q = 0; q < 2; q++)
-            if (h == (uint32_t)q) {
-                uint64_t *d = lds[64 * w + 32 * q + j];
-#pragma unroll
-                for (int e = 0; e < 4; e++) d[e] = gl::canon(s[q][e]);
-            }
+        for (int i = 0; i < 4; i++) {
+            uint64_t d = s[0][i], other = s[1][i];
+            swap_halves(d, other);
+            lds[t][i] = gl::canon(d);
+        }
     }
     __syncthreads();
 }
@@ -133,7 +133,7 @@ k_merkle_tile(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs on
 {
     __shared__ uint64_t lds[TPB][4];
     __shared__ uint32_t lds_last;
-    __shared__ uint64_t kt[HT == kPoseidon ? kMfmaRcWords : 1];
+    __shared__ MerkleTables<HT> tables;
     const uint32_t bid = blockIdx.x + block0;  // this work-group's tile in the whole launch list
     const MerkleArgs *job = njobs ? find_job(jobs, njobs, bid) : nullptr;
     const MerkleArgs a = njobs ? *job : one;
@@ -144,9 +144,9 @@ k_merkle_tile(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs on
     uint64_t first = ((uint64_t)bid - a.tile_begin) << a.tile_log;  // first node of the tile
 
     uint64_t h[4];
-    const bool mfma = HT == kPoseidon && cur >= 64 && a.leaf_size > 4 && !a.leaf_valu;
-    if constexpr (HT == kPoseidon)
-        if (mfma) leaf_hash_mfma<TPB>(a, first, cur, lds, kt);
+    const bool mfma = has_mfma(HT) && cur >= 64 && a.leaf_size > 4 && !(HT == kPoseidon && a.leaf_valu);
+    if constexpr (has_mfma(HT))
+        if (mfma) leaf_hash_mfma<HT, TPB>(a, first, cur, lds, tables);
     if (t < cur) {
         const uint64_t g = first + t;
         const uint64_t sub = g >> lg_w, idx = g & ((1ull << lg_w) - 1);
@@ -300,7 +300,7 @@ template <int HT>
 __global__ void __launch_bounds__(kMerkleLevelLanes) __attribute__((amdgpu_waves_per_eu(merkle_waves_per_eu(HT))))
 k_merkle_level(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs one, uint32_t block0)
 {
-    __shared__ uint64_t kt[HT == kPoseidon ? kMfmaRcWords : 1];
+    __shared__ MerkleTables<HT> tables;
     const uint32_t bid = blockIdx.x + block0;
     const MerkleArgs a = njobs ? *find_job(jobs, njobs, bid) : one;
     const uint32_t t = threadIdx.x, lw = a.lg_w;
@@ -310,25 +310,27 @@ k_merkle_level(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs o
     auto children = [&](uint64_t g) { return node_ptr(a, g >> lw, lw + 1, 2 * (g & wmask)); };
     const uint64_t g = g0 + t;
     uint64_t out[4];
-    if constexpr (HT == kPoseidon) {
-        mfma_fill_rc(kt, t, kMerkleLevelLanes);
+    if constexpr (has_mfma(HT)) {
+        mfma_fill<HT>(tables, t, kMerkleLevelLanes);
         __syncthreads();
         const uint32_t w = t >> 6, j = t & 31, h = (t >> 5) & 1;
-        const MfmaOps o = mfma_setup();
         uint64_t s[2][6];
 #pragma unroll
         for (int q = 0; q < 2; q++) {
             const uint64_t n = g0 + 64 * w + 32 * q + j;
-            const uint32_t el0 = 6 * ((h + q) & 1);  // this lane's first element of group q
-            const bool real = n < a.count;           // lanes past the level's end hash zeros
+            const bool real = n < a.count;  // lanes past the level's end hash zeros
             const gptr<const uint64_t> c = children(real ? n : 0);
 #pragma unroll
-            for (int e = 0; e < 6; e++) s[q][e] = real && el0 + e < 8 ? c[el0 + e] : 0;
+            for (int e = 0; e < 6; e++) s[q][e] = real && 6 * h + e < 8 ? c[6 * h + e] : 0;
         }
-        poseidon_permute_mfma(s, o, kt);
-        // elements 0-3 of group h sit in slots 0-3 of this lane: node g0 + 64w + 32h + j = g
+        permute_mfma<HT>(s, tables);
+        // elements 0-3 sit on half 0: lane 32 q + j takes those of group q
 #pragma unroll
-        for (int i = 0; i < 4; i++) out[i] = gl::canon(h ? s[1][i] : s[0][i]);
+        for (int i = 0; i < 4; i++) {
+            uint64_t d = s[0][i], other = s[1][i];
+            swap_halves(d, other);
+            out[i] = gl::canon(d);
+        }
     } else {
         if (g < a.count) {
             const gptr<const uint64_t> c = children(g);

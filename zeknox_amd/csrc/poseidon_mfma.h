@@ -1,192 +1,382 @@
-// Poseidon (Goldilocks, width 12; poseidon/poseidon.cu:563-838) with the MDS
-// layer on the matrix cores, for leaf hashing by whole waves.
+// Poseidon and Poseidon2 (Goldilocks, width 12; poseidon/poseidon.cu:563-838,
+// poseidon2/poseidon2.cu:65-209) with every linear map on the matrix cores,
+// 64 permutations per wave.
 //
-// The MDS is a 12 x 12 matrix with small coefficients applied to every
-// permutation of a wave: a batch of matrix-vector products.  Its integer
-// form is exact on the i8 MFMA once the 64-bit elements are cut into their
-// 8 bytes: with u_{C,b} the b-th byte of element C,
-//   y_R = sum_C CIRC[(C - R) mod 12] x_C = sum_b 2^(8b) D_b[R],
-//   D_b[R] = sum_C CIRC[(C - R) mod 12] u_{C,b}  (< 2^16),
-// so one MFMA output row per (output element, byte) and a block-diagonal
-// coefficient matrix (byte b of an input pairs only with row byte b).  The
-// vector unit then only recombines eight partials per element, instead of
-// 24 multiply-adds per element.
+// The maps between S-boxes (mfma_tables.h) are exact integer products of
+// bytes: the state's 64-bit slots are cut into their 8 bytes, a coefficient
+// and a byte give eight signed digits, and v_mfma_i32_32x32x32_i8 sums them.
+// The vector unit recombines eight digit sums per output element.
 //
-// Wave layout.  Two lanes hold one permutation, six elements each; a wave
-// holds two groups t of 32 permutations.  Lane l (column j = l & 31, half
-// h = l >> 5) holds, for group t, the elements
-//   E(t, h, e) = 6 ((h + t) mod 2) + e,  e = 0..5,
-// of permutation (t, j).  v_mfma_i32_32x32x32_i8 (gfx950, layout measured)
-// computes D[i][j] = sum_{h, q} A_{32h+i}[q] * B_{32h+j}[q] over the 16
-// bytes q each lane supplies, and lane 32h' + j receives D[i][j] for
-// i = 8k + 4h' + r in its register 4k + r.  So lane (j, h) supplies slots
-// 2kappa, 2kappa + 1 as B of K-chunk kappa (0..2, chained in place), and
-// M-block beta (0..2) row 8k + 4h' + r is output element
-// E(t, h', 2 beta + k / 2), byte 4 (k % 2) + r: every lane receives the
-// eight byte partials of exactly its own six output elements.  The
-// coefficient of that row and input slot e of half h is
-//   CIRC[(6 (h - h') + e - 2 beta - k / 2) mod 12]
-// for both groups (the rotation by 6t cancels in a circulant), so one set of
-// A operands (9 x 4 VGPRs) serves both.  Element 0 of group t sits in half
-// t: in a partial round each lane applies exactly one S-box.  MDS_DIAG (8 on
-// element 0) is added on the vector unit by the lanes that hold element 0.
-// (Measured on gfx950 beside full-rate vector work: 18 of these MFMAs per
-// round cost about half the issue time of 48 16x16x64 ones doing the same
-// products.  Accumulator chains stay within one opcode, in place: a
-// 16x16x64 result taken as the accumulator of a 16x16x32 product, issued
-// with no wait states between them, came out wrong.)
+// Wave layout.  A wave holds two groups t of 32 permutations, two lanes per
+// permutation: lane l (column j = l & 31, half h = l >> 5) holds elements
+// 6h..6h + 5 of permutation (t, j).  v_mfma_i32_32x32x32_i8 (gfx950, layout
+// measured) computes D[i][j] = sum_{h, q} A_{32h+i}[q] * B_{32h+j}[q] over
+// the 16 bytes q each lane supplies, and lane 32h' + j receives D[i][j] for
+// i = 8k + 4h' + r in its register 4k + r.  So a lane supplies its own slots
+// as B, and with the rows ordered by M-block as in mfma_tables.h it receives
+// the eight digit sums of its own elements 2 beta, 2 beta + 1.
 //
-// Signed bytes.  The MFMA takes signed i8: the state enters XORed with 0x80
-// in every byte (u - 128), so D_b = (byte-plane sum) - 128 * 256, in
-// [-32768, 32512]; the 32768 per byte plane goes back in with the folded
-// round constants (below), which keeps every partial sum non-negative.
+// Partial rounds.  A group of five: the sums of x_2..x_5 come first (one
+// M-block: x_2, x_3 on half 0 and x_4, x_5 on half 1, for both groups), and
+// v_permlane32_swap hands each lane those of one permutation, (h, j): every
+// lane then runs one permutation's five S-boxes, adding the earlier outputs
+// of the group itself (h_{j-i} y_i), swaps the outputs back into their slots
+// and the group's map gives the next state.  One recombination of twelve
+// elements per five rounds instead of one per round: 12 layers of vector
+// work instead of 30.
+//
+// Bound: VALU issue (1.07 of one wave instruction per 4 cycles per SIMD, the
+// MFMAs beside it).  Against one layer per round (the MDS on the matrix
+// cores for Poseidon, everything on the VALU for Poseidon2), wave
+// instructions per leaf permutation: Poseidon 205 -> 153 VALU, 8.4 -> 4.3
+// MFMA; Poseidon2 234 -> 162 VALU.  Leaf launch of 32 x 2^18 leaves of 135:
+// 56.4 -> 41.0 ms; of 2^21 leaves of 400 with Poseidon2: 36 -> 31.7 ms.
+// Five rounds: the map of four leaves a K-chunk unused and costs as much; six
+// needs a fifth chunk and weights beyond 32 bits.
 //
 // Recombination (per output element, lazy in and out, as hash.h):
 //   L = KL + (D0 + 2^8 D1) + 2^16 (D2 + 2^8 D3),  H = KH + (same on D4..D7),
-// with KL, KH = the low and high 32 bits of the next round's constant plus
-// 32768 * (1 + 2^8 + 2^16 + 2^24) each, then limb_combine(L, H)
-// (0 <= L, H < 2^42).  The chains run in signed 32x32+64 multiply-adds.
+// with KL, KH the map's constant pair (which keeps both non-negative), then
+// limb_combine(L, H) (0 <= L, H < 2^47).  The chains run in signed 32x32+64
+// multiply-adds.
+//
+// (Accumulator chains stay within one opcode, in place: a 16x16x64 result
+// taken as the accumulator of a 16x16x32 product, issued with no wait states
+// between them, came out wrong.)
 #pragma once
 #include "hash.h"
+#include "mfma_tables.h"
 
 namespace zkx {
 
 typedef int mf_v4i __attribute__((ext_vector_type(4)));
 typedef int mf_v16i __attribute__((ext_vector_type(16)));
 
-static __constant__ uint32_t c_poseidon_circ[12] = {ZK_POSEIDON_MDS_CIRC_LIST};
+// The tables in device memory; kernels that do not hash with HT never name
+// them, so each translation unit holds its own hash's alone.
+template <int HT>
+__device__ const mfma::Tables c_mfma = mfma::make<HT>();
 
-// Round-constant table in LDS: row r (0..30), element E -> {lo32, hi32} of
-// c_poseidon_rc[r][E], each widened to u64 (a multiply-add addend pair).
-constexpr int kMfmaRcWords = 31 * 12 * 2;
-
-// 32768 per byte plane of one 32-bit half: 32768 * (1 + 2^8 + 2^16 + 2^24)
-constexpr uint64_t kMfmaPlaneBias = 32768ull * 0x01010101ull;
-
-// Row 0 holds the first round's constants as they are (added before the
-// first S-box); rows 1..30 also carry kMfmaPlaneBias in each half.
-__device__ __forceinline__ void mfma_fill_rc(uint64_t *kt, uint32_t t, uint32_t nthreads)
-{
-    for (uint32_t i = t; i < 31 * 12; i += nthreads) {
-        const uint64_t c = c_poseidon_rc[i], b = i < 12 ? 0 : kMfmaPlaneBias;
-        kt[2 * i] = gl::lo32(c) + b;
-        kt[2 * i + 1] = gl::hi32(c) + b;
-    }
-}
-
-struct MfmaOps {
-    mf_v4i a[3][3];  // coefficient operands [M-block beta][K-chunk kappa]
-    uint32_t h;      // lane half
+// What a work-group keeps of them in LDS: the operands used all the time
+// (24 KiB) and the constant rows.
+struct MfmaLds {
+    mf_v4i op[mfma::kOpsLds][64];
+    uint64_t row[mfma::kRows][12][2];
 };
 
-__device__ __forceinline__ MfmaOps mfma_setup()
+template <int HT>
+__device__ __forceinline__ void mfma_fill(MfmaLds &m, uint32_t t, uint32_t nthreads)
 {
-    MfmaOps o;
-    const uint32_t l = threadIdx.x & 63, i = l & 31, h = l >> 5, k = i >> 3, hp = (i >> 2) & 1, r = i & 3;
-    const uint32_t sh = 8 * (4 * (k & 1) + r);  // bit offset of the row's byte within a slot
-    o.h = h;
-#pragma unroll
-    for (int beta = 0; beta < 3; beta++)
-#pragma unroll
-        for (int kappa = 0; kappa < 3; kappa++) {
-            uint64_t w[2];
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const uint32_t c = (6 * (h + 2 - hp) + 2 * kappa + u + 12 - 2 * beta - (k >> 1)) % 12;
-                w[u] = (uint64_t)c_poseidon_circ[c] << sh;
-            }
-            o.a[beta][kappa] = mf_v4i{(int)gl::lo32(w[0]), (int)gl::hi32(w[0]), (int)gl::lo32(w[1]), (int)gl::hi32(w[1])};
-        }
-    return o;
+    const mf_v4i *ops = reinterpret_cast<const mf_v4i *>(c_mfma<HT>.op);
+    for (uint32_t i = t; i < mfma::kOpsLds * 64; i += nthreads) m.op[0][i] = ops[i];
+    const uint64_t *rows = &c_mfma<HT>.row[0][0].l;
+    for (uint32_t i = t; i < mfma::kRows * 24; i += nthreads) m.row[0][0][i] = rows[i];
 }
 
-// Lanes of half t hold element 0 of group t.
-__device__ __forceinline__ bool mfma_own(uint32_t h, int t) { return h == (uint32_t)t; }
-
-// s <- MDS * s + RC[row] (krow: the next round's row of the LDS table).
-__device__ __forceinline__ void mds_mfma(uint64_t s[2][6], const MfmaOps &o, const uint64_t *krow)
+// Exchanges the upper half of a with the lower half of b: a becomes
+// (a of half 0, b of half 0), b becomes (a of half 1, b of half 1).
+// v_permlane32_swap_b32 needs two wait states after a VALU write of its
+// operands; the compiler does not count the writes of inline asm (the
+// reductions of gl64.h end in one), so the wait is part of the block.
+__device__ __forceinline__ void swap_halves(uint64_t &a, uint64_t &b)
 {
-    constexpr uint64_t XM = 0x8080808080808080ull;
+    uint32_t a0 = gl::lo32(a), a1 = gl::hi32(a), b0 = gl::lo32(b), b1 = gl::hi32(b);
+    asm("s_nop 1\n\t"
+        "v_permlane32_swap_b32 %[a0], %[b0]\n\t"
+        "v_permlane32_swap_b32 %[a1], %[b1]"
+        : [a0] "+v"(a0), [a1] "+v"(a1), [b0] "+v"(b0), [b1] "+v"(b1));
+    a = gl::pack(a0, a1);
+    b = gl::pack(b0, b1);
+}
+__device__ __forceinline__ void swap_halves(uint32_t (&a)[4], uint32_t (&b)[4])
+{
+    asm("s_nop 1\n\t"
+        "v_permlane32_swap_b32 %[a0], %[b0]\n\t"
+        "v_permlane32_swap_b32 %[a1], %[b1]\n\t"
+        "v_permlane32_swap_b32 %[a2], %[b2]\n\t"
+        "v_permlane32_swap_b32 %[a3], %[b3]"
+        : [a0] "+v"(a[0]), [a1] "+v"(a[1]), [a2] "+v"(a[2]), [a3] "+v"(a[3]), [b0] "+v"(b[0]), [b1] "+v"(b[1]),
+          [b2] "+v"(b[2]), [b3] "+v"(b[3]));
+}
+
+// A slot's bytes as the MFMA takes them (u - 128, signed).
+__device__ __forceinline__ uint64_t mfma_bytes(uint64_t x) { return x ^ 0x8080808080808080ull; }
+
+__device__ __forceinline__ mf_v4i mfma_pair(uint64_t x0, uint64_t x1)
+{
+    return mf_v4i{(int)gl::lo32(x0), (int)gl::hi32(x0), (int)gl::lo32(x1), (int)gl::hi32(x1)};
+}
+
+// D0 + 2^8 D1 of two digit sums.
+__device__ __forceinline__ uint32_t digit_pair(int d0, int d1) { return (uint32_t)d0 + ((uint32_t)d1 << 8); }
+
+// Keeps the operands of an MFMA chain in their registers until p, computed
+// from the chain's result, is there.  A register of a chain's A operand
+// overwritten by a v_mov right after the MFMA that reads it gave wrong sums
+// whenever another wave held the SIMD's matrix pipe (the second group of a
+// wave, at two or more waves per SIMD): the compiler lets go of the operands
+// as soon as the instruction is issued, and it reads them later than that.
+template <int NK>
+__device__ __forceinline__ void hold_operands(const mf_v4i (&a)[NK], const mf_v4i (&b)[NK], uint32_t p)
+{
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        mf_v4i b[3];
+    for (int kappa = 0; kappa < NK; kappa++) asm volatile("; hold %0 %1 %2" ::"v"(p), "v"(a[kappa]), "v"(b[kappa]));
+}
+
+// p01 + 2^16 p23 + k, in signed multiply-adds.
+__device__ __forceinline__ uint64_t half_sum(uint32_t p01, uint32_t p23, uint64_t k)
+{
+    const int64_t one = (int32_t)gl::opaque(1u), m16 = (int32_t)gl::opaque(65536u);
+    const uint64_t s = gl::vopaque64((uint64_t)((int64_t)(int32_t)p01 * one + (int64_t)k));
+    return gl::vopaque64((uint64_t)((int64_t)(int32_t)p23 * m16 + (int64_t)s));
+}
+
+// s <- the map with operands `op` (this lane's, [M-block][K-chunk] 64 lanes
+// apart) on the slots b, plus the constants `row` of this lane's elements.
+template <int NK>
+__device__ __forceinline__ void mfma_map(uint64_t s[2][6], const mf_v4i (&b)[2][NK], const mf_v4i *op,
+                                         const uint64_t (*row)[2])
+{
+    // one M-block and group at a time, recombined as soon as its chain is
+    // done: 16 accumulator VGPRs live
 #pragma unroll
-        for (int kappa = 0; kappa < 3; kappa++) {
-            const uint64_t x0 = s[t][2 * kappa] ^ XM, x1 = s[t][2 * kappa + 1] ^ XM;
-            b[kappa] = mf_v4i{(int)gl::lo32(x0), (int)gl::hi32(x0), (int)gl::lo32(x1), (int)gl::hi32(x1)};
-        }
-        const bool own = mfma_own(o.h, t);
-        const uint32_t dl = own ? gl::lo32(s[t][0]) : 0u, dh = own ? gl::hi32(s[t][0]) : 0u;
-        const uint64_t *k = krow + 12 * ((o.h + t) & 1);
-        // one M-block at a time, recombined as soon as its chain is done: 16
-        // accumulator VGPRs live instead of 48 (the operands b and dl, dh
-        // hold what the later blocks need of the old state)
+    for (int beta = 0; beta < 3; beta++) {
+        mf_v4i a[NK];
 #pragma unroll
-        for (int beta = 0; beta < 3; beta++) {
-            mf_v16i dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[beta][0], b[0], mf_v16i{}, 0, 0, 0);
-            dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[beta][1], b[1], dd, 0, 0, 0);
-            dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[beta][2], b[2], dd, 0, 0, 0);
+        for (int kappa = 0; kappa < NK; kappa++) a[kappa] = op[(beta * NK + kappa) * 64];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            mf_v16i dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[0], b[t][0], mf_v16i{}, 0, 0, 0);
+#pragma unroll
+            for (int kappa = 1; kappa < NK; kappa++)
+                dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[kappa], b[t][kappa], dd, 0, 0, 0);
+            hold_operands<NK>(a, b[t], digit_pair(dd[0], dd[1]));
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                const int e = 2 * beta + u;
-                const int q = 8 * u;  // registers q..q+3: bytes 0-3, q+4..q+7: bytes 4-7
-                const int32_t p01 = dd[q] + (int32_t)((uint32_t)dd[q + 1] << 8);
-                const int32_t p23 = dd[q + 2] + (int32_t)((uint32_t)dd[q + 3] << 8);
-                const int32_t q01 = dd[q + 4] + (int32_t)((uint32_t)dd[q + 5] << 8);
-                const int32_t q23 = dd[q + 6] + (int32_t)((uint32_t)dd[q + 7] << 8);
-                const int64_t one = (int32_t)gl::opaque(1u), m16 = (int32_t)gl::opaque(65536u);
-                uint64_t L = gl::vopaque64((uint64_t)((int64_t)p01 * one + (int64_t)k[2 * e]));
-                uint64_t H = gl::vopaque64((uint64_t)((int64_t)q01 * one + (int64_t)k[2 * e + 1]));
-                if (e == 0) {
-                    L = gl::vopaque64((uint64_t)dl * gl::opaque(8u) + L);
-                    H = gl::vopaque64((uint64_t)dh * gl::opaque(8u) + H);
-                }
-                L = gl::vopaque64((uint64_t)((int64_t)p23 * m16 + (int64_t)L));
-                H = gl::vopaque64((uint64_t)((int64_t)q23 * m16 + (int64_t)H));
+                const int e = 2 * beta + u, q = 8 * u;
+                const uint64_t L = half_sum(digit_pair(dd[q], dd[q + 1]), digit_pair(dd[q + 2], dd[q + 3]), row[e][0]);
+                const uint64_t H =
+                    half_sum(digit_pair(dd[q + 4], dd[q + 5]), digit_pair(dd[q + 6], dd[q + 7]), row[e][1]);
                 s[t][e] = limb_combine(L, H);
             }
         }
     }
 }
 
-// The permutation of 64 states (layout above); kt: the LDS round-constant
-// table.  Lazy in and out.  All 64 lanes of the wave must be active.
-__device__ __forceinline__ void poseidon_permute_mfma(uint64_t s[2][6], const MfmaOps &o, const uint64_t *kt)
+// The digit pairs of the outputs of one M-block: x[t][u] for this lane's
+// half, swapped so that x[h'][u] is output 2h' + u of permutation (h, j).
+__device__ __forceinline__ void mfma_outputs(uint32_t (&x)[2][2][4], const mf_v4i (&b)[2][3], const mf_v4i *op)
 {
+    mf_v4i a[3];
+#pragma unroll
+    for (int kappa = 0; kappa < 3; kappa++) a[kappa] = op[kappa * 64];
 #pragma unroll
     for (int t = 0; t < 2; t++) {
-        const uint64_t *k = kt + 12 * ((o.h + t) & 1);
+        mf_v16i dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[0], b[t][0], mf_v16i{}, 0, 0, 0);
+        dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[1], b[t][1], dd, 0, 0, 0);
+        dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[2], b[t][2], dd, 0, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 6; e++) s[t][e] = gl::add(s[t][e], gl::pack(gl::lo32(k[2 * e]), gl::lo32(k[2 * e + 1])));
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int n = 0; n < 4; n++) x[t][u][n] = digit_pair(dd[8 * u + 2 * n], dd[8 * u + 2 * n + 1]);
+        hold_operands<3>(a, b[t], x[t][0][0]);
     }
-    // rounds 0-3 and 26-29 full, 4-25 partial (two per iteration)
+#pragma unroll
+    for (int u = 0; u < 2; u++) swap_halves(x[0][u], x[1][u]);
+}
+
+// An S-box input: the recombined output (digit pairs d, constant k) plus
+// sum_i h[m - i] y[i] over the m earlier outputs of its group.  Weights below
+// 2^32 enter the recombination as multiply-adds of the output's halves (their
+// sum is below 2^30); larger ones as lazy products.
+template <int HT>
+constexpr uint64_t mfma_h(int m)
+{
+    constexpr auto h = mfma::partial_weights<HT>();
+    return h.v[m];
+}
+
+template <int HT>
+constexpr uint64_t mfma_h_sum()
+{
+    uint64_t s = 0;
+    for (int m = 1; m < mfma::kGroupRounds; m++)
+        if (mfma_h<HT>(m) < (1ull << 32)) s += mfma_h<HT>(m);
+    return s;
+}
+static_assert(mfma_h_sum<kPoseidon>() < (1ull << 30) && mfma_h_sum<kPoseidon2>() < (1ull << 30),
+              "2^47 + sum of weights * 2^32 stays below 2^63");
+
+template <int HT, int M, int I>
+__device__ __forceinline__ void add_earlier_small(uint64_t &L, uint64_t &H, const uint64_t *y)
+{
+    if constexpr (I < M) {
+        constexpr uint64_t w = mfma_h<HT>(M - I);
+        if constexpr (w < (1ull << 32)) {
+            L = gl::vopaque64((uint64_t)gl::lo32(y[I]) * gl::opaque((uint32_t)w) + L);
+            H = gl::vopaque64((uint64_t)gl::hi32(y[I]) * gl::opaque((uint32_t)w) + H);
+        }
+        add_earlier_small<HT, M, I + 1>(L, H, y);
+    }
+}
+
+// x + w * y, lazy.  The sum added to the product's low word carries at most 1
+// into the high word, and the total stays below (2^64 - 1)^2 + 2^64, so the
+// high word plus the product's carry fits 64 bits.
+__device__ __forceinline__ uint64_t mul_add_lazy(uint64_t y, uint64_t w, uint64_t x)
+{
+    uint64_t lo, hi, pc;
+    gl::mul128c(y, w, lo, hi, pc);
+    uint32_t c1, c2, c3, c4;
+    const uint32_t l0 = __builtin_addc(gl::lo32(lo), gl::lo32(x), 0u, &c1);
+    const uint32_t l1 = __builtin_addc(gl::hi32(lo), gl::hi32(x), c1, &c2);
+    const uint32_t h0 = __builtin_addc(gl::lo32(hi), 0u, c2, &c3);
+    const uint32_t h1 = __builtin_addc(gl::hi32(hi), 0u, c3, &c4);
+    return gl::reduce128c_lazy(gl::pack(l0, l1), gl::pack(h0, h1), pc);
+}
+
+template <int HT, int M, int I>
+__device__ __forceinline__ void add_earlier_large(uint64_t &x, const uint64_t *y)
+{
+    if constexpr (I < M) {
+        constexpr uint64_t w = mfma_h<HT>(M - I);
+        if constexpr (w >= (1ull << 32)) x = mul_add_lazy(y[I], w, x);
+        add_earlier_large<HT, M, I + 1>(x, y);
+    }
+}
+
+template <int HT, int M>
+__device__ __forceinline__ uint64_t sbox_input(const uint32_t (&d)[4], const mfma::Pair &k, const uint64_t *y)
+{
+    uint64_t L = half_sum(d[0], d[1], k.l), H = half_sum(d[2], d[3], k.h);
+    add_earlier_small<HT, M, 0>(L, H, y);
+    uint64_t x = limb_combine(L, H);
+    add_earlier_large<HT, M, 0>(x, y);
+    return x;
+}
+
+__device__ __forceinline__ void mfma_sboxes(uint64_t s[2][6])
+{
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int e = 0; e < 6; e += 2) gl::pow7_lazy2(s[t][e], s[t][e + 1]);
+}
+
+// This lane's slots 0..11 as B operands.
+template <int NK>
+__device__ __forceinline__ void mfma_state(mf_v4i (&b)[2][NK], const uint64_t s[2][6])
+{
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int kappa = 0; kappa < 3; kappa++)
+            b[t][kappa] = mfma_pair(mfma_bytes(s[t][2 * kappa]), mfma_bytes(s[t][2 * kappa + 1]));
+}
+
+// The permutation of 64 states (layout above); m: the work-group's tables.
+// Lazy in and out.  All 64 lanes of the wave must be active.
+template <int HT>
+__device__ __forceinline__ void permute_mfma(uint64_t s[2][6], const MfmaLds &m)
+{
+    using namespace mfma;
+    const uint32_t l = threadIdx.x & 63, h = l >> 5;
+    // the tables through an offset the compiler cannot see through: operands
+    // are read where they are used, not kept in registers across rounds
+    auto tables = [&](const mf_v4i *&op, const uint64_t (*&row)[12][2]) {
+        uint32_t lane = l, half = h;
+        asm volatile("; tables %0 %1" : "+v"(lane), "+v"(half));
+        op = &m.op[0][lane];
+        row = reinterpret_cast<const uint64_t(*)[12][2]>(&m.row[0][6 * half][0]);
+    };
+    auto full_layer = [&](int r) {
+        const mf_v4i *op;
+        const uint64_t(*row)[12][2];
+        tables(op, row);
+        mf_v4i b[2][3];
+        mfma_state(b, s);
+        mfma_map<3>(s, b, op + 64 * kOpLayer, row[r]);
+    };
+    if constexpr (HT == kPoseidon) {
+#pragma unroll
+        for (int e = 0; e < 6; e++) {
+            const uint64_t k = m.row[kRowFirst][6 * h + e][0];
+#pragma unroll
+            for (int t = 0; t < 2; t++) s[t][e] = gl::add(s[t][e], k);
+        }
+    } else {
+        full_layer(kRowFirst);
+    }
+#pragma unroll 1
+    for (int r = 0; r < 3; r++) {
+        mfma_sboxes(s);
+        full_layer(kRowFull + r);
+    }
+    mfma_sboxes(s);
+    {  // full round 3's layer and partial rounds 4, 5
+        const mf_v4i *op;
+        const uint64_t(*row)[12][2];
+        tables(op, row);
+        const mf_v4i *eop = reinterpret_cast<const mf_v4i *>(c_mfma<HT>.op) + l;
+        mf_v4i b3[2][3];
+        mfma_state(b3, s);
+        uint32_t x[2][2][4];
+        mfma_outputs(x, b3, eop + 64 * kOpEntryX);
+        uint64_t y[2];
+        y[0] = gl::pow7_lazy(sbox_input<HT, 0>(x[0][0], c_mfma<HT>.x_entry[0], y));
+        y[1] = gl::pow7_lazy(sbox_input<HT, 1>(x[1][0], c_mfma<HT>.x_entry[1], y));
+        uint64_t y1 = mfma_bytes(y[0]), y2 = mfma_bytes(y[1]);
+        swap_halves(y1, y2);
+        mf_v4i b[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+#pragma unroll
+            for (int kappa = 0; kappa < 3; kappa++) b[t][kappa] = b3[t][kappa];
+            b[t][3] = mfma_pair(t ? y2 : y1, 0);
+        }
+        mfma_map<4>(s, b, eop + 64 * kOpEntry, row[kRowEntry]);
+    }
+#pragma unroll 1
+    for (int g = 0; g < kGroups; g++) {  // five partial rounds each
+        const mf_v4i *op;
+        const uint64_t(*row)[12][2];
+        tables(op, row);
+        mf_v4i b3[2][3];
+        mfma_state(b3, s);
+        uint32_t x[2][2][4];
+        mfma_outputs(x, b3, op + 64 * kOpGroupX);
+        // element 0 of permutation (h, j), and element 6 of both groups
+        uint64_t x1 = s[0][0], e6 = s[1][0];
+        swap_halves(x1, e6);
+        const Pair *k = c_mfma<HT>.x_group[g];
+        uint64_t y[5];
+        y[0] = gl::pow7_lazy(x1);
+        y[1] = gl::pow7_lazy(sbox_input<HT, 1>(x[0][0], k[0], y));
+        y[2] = gl::pow7_lazy(sbox_input<HT, 2>(x[0][1], k[1], y));
+        y[3] = gl::pow7_lazy(sbox_input<HT, 3>(x[1][0], k[2], y));
+        y[4] = gl::pow7_lazy(sbox_input<HT, 4>(x[1][1], k[3], y));
+#pragma unroll
+        for (int i = 0; i < 5; i++) y[i] = mfma_bytes(y[i]);
+        e6 = mfma_bytes(e6);
+        swap_halves(y[0], e6);    // slot 0: y_1 on half 0, element 6 on half 1
+        swap_halves(y[1], y[3]);  // slots 12, 14
+        swap_halves(y[2], y[4]);  // slots 13, 15
+        mf_v4i b[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+#pragma unroll
+            for (int kappa = 0; kappa < 3; kappa++) b[t][kappa] = b3[t][kappa];
+            const uint64_t s0 = t ? e6 : y[0];
+            b[t][0][0] = (int)gl::lo32(s0);
+            b[t][0][1] = (int)gl::hi32(s0);
+            b[t][3] = mfma_pair(t ? y[3] : y[1], t ? y[4] : y[2]);
+        }
+        mfma_map<4>(s, b, op + 64 * kOpGroup, row[kRowGroup + g]);
+    }
 #pragma unroll 1
     for (int r = 0; r < 4; r++) {
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int e = 0; e < 6; e += 2) gl::pow7_lazy2(s[t][e], s[t][e + 1]);
-        mds_mfma(s, o, kt + 24 * (r + 1));
-    }
-#pragma unroll 1
-    for (int r = 4; r < 26; r += 2) {
-#pragma unroll
-        for (int hh = 0; hh < 2; hh++) {
-            // each lane holds element 0 of exactly one group
-            uint64_t x = mfma_own(o.h, 1) ? s[1][0] : s[0][0];
-            x = gl::pow7_lazy(x);
-            s[0][0] = mfma_own(o.h, 0) ? x : s[0][0];
-            s[1][0] = mfma_own(o.h, 1) ? x : s[1][0];
-            mds_mfma(s, o, kt + 24 * (r + hh + 1));
-        }
-    }
-#pragma unroll 1
-    for (int r = 26; r < 30; r++) {
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int e = 0; e < 6; e += 2) gl::pow7_lazy2(s[t][e], s[t][e + 1]);
-        mds_mfma(s, o, kt + 24 * (r + 1));
+        mfma_sboxes(s);
+        full_layer(kRowLast + r);
     }
 }
 
