@@ -1,6 +1,6 @@
-"""Whole-wave Poseidon and Poseidon2 permutations (linear maps on the matrix
-cores) against the oracle, at the edges of their chunks and tiles and with
-every SIMD busy.  Bit-exact (tolerance zero)."""
+"""Poseidon and Poseidon2 permutations with their linear maps on the matrix
+cores (64 and 16 per wave) against the oracle, at the edges of their chunks,
+tiles and size rules and with every SIMD busy.  Bit-exact (tolerance zero)."""
 import numpy as np
 import pytest
 
@@ -10,10 +10,19 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("ht", [0, 3])
-@pytest.mark.parametrize("lg_l,ls,h", [(6, 5, 6),      # one wave, part of one chunk, no levels
+@pytest.mark.parametrize("lg_l,ls,h", [(0, 9, 0),      # 16 per wave: one leaf
+                                       (1, 4, 0),      # leaves hashed as they are, one level
+                                       (3, 17, 1),
+                                       (4, 1, 4),
+                                       (6, 5, 6),      # one tile, part of one chunk, no levels
                                        (6, 8, 0),      # exactly one chunk
                                        (7, 9, 2),      # one element in the second chunk
-                                       (9, 135, 3),
+                                       (9, 135, 3),    # an upper pass
+                                       (14, 6, 0),     # two upper passes
+                                       (15, 12, 4),    # the largest built in one launch
+                                       (16, 10, 4),    # 64 per wave, every level 16 per wave
+                                       (16, 3, 16),    # no levels
+                                       (17, 6, 4),     # the first level 64 per wave
                                        (17, 7, 17),    # two waves on every SIMD, leaves only
                                        (18, 13, 18),   # four waves on every SIMD
                                        (18, 5, 2)])    # and the levels above them
@@ -68,3 +77,29 @@ def test_batch_levels(zk, ht, tile_log):
         assert np.array_equal(leaves, want)
         assert np.array_equal(caps, ecap)
         assert np.array_equal(dig, edig)
+
+
+@pytest.mark.parametrize("ht", [0, 3])
+@pytest.mark.parametrize("shapes", [[(5, 2, 1, 0), (3, 3, 1, 4), (9, 6, 2, 8), (17, 9, 3, 1)],  # 16 per wave, whole
+                                    [(6, 13, 2, 2), (3, 13, 2, 15), (9, 4, 1, 0)],               # every level 16 per wave
+                                    [(5, 15, 2, 4), (9, 3, 1, 0)]])                              # the first one 64 per wave
+def test_batch_forests(zk, ht, shapes):
+    """Trees of several sizes in one batch, three times over (the third call
+    replays a captured graph): arrival counters return to zero."""
+    zk.init_coset_rs(0, max(n + r for _, n, r, _ in shapes), 7)
+    jobs = []
+    for k, (cols, lg_n, rate, cap) in enumerate(shapes):
+        coeffs = ob.canonical(cols << lg_n, 300 + k)
+        jobs.append((zk.Commit(coeffs, cols, lg_n, rate, cap, ht), coeffs, cols, lg_n, rate, cap))
+    want = []
+    for _, coeffs, cols, lg_n, rate, cap in jobs:
+        rows = ob.transpose_rev(ob.lde(coeffs, lg_n, rate, cols), lg_n + rate, cols)
+        want.append((rows, *ob.merkle(rows, cols, cap, ht)))
+    for _ in range(4):
+        for j in jobs:
+            j[0].d_digests.zero()
+            j[0].d_caps.zero()
+        zk.commit_batch([j[0] for j in jobs])
+        for (c, *_), w in zip(jobs, want):
+            for got, exp in zip(c.results(), w):
+                assert np.array_equal(got, exp)

@@ -94,7 +94,7 @@ private:
         size_t offset;      // bytes into desc_
         uint32_t count;
         uint64_t blocks;
-        int kind;           // 0 NTT, 1 Merkle (leaves, or fused trees), 2 Merkle level
+        int kind;           // 0 NTT, 1 Merkle (leaves, or fused trees), 2 Merkle level, 3 narrow Merkle
         int hash;           // NTT: contiguous; Merkle: hash type
         int kernel;         // NTT: ntt_kernel_kind of the list
         uint32_t tile_log;  // Merkle work-group size (log2 lanes)

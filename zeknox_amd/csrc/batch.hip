@@ -147,13 +147,22 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
     uint64_t tree_leaves = 0;
     for (size_t i = 0; i < n; i++)
         if (jobs[i].cap_height < jobs[i].lg_n + jobs[i].rate) tree_leaves += 1ull << (jobs[i].lg_n + jobs[i].rate);
-    const bool by_level = tree_leaves > 0 && tree_leaves >= dev_.level_launch_leaves.load();
+    // (Poseidon and Poseidon2 forests small enough for it run on the
+    // 16-permutations-per-wave kernel, whatever the others of the batch do)
+    std::map<int, uint64_t> hash_leaves;
+    for (size_t i = 0; i < n; i++) hash_leaves[(int)jobs[i].hash_type] += 1ull << (jobs[i].lg_n + jobs[i].rate);
+    auto narrow_trees = [&](uint64_t ht) { return has_narrow_kernel(ht) && hash_leaves[(int)ht] <= kNarrowLeaves; };
+    const uint64_t apart_from = dev_.level_launch_leaves.load();
+    auto by_level = [&](uint64_t ht) {
+        return !narrow_trees(ht) && batch_levels_apart(tree_leaves, ht, apart_from);
+    };
 
     // ---- plans
     std::vector<std::vector<NttPass>> ntt_plan(n);
     std::vector<uint64_t> ntt_tiles(n);
     std::vector<MerkleArgs> mk(n);  // every pass of a tree in one descriptor
     std::vector<uint64_t> mk_ctr(n);
+    std::vector<MerkleSpec> specs(n);
     uint64_t total_ctr = 0;
     size_t max_ntt = 0;
     for (size_t i = 0; i < n; i++) {
@@ -176,15 +185,18 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
         s.col_stride = 1ull << lg;
         s.leaf_valu = tun[i].merkle_valu;
         check_merkle(s);
-        std::vector<MerkleArgs> passes;
-        plan_merkle(s, passes, tun[i].merkle_tile_log);
+        specs[i] = s;
         mk_ctr[i] = total_ctr;
-        if (by_level) {
-            mk[i] = passes[0];  // the leaf pass alone: its levels are launched apart
-            mk[i].leaves_only = 1;
+        uint64_t nctr = 0;
+        if (narrow_trees(j.hash_type)) {
+            nctr = plan_merkle_narrow(s, nullptr, mk[i]);
         } else {
-            total_ctr += fuse_merkle_passes(passes, mk[i]);
+            std::vector<MerkleArgs> passes;
+            plan_merkle(s, passes, tun[i].merkle_tile_log);
+            nctr = fuse_merkle_passes(passes, mk[i]);
         }
+        if (by_level(j.hash_type)) mk[i].leaves_only = 1;  // the leaf pass alone: its levels are launched apart
+        else total_ctr += nctr;
         max_ntt = std::max(max_ntt, ntt_plan[i].size());
     }
 
@@ -198,6 +210,52 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
         memcpy(host.data() + off, p, bytes);
         return off;
     };
+    // levels launched apart, by hash kind: level k above the leaves of every
+    // tree that has it in one launch each, and for the hashes with the
+    // 16-permutations-per-wave kernel every level from the first one whose
+    // children are few enough in one launch of that
+    struct LevelLaunch {
+        int hash;
+        bool narrow;
+        std::vector<MerkleArgs> list;
+        std::vector<uint64_t> first_ctr;
+        uint64_t blocks = 0;
+    };
+    std::vector<LevelLaunch> levels;
+    for (int ht : {kPoseidon, kKeccak, kPoseidonBN128, kPoseidon2, kMonolith})
+        if (by_level((uint64_t)ht)) {
+            auto apart = [&](size_t i, uint32_t k) {
+                return (int)jobs[i].hash_type == ht && mk[i].lg_w >= k;
+            };
+            // mk[i].lg_w is the log2 width of tree i's leaf level per subtree
+            // (0: caps == leaves, no levels)
+            for (uint32_t k = 1;; k++) {
+                LevelLaunch l{ht, false, {}, {}};
+                uint64_t children = 0;
+                for (size_t i = 0; i < n; i++)
+                    if (apart(i, k)) children += specs[i].num_caps << (mk[i].lg_w - k + 1);
+                if (!children) break;
+                l.narrow = has_narrow_kernel((uint64_t)ht) && children <= kNarrowNodes;
+                for (size_t i = 0; i < n; i++) {
+                    if (!apart(i, k)) continue;
+                    MerkleArgs a;
+                    if (l.narrow) {
+                        l.first_ctr.push_back(total_ctr);
+                        const uint32_t written = mk[i].lg_w - k + 1;
+                        total_ctr += plan_merkle_narrow(specs[i], &written, a);
+                    } else {
+                        a = merkle_level_args(mk[i], mk[i].lg_w - k);  // the level written (0: the caps)
+                    }
+                    a.tile_begin = l.blocks;
+                    l.blocks += l.narrow ? a.count >> a.tile_log
+                                         : (a.count + kMerkleLevelLanes - 1) / kMerkleLevelLanes;
+                    l.list.push_back(a);
+                }
+                const bool last = l.narrow;
+                levels.push_back(std::move(l));
+                if (last) break;
+            }
+        }
     // arrival counters of the fused upper Merkle passes: zero between launches
     if (ctr_.bytes < total_ctr * sizeof(uint32_t)) {
         sync();
@@ -234,44 +292,29 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
         }
     }
     for (int ht : {kPoseidon, kKeccak, kPoseidonBN128, kPoseidon2, kMonolith})
-        for (uint32_t tl = kMerkleMinTileLog; tl <= (uint32_t)kMerkleMaxTileLog; tl++) {
+        for (uint32_t tl : {(uint32_t)kMerkleNarrowTileLog, 8u, 9u, 10u}) {
+            const bool narrow = tl == (uint32_t)kMerkleNarrowTileLog;
             std::vector<MerkleArgs> list;
             uint64_t blocks = 0;
             for (size_t i = 0; i < n; i++) {
-                if ((int)jobs[i].hash_type != ht || tun[i].merkle_tile_log != tl) continue;
+                if ((int)jobs[i].hash_type != ht || narrow != narrow_trees(jobs[i].hash_type)) continue;
+                if (!narrow && tun[i].merkle_tile_log != tl) continue;
                 MerkleArgs a = mk[i];
                 a.tile_begin = blocks;
-                a.ctr = by_level ? nullptr : ctr_.as<uint32_t>() + mk_ctr[i];
+                a.ctr = by_level((uint64_t)ht) ? nullptr : ctr_.as<uint32_t>() + mk_ctr[i];
                 blocks += a.count >> a.tile_log;
                 list.push_back(a);
             }
             if (list.empty()) continue;
             const size_t off = push(list.data(), list.size() * sizeof(MerkleArgs));
-            launches.push_back({off, (uint32_t)list.size(), blocks, 1, ht, 0, tl});
+            launches.push_back({off, (uint32_t)list.size(), blocks, narrow ? 3 : 1, ht, 0, tl});
             host.resize(align_up(host.size()));
         }
-    if (by_level) {
-        // level k above the leaves of every tree that has it, one launch per
-        // hash kind; mk[i].lg_w is the log2 width of tree i's leaf level per
-        // subtree (0: caps == leaves, no levels)
-        uint32_t depth = 0;
-        for (size_t i = 0; i < n; i++) depth = std::max(depth, mk[i].lg_w);
-        for (uint32_t k = 1; k <= depth; k++)
-            for (int ht : {kPoseidon, kKeccak, kPoseidonBN128, kPoseidon2, kMonolith}) {
-                std::vector<MerkleArgs> list;
-                uint64_t blocks = 0;
-                for (size_t i = 0; i < n; i++) {
-                    if ((int)jobs[i].hash_type != ht || mk[i].lg_w < k) continue;
-                    MerkleArgs a = merkle_level_args(mk[i], mk[i].lg_w - k);  // the level written (0: the caps)
-                    a.tile_begin = blocks;
-                    blocks += (a.count + kMerkleLevelLanes - 1) / kMerkleLevelLanes;
-                    list.push_back(a);
-                }
-                if (list.empty()) continue;
-                const size_t off = push(list.data(), list.size() * sizeof(MerkleArgs));
-                launches.push_back({off, (uint32_t)list.size(), blocks, 2, ht, 0, 0});
-                host.resize(align_up(host.size()));
-            }
+    for (LevelLaunch &l : levels) {
+        for (size_t i = 0; l.narrow && i < l.list.size(); i++) l.list[i].ctr = ctr_.as<uint32_t>() + l.first_ctr[i];
+        const size_t off = push(l.list.data(), l.list.size() * sizeof(MerkleArgs));
+        launches.push_back({off, (uint32_t)l.list.size(), l.blocks, l.narrow ? 3 : 2, l.hash, 0, 0});
+        host.resize(align_up(host.size()));
     }
     size_t off0 = 0;
     const void *desc_before = desc_.p;
@@ -347,6 +390,9 @@ void Engine::issue(hipStream_t s, const std::vector<Launch> &launches, const Lau
         } else if (l.kind == 1) {
             launch_merkle_pass(s, l.hash, reinterpret_cast<const MerkleArgs *>(base), l.count, MerkleArgs{},
                                l.blocks, l.tile_log, pieces.merkle_groups);
+        } else if (l.kind == 3) {
+            launch_merkle_narrow(s, l.hash, reinterpret_cast<const MerkleArgs *>(base), l.count, MerkleArgs{}, l.blocks,
+                                 l.tile_log ? "merkle_leaves" : "merkle_levels", pieces.merkle_groups);
         } else {
             launch_merkle_level(s, l.hash, reinterpret_cast<const MerkleArgs *>(base), l.count, l.blocks,
                                 pieces.merkle_groups);

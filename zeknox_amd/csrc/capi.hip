@@ -105,7 +105,7 @@ void merkle_entry(void *dig, void *cap, const void *leaves, uint64_t nd, uint64_
     Device &d = device(gpu_id);
     std::lock_guard<std::mutex> g(d.mu);
     try {
-        merkle_build(d, s);
+        merkle_build(d, s, device_merkle_scratch());
         d.sync();
     } catch (...) {
         d.merkle_ctr_dirty = true;  // a failed launch may leave arrival counts behind

@@ -45,11 +45,29 @@ void launch_merkle_pass(hipStream_t stream, int hash_type, const MerkleArgs *dev
 // total, issued in ranges of at most `chunk` work-groups when chunk > 0.
 void launch_merkle_level(hipStream_t stream, int hash_type, const MerkleArgs *dev_list, uint32_t n, uint64_t blocks,
                          uint64_t chunk = 0, const MerkleArgs &one = MerkleArgs{});
+// The passes of a tree (written null: leaves in tiles of 2^6), or of what lies
+// above its level of width 2^*written per subtree (nodes in tiles of 2^7),
+// fused into one descriptor for launch_merkle_narrow; returns the arrival
+// counters it needs.
+uint64_t plan_merkle_narrow(const MerkleSpec &s, const uint32_t *written, MerkleArgs &out);
+// One launch of the 16-permutations-per-wave kernel (merkle_narrow.h; Poseidon
+// and Poseidon2) over n such descriptors in device memory, or over `one`
+// (n == 0); `blocks` tiles in total, issued in ranges of at most `chunk`.
+void launch_merkle_narrow(hipStream_t stream, int hash_type, const MerkleArgs *dev_list, uint32_t n,
+                          const MerkleArgs &one, uint64_t blocks, const char *name, uint64_t chunk = 0);
 // Level descriptor (k_merkle_level) of the level of width 2^lg_w per subtree
 // (0: the caps) of the tree whose leaf pass is `leaf` (plan_merkle's first
 // pass); tile_begin 0.
 MerkleArgs merkle_level_args(const MerkleArgs &leaf, uint32_t lg_w);
-// The whole tree in one launch on the device stream; call with d.mu held.
-void merkle_build(Device &d, const MerkleSpec &s);
+// Where merkle_build gets the memory of a fused launch from: zeroed arrival
+// counters, and a device copy of its descriptor.  Both are on d.stream.
+struct MerkleScratch {
+    uint32_t *(*counters)(Device &d, uint64_t n);
+    MerkleArgs *(*descriptor)(Device &d, const MerkleArgs &f);
+};
+// Scratch from the device's buffers, which grow on demand.
+MerkleScratch device_merkle_scratch();
+// The whole tree on the device stream; call with d.mu held.
+void merkle_build(Device &d, const MerkleSpec &s, const MerkleScratch &scratch);
 
 }  // namespace zkx

@@ -33,10 +33,11 @@ void check_merkle(const MerkleSpec &s)
     if (!s.digests) invalid("null digest buffer");
 }
 
-uint32_t plan_merkle(const MerkleSpec &s, MerkleArgs (&passes)[kMerkleMaxPasses], uint32_t tile_log_max)
+// Passes from the level of width 2^lg_w per subtree up, in tiles of at most
+// 2^tile_log_max nodes, those above the first pass of 2^upper_log_max.
+static uint32_t plan_passes(const MerkleSpec &s, MerkleArgs (&passes)[kMerkleMaxPasses], uint32_t tile_log_max,
+                            uint32_t upper_log_max, uint32_t lg_w)
 {
-    if (tile_log_max < (uint32_t)kMerkleMinTileLog || tile_log_max > (uint32_t)kMerkleMaxTileLog)
-        invalid("Merkle tile size out of range");
     MerkleArgs a{};
     a.leaves = s.leaves;
     a.leaves_out = s.leaves_out;
@@ -54,19 +55,35 @@ uint32_t plan_merkle(const MerkleSpec &s, MerkleArgs (&passes)[kMerkleMaxPasses]
         return 1;
     }
     const uint32_t h = log2u(s.num_caps);
-    uint32_t lg_w = log2u(s.num_leaves) - h;  // per-subtree width of the input level
     a.sdl = s.num_digests >> h;
     uint32_t n = 0;
     while (true) {
         if (n == (uint32_t)kMerkleMaxPasses) invalid("tree too large");
         a.count = s.num_caps << lg_w;
         a.lg_w = lg_w;
-        a.tile_log = std::min<uint32_t>(tile_log_max, log2u(a.count));
+        a.tile_log = std::min<uint32_t>(n ? upper_log_max : tile_log_max, log2u(a.count));
         passes[n++] = a;
         if (lg_w <= a.tile_log) break;  // this pass reaches the caps
         lg_w -= a.tile_log;
     }
     return n;
+}
+
+uint32_t plan_merkle(const MerkleSpec &s, MerkleArgs (&passes)[kMerkleMaxPasses], uint32_t tile_log_max)
+{
+    if (tile_log_max < (uint32_t)kMerkleMinTileLog || tile_log_max > (uint32_t)kMerkleMaxTileLog)
+        invalid("Merkle tile size out of range");
+    return plan_passes(s, passes, tile_log_max, tile_log_max, log2u(s.num_leaves) - log2u(s.num_caps));
+}
+
+uint64_t plan_merkle_narrow(const MerkleSpec &s, const uint32_t *written, MerkleArgs &out)
+{
+    MerkleArgs passes[kMerkleMaxPasses];
+    const uint32_t n = plan_passes(s, passes, written ? kMerkleNarrowNodesLog : kMerkleNarrowTileLog,
+                                   kMerkleNarrowNodesLog,
+                                   written ? *written : log2u(s.num_leaves) - log2u(s.num_caps));
+    if (written) passes[0].leaves = nullptr;
+    return fuse_merkle_passes(passes, n, out);
 }
 
 void plan_merkle(const MerkleSpec &s, std::vector<MerkleArgs> &passes, uint32_t tile_log_max)
@@ -155,7 +172,49 @@ void launch_merkle_level(hipStream_t stream, int hash_type, const MerkleArgs *de
     }
 }
 
-void merkle_build(Device &d, const MerkleSpec &s)
+void launch_merkle_narrow(hipStream_t stream, int hash_type, const MerkleArgs *dev_list, uint32_t n,
+                          const MerkleArgs &one, uint64_t blocks, const char *name, uint64_t chunk)
+{
+    if (blocks == 0) return;
+    if (blocks > 0x7FFFFFFFull) invalid("tree too large for one launch");
+    ProfScope ps(name, stream);
+    const uint64_t step = (chunk && n > 0) ? chunk : blocks;
+    for (uint64_t b0 = 0; b0 < blocks; b0 += step) {
+        const uint64_t nb = std::min(step, blocks - b0);
+        if (hash_type == kPoseidon2)
+            launch_merkle_narrow_hash<kPoseidon2>(stream, dev_list, n, one, nb, (uint32_t)b0);
+        else launch_merkle_narrow_hash<kPoseidon>(stream, dev_list, n, one, nb, (uint32_t)b0);
+        ZKX_HIP(hipGetLastError());
+    }
+}
+
+namespace {
+
+uint32_t *device_counters(Device &d, uint64_t n) { return d.merkle_counters(n); }
+
+MerkleArgs *device_descriptor(Device &d, const MerkleArgs &f)
+{
+    MerkleArgs *dj = d.merkle_descriptor();
+    ZKX_HIP(hipMemcpyAsync(dj, &f, sizeof(f), hipMemcpyHostToDevice, d.stream));
+    return dj;
+}
+
+// The tree, or what lies above the level of width 2^*written per subtree, in
+// one launch.
+void build_narrow(Device &d, const MerkleSpec &s, const uint32_t *written, const MerkleScratch &scratch)
+{
+    MerkleArgs f;
+    const uint64_t nctr = plan_merkle_narrow(s, written, f);
+    if (nctr) f.ctr = scratch.counters(d, nctr);
+    launch_merkle_narrow(d.stream, (int)s.hash_type, nullptr, 0, f, f.count >> f.tile_log,
+                         f.leaves ? "merkle_leaves" : "merkle_levels");
+}
+
+}  // namespace
+
+MerkleScratch device_merkle_scratch() { return MerkleScratch{device_counters, device_descriptor}; }
+
+void merkle_build(Device &d, const MerkleSpec &s, const MerkleScratch &scratch)
 {
     check_merkle(s);
     const Tuning tun = d.cabi_merkle_tuning(s.num_leaves, s.hash_type);
@@ -164,6 +223,11 @@ void merkle_build(Device &d, const MerkleSpec &s)
     sv.leaf_valu = tun.merkle_valu;
     MerkleArgs passes[kMerkleMaxPasses];
     const uint32_t np = plan_merkle(sv, passes, tl);
+    const bool narrow = has_narrow_kernel(s.hash_type);
+    if (narrow && s.num_leaves <= kNarrowLeaves) {
+        build_narrow(d, s, nullptr, scratch);
+        return;
+    }
     if (s.num_caps < s.num_leaves && lone_tree_levels_apart(s.num_leaves, s.hash_type, d.lone_level_leaves.load())) {
         // a large tree: the leaf digests in one launch, then one launch per
         // level (k_merkle_level), each level's descriptor passed by value
@@ -171,6 +235,11 @@ void merkle_build(Device &d, const MerkleSpec &s)
         leaf.leaves_only = 1;
         launch_merkle_pass(d.stream, (int)s.hash_type, nullptr, 0, leaf, leaf.count >> leaf.tile_log, tl);
         for (uint32_t w = leaf.lg_w; w-- > 0;) {
+            if (narrow && s.num_caps << (w + 1) <= kNarrowNodes) {
+                const uint32_t written = w + 1;
+                build_narrow(d, s, &written, scratch);
+                break;
+            }
             const MerkleArgs lv = merkle_level_args(leaf, w);
             launch_merkle_level(d.stream, (int)s.hash_type, nullptr, 0,
                                 (lv.count + kMerkleLevelLanes - 1) / kMerkleLevelLanes, 0, lv);
@@ -185,9 +254,8 @@ void merkle_build(Device &d, const MerkleSpec &s)
         return;
     }
     // fused upper passes read their fields from a descriptor in device memory
-    f.ctr = d.merkle_counters(nctr);
-    MerkleArgs *dj = d.merkle_descriptor();
-    ZKX_HIP(hipMemcpyAsync(dj, &f, sizeof(f), hipMemcpyHostToDevice, d.stream));
+    f.ctr = scratch.counters(d, nctr);
+    const MerkleArgs *dj = scratch.descriptor(d, f);
     launch_merkle_pass(d.stream, (int)s.hash_type, dj, 1, MerkleArgs{}, f.count >> f.tile_log, tl);
 }
 

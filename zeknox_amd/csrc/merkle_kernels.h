@@ -84,7 +84,7 @@ __device__ __forceinline__ void leaf_hash_mfma(const MerkleArgs &a, uint64_t fir
                                                MfmaLds &m)
 {
     const uint32_t t = threadIdx.x, w = t >> 6, j = t & 31, h = (t >> 5) & 1;
-    mfma_fill<HT>(m, t, TPB);
+    mfma_fill<HT, TPB>(m);
     __syncthreads();
     if (64 * w < cur) {
         const uint32_t ls = a.leaf_size;
@@ -311,7 +311,7 @@ k_merkle_level(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs o
     const uint64_t g = g0 + t;
     uint64_t out[4];
     if constexpr (has_mfma(HT)) {
-        mfma_fill<HT>(tables, t, kMerkleLevelLanes);
+        mfma_fill<HT, kMerkleLevelLanes>(tables);
         __syncthreads();
         const uint32_t w = t >> 6, j = t & 31, h = (t >> 5) & 1;
         uint64_t s[2][6];

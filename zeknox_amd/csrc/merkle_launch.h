@@ -20,5 +20,11 @@ void launch_merkle_hash(hipStream_t stream, const MerkleArgs *dev_list, uint32_t
 template <int HT>
 void launch_merkle_level_hash(hipStream_t stream, const MerkleArgs *dev_list, uint32_t n, const MerkleArgs &one,
                               uint64_t blocks, uint32_t block0);
+// One launch of k_merkle_narrow (Poseidon and Poseidon2) over the n
+// descriptors at dev_list (n > 0) or the single descriptor `one` (n == 0),
+// running tiles block0 .. block0 + blocks - 1.
+template <int HT>
+void launch_merkle_narrow_hash(hipStream_t stream, const MerkleArgs *dev_list, uint32_t n, const MerkleArgs &one,
+                               uint64_t blocks, uint32_t block0);
 
 }  // namespace zkx

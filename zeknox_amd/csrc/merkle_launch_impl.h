@@ -3,6 +3,7 @@
 #pragma once
 #include "merkle_kernels.h"
 #include "merkle_launch.h"
+#include "merkle_narrow.h"
 
 namespace zkx {
 
@@ -23,6 +24,14 @@ void launch_merkle_level_hash(hipStream_t stream, const MerkleArgs *dev_list, ui
                               uint64_t blocks, uint32_t block0)
 {
     hipLaunchKernelGGL((k_merkle_level<HT>), dim3((uint32_t)blocks), dim3(kMerkleLevelLanes), 0, stream, dev_list, n,
+                       one, block0);
+}
+
+template <int HT>
+void launch_merkle_narrow_hash(hipStream_t stream, const MerkleArgs *dev_list, uint32_t n, const MerkleArgs &one,
+                               uint64_t blocks, uint32_t block0)
+{
+    hipLaunchKernelGGL((k_merkle_narrow<HT>), dim3((uint32_t)blocks), dim3(kMerkleNarrowLanes), 0, stream, dev_list, n,
                        one, block0);
 }
 

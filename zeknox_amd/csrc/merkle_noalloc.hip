@@ -35,15 +35,14 @@ constexpr int kMaxDevices = 64;
 // device (under the device's lock) and never changed afterwards.
 unsigned char *g_scratch[kMaxDevices] = {};
 
-// Writes the launch's descriptor and zeroes its arrival counters: every call
+// Write a launch's descriptor and zero its arrival counters: every call
 // starts from zero whatever an earlier (possibly failed) launch left behind.
-// A fill kernel rather than hipMemsetAsync, so that captured streams record
-// kernel nodes only.
-__global__ void k_noalloc_setup(MerkleArgs *desc, MerkleArgs f, uint32_t *ctr, uint32_t nctr)
+// Kernels rather than hipMemcpyAsync and hipMemsetAsync, so that captured
+// streams record kernel nodes only.
+__global__ void k_noalloc_descriptor(MerkleArgs *desc, MerkleArgs f) { *desc = f; }
+__global__ void k_noalloc_counters(uint32_t *ctr, uint32_t nctr)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) *desc = f;
-    for (uint32_t k = i; k < nctr; k += gridDim.x * blockDim.x) ctr[k] = 0;
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < nctr; k += gridDim.x * blockDim.x) ctr[k] = 0;
 }
 
 unsigned char *scratch_of(Device &d)
@@ -57,6 +56,24 @@ unsigned char *scratch_of(Device &d)
         g_scratch[d.id] = static_cast<unsigned char *>(p);
     }
     return g_scratch[d.id];
+}
+
+uint32_t *noalloc_counters(Device &d, uint64_t n)
+{
+    if (n > kMaxCounters) invalid("internal: more arrival counters than the scratch holds");
+    uint32_t *ctr = reinterpret_cast<uint32_t *>(scratch_of(d) + kDescBytes);
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + 255) / 256, 256);
+    hipLaunchKernelGGL(k_noalloc_counters, dim3(blocks), dim3(256), 0, d.stream, ctr, (uint32_t)n);
+    ZKX_HIP(hipGetLastError());
+    return ctr;
+}
+
+MerkleArgs *noalloc_descriptor(Device &d, const MerkleArgs &f)
+{
+    MerkleArgs *desc = reinterpret_cast<MerkleArgs *>(scratch_of(d));
+    hipLaunchKernelGGL(k_noalloc_descriptor, dim3(1), dim3(1), 0, d.stream, desc, f);
+    ZKX_HIP(hipGetLastError());
+    return desc;
 }
 
 void merkle_noalloc(void *dig, void *cap, void *leaves, uint64_t nd, uint64_t nc, uint64_t nl, uint64_t ls,
@@ -77,10 +94,8 @@ void merkle_noalloc(void *dig, void *cap, void *leaves, uint64_t nd, uint64_t nc
     check_merkle(s);
     Device &d = device(gpu_id);
     std::lock_guard<std::mutex> g(d.mu);
-    unsigned char *const base = scratch_of(d);
-    const Tuning tun = d.cabi_merkle_tuning(s.num_leaves, s.hash_type);
-    const uint32_t tl = tun.merkle_tile_log;
-    s.leaf_valu = tun.merkle_valu;
+    // the fused launch of every tree it takes fits the scratch
+    const uint32_t tl = d.cabi_merkle_tuning(s.num_leaves, s.hash_type).merkle_tile_log;
     MerkleArgs passes[kMerkleMaxPasses];
     const uint32_t np = plan_merkle(s, passes, tl);
     MerkleArgs f;
@@ -89,17 +104,7 @@ void merkle_noalloc(void *dig, void *cap, void *leaves, uint64_t nd, uint64_t nc
         invalid("tree needs " + std::to_string(nctr) + " arrival counters; the allocation-free entry point holds " +
                 std::to_string(kMaxCounters) + " (" + std::to_string(kScratchBytes) +
                 " bytes of scratch); use fill_digests_buf_linear_gpu_with_gpu_ptr");
-    f.tile_begin = 0;
-    if (!nctr) {
-        launch_merkle_pass(d.stream, (int)s.hash_type, nullptr, 0, f, f.count >> f.tile_log, tl);
-    } else {
-        MerkleArgs *desc = reinterpret_cast<MerkleArgs *>(base);
-        f.ctr = reinterpret_cast<uint32_t *>(base + kDescBytes);
-        const uint32_t blocks = (uint32_t)std::min<uint64_t>((nctr + 255) / 256, 256);
-        hipLaunchKernelGGL(k_noalloc_setup, dim3(blocks), dim3(256), 0, d.stream, desc, f, f.ctr, (uint32_t)nctr);
-        ZKX_HIP(hipGetLastError());
-        launch_merkle_pass(d.stream, (int)s.hash_type, desc, 1, MerkleArgs{}, f.count >> f.tile_log, tl);
-    }
+    merkle_build(d, s, MerkleScratch{noalloc_counters, noalloc_descriptor});
     d.sync();
 }
 

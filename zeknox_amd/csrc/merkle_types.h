@@ -14,11 +14,16 @@ constexpr int kMerkleMinTileLog = 8;
 constexpr int kMerkleMaxTileLog = 10;
 // Passes of one tree: tiles of >= 2^8 nodes reduce 2^32 leaves in 4.
 constexpr int kMerkleMaxPasses = 4;
+// Tiles (log2) and work-group size of the 16-permutations-per-wave kernel
+// (merkle_narrow.h).
+constexpr int kMerkleNarrowTileLog = 6;   // leaves
+constexpr int kMerkleNarrowNodesLog = 7;  // nodes of a level that is written
+constexpr int kMerkleNarrowLanes = 256;
 // Work-group size (nodes) of the one-level-per-launch kernel.
 constexpr int kMerkleLevelLanes = 256;
 
 struct MerkleArgs {
-    const uint64_t *leaves;  // first pass: leaf source
+    const uint64_t *leaves;  // first pass: leaf source (null, k_merkle_narrow only: the level lg_w is written)
     uint64_t *leaves_out;    // first pass, optional: leaf rows [t][leaf_size]
     uint64_t *dig;
     uint64_t *cap;

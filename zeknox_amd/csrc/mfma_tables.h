@@ -1,6 +1,8 @@
 // Compile-time tables of the matrix-core Poseidon and Poseidon2 permutations
-// (poseidon_mfma.h): the linear maps between S-boxes, cut into signed bytes
-// as operands of v_mfma_i32_32x32x32_i8, and their folded constants.
+// (poseidon_mfma.h: 64 per wave; poseidon_narrow.h: 16 per wave): the linear
+// maps between S-boxes, cut into signed bytes as operands of
+// v_mfma_i32_32x32x32_i8 and v_mfma_i32_16x16x64_i8, and their folded
+// constants.
 //
 // Both permutations are 8 full rounds and 22 partial rounds of x^7 with a
 // linear layer after each round (poseidon/poseidon.cu:563-838,
@@ -18,9 +20,10 @@
 //
 // Slots.  A map reads 16 slots of 64 bits: slots 0..11 the state elements
 // (slot 0: y_1 in a group), slots 12..15 further S-box outputs (a group:
-// y_2..y_5; the entry: y_1 in 12, y_2 in 14).  K-chunk kappa of 32 bytes
-// holds the slots 6h + 2 kappa + {0, 1} of lane half h for kappa < 3, and
-// 12 + 2h + {0, 1} for kappa = 3.
+// y_2..y_5; the entry: y_1 in 12, y_2 in 14).  64 per wave: K-chunk kappa of
+// 32 bytes holds the slots 6h + 2 kappa + {0, 1} of lane half h for
+// kappa < 3, and 12 + 2h + {0, 1} for kappa = 3.  16 per wave: K-chunk kappa
+// of 64 bytes holds the slots 8 kappa + q and 8 kappa + 4 + q of lane group q.
 //
 // Bytes.  A coefficient c applied to byte b of a slot contributes
 // c * 2^(8b) mod p, written in eight signed digits of base 256: one output
@@ -62,9 +65,23 @@ struct Pair {
 
 struct Tables {
     alignas(16) uint8_t op[kOps][64][16];
-    Pair row[kRows][12];
+    alignas(16) Pair row[kRows][12];
     Pair x_entry[2];         // constants of x_1, x_2 of the entry map
     Pair x_group[kGroups][4];  // constants of x_2..x_5 of each group
+};
+
+// Operands of the 16-per-wave form, in the order [M-block][K-chunk of 2]: M-
+// block 2a + n holds digits 4n..4n + 3 of element 4a + q for lane group q, or
+// of output a for every lane group.
+constexpr int kNarrowLayer = 0;    // 12: the full rounds' layer
+constexpr int kNarrowGroup = 12;   // 12: F of five partial rounds
+constexpr int kNarrowGroupX = 24;  // 16: x_2..x_5
+constexpr int kNarrowEntry = 40;   // 12: F of the entry map
+constexpr int kNarrowEntryX = 52;  // 8: x_1, x_2
+constexpr int kNarrowOps = 60;
+
+struct NarrowTables {
+    alignas(16) uint8_t op[kNarrowOps][64][16];
 };
 
 constexpr uint64_t cadd(uint64_t a, uint64_t b)
@@ -208,60 +225,108 @@ constexpr Weights partial_weights()
     return w;
 }
 
+// Rows of the 16-per-wave operands from `op` on.
+constexpr void put_narrow(NarrowTables &t, int op, const Form *rows, int nrows, bool every_group)
+{
+    for (int R = 0; R < nrows; R++)
+        for (int q = 0; q < 16; q++) {
+            uint64_t v = rows[R].c[q];
+            if (!v) continue;
+            for (int b = 0; b < 8; b++) {
+                int d[8] = {};
+                digits(v, d);
+                for (int n = 0; n < 8; n++) {
+                    const int block = 2 * (every_group ? R : R / 4) + n / 4;
+                    for (int g = every_group ? 0 : R % 4; g <= (every_group ? 3 : R % 4); g++)
+                        t.op[op + 2 * block + q / 8][16 * (q % 4) + 4 * g + n % 4][8 * (q / 4 % 2) + b] = (uint8_t)d[n];
+                }
+                v = gl::cmul(v, 256);
+            }
+        }
+}
+
 constexpr uint32_t kState = 0x0FFF, kAll = 0xFFFF;
+
+// The maps as affine forms: what the operands and constants are made of.
+struct Maps {
+    State full;               // the full rounds' layer, without constants
+    State entry;              // the layer of full round 3, then partial rounds 4 and 5
+    Form x_entry[2];          // x_1, x_2
+    State group[kGroups];     // five partial rounds
+    Form x_group[kGroups][4];  // x_2..x_5, their y terms left out
+};
+
+constexpr Form of_state(Form f, int first)
+{
+    for (int q = 0; q < 16; q++)
+        if (q < first || q >= 12) f.c[q] = 0;
+    return f;
+}
+
+template <int HT>
+constexpr Maps maps()
+{
+    Maps m{};
+    m.full = step<HT>(identity(), false, 30);
+    m.entry = identity();
+    for (int j = 0; j <= kEntryRounds; j++) {
+        m.entry = step<HT>(m.entry, j > 0, 4 + j);
+        if (j == kEntryRounds) break;
+        m.x_entry[j] = of_state(m.entry.e[0], 0);  // x_2's y_1 term: h_1
+        m.entry.e[0] = slot(12 + 2 * j);
+    }
+    for (int g = 0; g < kGroups; g++) {
+        State &v = m.group[g];
+        v = identity();  // slot 0: y_1
+        for (int j = 0; j < kGroupRounds; j++) {
+            v = step<HT>(v, true, 4 + kEntryRounds + kGroupRounds * g + j + 1);
+            if (j == kGroupRounds - 1) break;
+            m.x_group[g][j] = of_state(v.e[0], 1);
+            v.e[0] = slot(12 + j);
+        }
+    }
+    return m;
+}
 
 template <int HT>
 constexpr Tables make()
 {
     Tables t{};
-    // full rounds
-    State m = step<HT>(identity(), false, 30);
-    put(t, kOpLayer, 3, 3, m.e, 12);
+    Maps m = maps<HT>();
+    put(t, kOpLayer, 3, 3, m.full.e, 12);
     for (int i = 0; i < 12; i++) {
         if (HT == kPoseidon) t.row[kRowFirst][i] = Pair{round_constant<HT>(0, i), 0};
         auto row = [&](int at, int r) {
-            m.e[i].k = round_constant<HT>(r, i);
-            t.row[at][i] = addend(m.e[i], kState);
+            m.full.e[i].k = round_constant<HT>(r, i);
+            t.row[at][i] = addend(m.full.e[i], kState);
         };
         if (HT != kPoseidon) row(kRowFirst, 0);
         for (int r = 0; r < 3; r++) row(kRowFull + r, r + 1);
         for (int r = 0; r < 4; r++) row(kRowLast + r, r + 27);
+        t.row[kRowEntry][i] = addend(m.entry.e[i], kAll);
+        for (int g = 0; g < kGroups; g++) t.row[kRowGroup + g][i] = addend(m.group[g].e[i], kAll);
     }
-    // entry: the layer of full round 3, then partial rounds 4 and 5
-    {
-        State v = identity();
-        Form x[4];
-        for (int j = 0; j <= kEntryRounds; j++) {
-            v = step<HT>(v, j > 0, 4 + j);
-            if (j == kEntryRounds) break;
-            x[2 * j] = v.e[0];  // x_1 on half 0, x_2 on half 1 (its y_1 term: h_1)
-            t.x_entry[j] = addend(v.e[0], kState);
-            v.e[0] = slot(12 + 2 * j);
-        }
-        for (auto &f : x) for (int q = 12; q < 16; q++) f.c[q] = 0;
-        put(t, kOpEntryX, 1, 3, x, 4);
-        put(t, kOpEntry, 3, 4, v.e, 12);
-        for (int i = 0; i < 12; i++) t.row[kRowEntry][i] = addend(v.e[i], kAll);
-    }
-    // groups of five partial rounds
-    for (int g = 0; g < kGroups; g++) {
-        State v = identity();  // slot 0: y_1
-        Form x[4];
-        for (int j = 0; j < kGroupRounds; j++) {
-            v = step<HT>(v, true, 4 + kEntryRounds + kGroupRounds * g + j + 1);
-            if (j == kGroupRounds - 1) break;
-            x[j] = v.e[0];
-            x[j].c[0] = 0;
-            for (int q = 12; q < 16; q++) x[j].c[q] = 0;
-            t.x_group[g][j] = addend(x[j], kState);
-            v.e[0] = slot(12 + j);
-        }
-        if (g == 0) {
-            put(t, kOpGroupX, 1, 3, x, 4);
-            put(t, kOpGroup, 3, 4, v.e, 12);
-        }
-        for (int i = 0; i < 12; i++) t.row[kRowGroup + g][i] = addend(v.e[i], kAll);
-    }
+    const Form xe[4] = {m.x_entry[0], Form{}, m.x_entry[1], Form{}};  // x_1 on half 0, x_2 on half 1
+    put(t, kOpEntryX, 1, 3, xe, 4);
+    put(t, kOpEntry, 3, 4, m.entry.e, 12);
+    put(t, kOpGroupX, 1, 3, m.x_group[0], 4);
+    put(t, kOpGroup, 3, 4, m.group[0].e, 12);
+    for (int j = 0; j < kEntryRounds; j++) t.x_entry[j] = addend(m.x_entry[j], kState);
+    for (int g = 0; g < kGroups; g++)
+        for (int j = 0; j < 4; j++) t.x_group[g][j] = addend(m.x_group[g][j], kState);
+    return t;
+}
+
+template <int HT>
+constexpr NarrowTables make_narrow()
+{
+    NarrowTables t{};
+    const Maps m = maps<HT>();
+    put_narrow(t, kNarrowLayer, m.full.e, 12, false);
+    put_narrow(t, kNarrowGroup, m.group[0].e, 12, false);
+    put_narrow(t, kNarrowGroupX, m.x_group[0], 4, true);
+    put_narrow(t, kNarrowEntry, m.entry.e, 12, false);
+    put_narrow(t, kNarrowEntryX, m.x_entry, kEntryRounds, true);
     return t;
 }
 

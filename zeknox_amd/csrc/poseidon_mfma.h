@@ -61,16 +61,30 @@ __device__ const mfma::Tables c_mfma = mfma::make<HT>();
 // (24 KiB) and the constant rows.
 struct MfmaLds {
     mf_v4i op[mfma::kOpsLds][64];
-    uint64_t row[mfma::kRows][12][2];
+    alignas(16) uint64_t row[mfma::kRows][12][2];
 };
 
-template <int HT>
-__device__ __forceinline__ void mfma_fill(MfmaLds &m, uint32_t t, uint32_t nthreads)
+// dst <- src, COUNT 16-byte words by a work-group of N lanes: every load in
+// flight before the first write.
+template <int COUNT, int N>
+__device__ __forceinline__ void copy_to_lds(mf_v4i *dst, const mf_v4i *src)
 {
-    const mf_v4i *ops = reinterpret_cast<const mf_v4i *>(c_mfma<HT>.op);
-    for (uint32_t i = t; i < mfma::kOpsLds * 64; i += nthreads) m.op[0][i] = ops[i];
-    const uint64_t *rows = &c_mfma<HT>.row[0][0].l;
-    for (uint32_t i = t; i < mfma::kRows * 24; i += nthreads) m.row[0][0][i] = rows[i];
+    constexpr int kSteps = (COUNT + N - 1) / N;
+    const uint32_t t = threadIdx.x;
+    mf_v4i v[kSteps];
+#pragma unroll
+    for (int i = 0; i < kSteps; i++)
+        if (COUNT % N == 0 || t + i * N < COUNT) v[i] = src[t + i * N];
+#pragma unroll
+    for (int i = 0; i < kSteps; i++)
+        if (COUNT % N == 0 || t + i * N < COUNT) dst[t + i * N] = v[i];
+}
+
+template <int HT, int N>
+__device__ __forceinline__ void mfma_fill(MfmaLds &m)
+{
+    copy_to_lds<mfma::kOpsLds * 64, N>(&m.op[0][0], reinterpret_cast<const mf_v4i *>(c_mfma<HT>.op));
+    copy_to_lds<mfma::kRows * 12, N>(reinterpret_cast<mf_v4i *>(m.row), reinterpret_cast<const mf_v4i *>(c_mfma<HT>.row));
 }
 
 // Exchanges the upper half of a with the lower half of b: a becomes

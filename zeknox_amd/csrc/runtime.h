@@ -110,19 +110,13 @@ struct Device {
     // graphs (zkx_set_commit_graphs); read at each commit.
     std::atomic<bool> commit_graphs{true};
     // Batches whose trees hold at least this many leaves in total build the
-    // levels above the leaves with one launch per level over all trees
-    // (zkx_set_level_launches); smaller ones, one fused launch per hash kind.
-    // Measured on 1-16 commits of 135 x 2^15 rate 3 and 20 x 2^12 rate 2
-    // (Poseidon, Poseidon2): by level 0.93-0.99 of the fused time from 2^18
-    // leaves up, 1.14-1.16 below (each level launch costs at least one
-    // permutation's latency, about 43 us).
+    // levels above the leaves in launches of their own over all trees
+    // (zkx_set_level_launches, batch_levels_apart); smaller ones, one fused
+    // launch per hash kind.  Keccak-256 and Monolith, 1-16 commits: by level
+    // 0.93-0.99 of the fused time from 2^18 leaves up, 1.14-1.16 below.
     std::atomic<uint64_t> level_launch_leaves{1ull << 18};
     // The same for one tree through the C-ABI Merkle entry points
-    // (fill_digests_buf_linear_gpu_with_gpu_ptr; the allocation-free entry
-    // point always runs one fused launch); Keccak-256 and Monolith trees
-    // from a quarter of this, Poseidon-BN128 trees from a 32nd
-    // (lone_tree_levels_apart): a lone tree's narrow levels are
-    // latency-bound either way, so only wide trees gain.
+    // (zkx_set_lone_level_launches, lone_tree_levels_apart).
     std::atomic<uint64_t> lone_level_leaves{1ull << 20};
     Tuning tuning_default();
     // The schedule of the C-ABI Merkle entry points for one tree: the

@@ -53,27 +53,54 @@ using TuneKey = std::tuple<uint32_t, uint32_t, uint32_t, uint32_t, bool>;
 
 bool valid_tuning(const Tuning &t);
 
+// Poseidon and Poseidon2 have a kernel with 16 permutations per wave
+// (merkle_narrow.h) besides those with 64, for work whose time is one
+// permutation's latency.
+inline bool has_narrow_kernel(uint64_t hash_type) { return hash_type == 0 || hash_type == 3; }
+// It builds forests of at most this many leaves (all trees of one hash in a
+// launch) in one launch, all work-groups resident, two waves per SIMD.
+// (135-element leaves, cap 4, in us, 64 / 16 per wave: Poseidon 2^13 690 /
+// 325, 2^15 880 / 453, Poseidon2 2^15 890 / 502; 2^16 needs two rounds of the
+// 16-per-wave waves, 590 us for the leaves against 580.)
+constexpr uint64_t kNarrowLeaves = 1ull << 15;
+// It finishes larger trees from the first level of at most this many children
+// (over all trees of one hash): every tile of 128 is resident at once.
+constexpr uint64_t kNarrowNodes = 1ull << 16;
+
 // Whether one tree through the C-ABI Merkle entry points builds its levels
-// with one launch per level (after a leaf-digests-only launch) rather than
+// with one launch per level (after a leaf-digests-only launch; Poseidon and
+// Poseidon2 finish with one launch of the 16-per-wave kernel) rather than
 // inside its leaf launch, given the device threshold `min_leaves` (default
-// 2^20): Poseidon and Poseidon2 trees switch at min_leaves, Keccak-256 and
-// Monolith at min_leaves / 4, Poseidon-BN128 at min_leaves / 32 (0: always).
-// Measured, fused against by level, 135-element leaves, cap 4, one GPU, ms:
+// 2^20): Poseidon and Poseidon2 trees switch at min_leaves / 32, Keccak-256
+// and Monolith at min_leaves / 4, Poseidon-BN128 at min_leaves / 32 (0:
+// always).  Measured, fused against apart, 135-element leaves, cap 4, ms:
 //   leaves  Poseidon      Poseidon2     Keccak-256     Monolith       Poseidon-BN128
-//   2^15    0.90 / 1.10   1.10 / 1.27   0.248 / 0.251  0.540 / 0.533  36.2 / 33.5
-//   2^17    1.30 / 1.48   1.43 / 1.59   0.330 / 0.333  0.695 / 0.697  48.5 / 46.2
-//   2^18    2.32 / 2.45   2.34 / 2.42   0.503 / 0.485  1.078 / 1.056  75.3 / 72.8
-//   2^19    4.33 / 4.34   4.02 / 4.01   1.095 / 0.779  2.069 / 1.760
-//   2^20    8.28 / 8.16   7.34 / 7.12   1.928 / 1.344  3.639 / 3.143
-// Poseidon's fused levels (rows of 16 lanes) are the fastest of the hashes';
-// Keccak's and Monolith's permutations are short, so their fused trees'
-// tops, one permutation's latency per level on ever fewer lanes, weigh
-// more; Poseidon-BN128's levels are slow enough that a full-GPU launch per
-// level pays at every size measured.
+//   2^15                                0.248 / 0.251  0.540 / 0.533  36.2 / 33.5
+//   2^16                  0.92 / 0.76
+//   2^17                  1.11 / 0.96   0.330 / 0.333  0.695 / 0.697  48.5 / 46.2
+//   2^18    1.74 / 1.53   1.86 / 1.65   0.503 / 0.485  1.078 / 1.056  75.3 / 72.8
+//   2^19                  3.66 / 3.25   1.095 / 0.779  2.069 / 1.760
+//   2^20    6.36 / 5.67   7.01 / 6.02   1.928 / 1.344  3.639 / 3.143
+// Poseidon's and Poseidon2's narrow levels cost 12 us each in the 16-per-wave
+// kernel against 25-36 us on lane pairs and rows inside the leaf launch, so
+// every tree that is not built whole by that kernel gains.  Keccak's and
+// Monolith's permutations are short, so their fused trees' tops, one
+// permutation's latency per level on ever fewer lanes, weigh more;
+// Poseidon-BN128's levels are slow enough that a full-GPU launch per level
+// pays at every size measured.
 inline bool lone_tree_levels_apart(uint64_t num_leaves, uint64_t hash_type, uint64_t min_leaves)
 {
-    const uint32_t shift = hash_type == 1 || hash_type == 4 ? 2 : hash_type == 2 ? 5 : 0;
+    const uint32_t shift = hash_type == 1 || hash_type == 4 ? 2 : 5;
     return num_leaves >= (min_leaves >> shift);
+}
+// The same for the forests of one hash in a batch of `batch_leaves` leaves in
+// total (default threshold 2^18; Poseidon and Poseidon2 at an eighth).
+// Commits of 135 x 2^n rate 3, Poseidon, fused against apart, ms: 2^16 leaves
+// 0.93 / 0.85, 2^17 1.23 / 1.12, 2^18 2.28 / 2.00; 8 of 20 x 2^12 rate 3
+// (2^18 leaves) 0.71 / 0.55.
+inline bool batch_levels_apart(uint64_t batch_leaves, uint64_t hash_type, uint64_t min_leaves)
+{
+    return batch_leaves > 0 && batch_leaves >= (has_narrow_kernel(hash_type) ? min_leaves >> 3 : min_leaves);
 }
 
 }  // namespace zkx
