@@ -103,3 +103,83 @@ def test_batch_forests(zk, ht, shapes):
         for (c, *_), w in zip(jobs, want):
             for got, exp in zip(c.results(), w):
                 assert np.array_equal(got, exp)
+
+
+def _borrows(a, b):
+    """Whether u - h1 borrows in the lazy product of a and b (gl64.h
+    reduce128_rare): a b = lo + (h0 + 2^32 h1) 2^64 with the carry of the
+    middle sum taken out of the high word, u = lo + h0 (2^32 - 1) mod 2^64."""
+    m = (1 << 32) - 1
+    a0, a1, b0, b1 = a & m, a >> 32, b & m, b >> 32
+    u = a0 * b0
+    w = a1 * b0 + a0 * b1 + (u >> 32)
+    c, w = w >> 64, w & ((1 << 64) - 1)
+    hi = a1 * b1 + (w >> 32)
+    lo = (u & m) | ((w & m) << 32)
+    return (lo + (hi & m) * m) % (1 << 64) < (hi >> 32) + c
+
+
+def _reduced(x):
+    return x % ob.P
+
+
+def _rare_inputs():
+    """S-box inputs by the product that borrows."""
+    found = {}
+    rng = np.random.default_rng(1)
+    for e in range(20000):
+        k = int(rng.integers(0, 64))
+        x = ((1 << k) * int(rng.integers(1, 1 << int(rng.integers(1, 6)))) + (0 if e % 2 else (1 << int(rng.integers(0, 64))))) % ob.P
+        x2 = _reduced(x * x)
+        x3, x4 = _reduced(x2 * x), _reduced(x2 * x2)
+        for step, (a, b) in enumerate([(x, x), (x2, x), (x2, x2), (x3, x4)]):
+            if _borrows(a, b):
+                found.setdefault(step, set()).add(x)
+    assert set(found) >= {0, 2, 3}  # x^2, x^4 and x^7: powers of two times small numbers
+    return [sorted(found[s])[:16] for s in sorted(found)]
+
+
+def _solve(m, v):
+    """x with m x = v mod p."""
+    n, rows = len(v), [list(r) + [t] for r, t in zip(m, v)]
+    for i in range(n):
+        k = next(k for k in range(i, n) if rows[k][i])
+        rows[i], rows[k] = rows[k], rows[i]
+        inv = pow(rows[i][i], ob.P - 2, ob.P)
+        rows[i] = [x * inv % ob.P for x in rows[i]]
+        for k in range(n):
+            if k != i:
+                f = rows[k][i]
+                rows[k] = [(x - f * y) % ob.P for x, y in zip(rows[k], rows[i])]
+    return [r[n] for r in rows]
+
+
+@pytest.mark.parametrize("ht", [0, 3])
+def test_rare_borrows(zk, ht):
+    """Leaves made so that first-round S-boxes take the exact form of a product
+    (one lane of a wave, several, all)."""
+    import re
+    text = open(ob.ROOT + "/zeknox_amd/csrc/gl_constants.h").read()
+
+    def table(name):
+        body = re.search(r"#define " + name + r" \\\n(.*?)\n\n", text, re.S).group(1)
+        return [int(t, 0) for t in re.findall(r"0x[0-9a-fA-F]+|\b\d+", body.replace("ULL", "").replace("ull", ""))]
+
+    rc = table("ZK_POSEIDON_RC_LIST" if ht == 0 else "ZK_POSEIDON2_RC_LIST")[:12]
+    m4 = [[5, 7, 1, 3], [4, 6, 1, 1], [1, 3, 5, 7], [1, 1, 4, 6]]
+    external = [[m4[r % 4][c % 4] * (2 if r // 4 == c // 4 else 1) for c in range(8)] for r in range(8)]
+    rare = _rare_inputs()
+    rng = np.random.default_rng(2)
+    n, ls = 1 << 16, 8  # 64 per wave from 2^16 leaves
+    leaves = ob.canonical(n * ls, 31).reshape(n, ls)
+    for leaf in [0, 5, 64, 95, 100, 101, 128 + 63] + list(range(192, 256)):
+        want = [int(rng.choice(rare[int(rng.integers(0, len(rare)))])) if rng.random() < 0.5 else int(rng.integers(0, 1 << 62))
+                for _ in range(8)]
+        want[0] = int(rng.choice(rare[leaf % len(rare)]))
+        v = [(x - k) % ob.P for x, k in zip(want, rc)]
+        leaves[leaf] = v if ht == 0 else _solve(external, v)
+    flat = np.ascontiguousarray(leaves.reshape(-1))
+    dig, caps = zk.merkle_tree(flat, ls, 4, ht)
+    edig, ecap = ob.merkle(flat, ls, 4, ht)
+    assert np.array_equal(caps, ecap)
+    assert np.array_equal(dig, edig)

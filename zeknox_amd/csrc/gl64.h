@@ -442,6 +442,139 @@ __device__ __forceinline__ void pow7_lazy2(uint64_t &x, uint64_t &y)
     mul_lazy2(x3, x4, y3, y4, x, y);
 }
 
+// ---- products that leave a rare borrow to the caller
+//
+// In reduce128c_lazy the borrow b of u - h1 is all but impossible for a random
+// product (u is below h1 < 2^32: 2^-32), yet folding it into the correction
+// costs two of the seven instructions.  These forms leave it out,
+//   r = z + c * EPS   (exact unless b),
+// and or the borrow lanes into `bad`: a caller whose mask comes back nonzero
+// throws the results away and takes the exact form.  Per product 12
+// instructions instead of 14; 32 commits of 135 x 2^15 51.4 -> 48.8 ms,
+// Poseidon2 400 x 2^20 40.1 -> 38.0 ms (alternating builds).  A wave alone on
+// its SIMD loses by it: it waits out the branches.
+
+__device__ __forceinline__ uint64_t reduce128_rare(uint64_t lo, uint64_t hi, uint64_t cin, uint64_t &bad)
+{
+    uint64_t u, sc;
+    uint32_t cv;
+    asm("v_mad_u64_u32 %[u], %[sc], %[h0], -1, %[lo]\n\t"
+        "s_nop 1\n\t"
+        "v_cndmask_b32_e64 %[cv], 0, 1, %[sc]"
+        : [u] "=&v"(u), [sc] "=&s"(sc), [cv] "=&v"(cv)
+        : [h0] "v"(lo32(hi)), [lo] "v"(lo));
+    uint32_t zlo, zhi;
+    uint64_t b1, b;
+    asm("v_subb_co_u32_e64 %[zlo], %[b1], %[ulo], %[h1], %[cin]\n\t"
+        "s_nop 1\n\t"
+        "v_subb_co_u32_e64 %[zhi], %[b], %[uhi], 0, %[b1]"
+        : [zlo] "=&v"(zlo), [zhi] "=&v"(zhi), [b1] "=&s"(b1), [b] "=&s"(b)
+        : [ulo] "v"(lo32(u)), [uhi] "v"(hi32(u)), [h1] "v"(hi32(hi)), [cin] "s"(cin));
+    uint64_t r, j;
+    asm("v_mad_u64_u32 %[r], %[j], %[cv], -1, %[z]" : [r] "=&v"(r), [j] "=&s"(j) : [cv] "v"(cv), [z] "v"(pack(zlo, zhi)));
+    bad |= b;
+    return r;
+}
+
+__device__ __forceinline__ void reduce128_rare2(uint64_t lo0, uint64_t hi0, uint64_t cin0, uint64_t lo1, uint64_t hi1,
+                                                uint64_t cin1, uint64_t &r0, uint64_t &r1, uint64_t &bad)
+{
+    uint64_t u0, u1, sc0, sc1;
+    uint32_t cv0, cv1;
+    asm("v_mad_u64_u32 %[u0], %[sc0], %[a0], -1, %[l0]\n\t"
+        "v_mad_u64_u32 %[u1], %[sc1], %[a1], -1, %[l1]\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32_e64 %[cv0], 0, 1, %[sc0]\n\t"
+        "v_cndmask_b32_e64 %[cv1], 0, 1, %[sc1]"
+        : [u0] "=&v"(u0), [u1] "=&v"(u1), [sc0] "=&s"(sc0), [sc1] "=&s"(sc1), [cv0] "=&v"(cv0), [cv1] "=&v"(cv1)
+        : [a0] "v"(lo32(hi0)), [l0] "v"(lo0), [a1] "v"(lo32(hi1)), [l1] "v"(lo1));
+    uint32_t zl0, zh0, zl1, zh1;
+    uint64_t b10, b0, b11, b1;
+    asm("v_subb_co_u32_e64 %[zl0], %[b10], %[ul0], %[h10], %[ci0]\n\t"
+        "v_subb_co_u32_e64 %[zl1], %[b11], %[ul1], %[h11], %[ci1]\n\t"
+        "s_nop 0\n\t"
+        "v_subb_co_u32_e64 %[zh0], %[b0], %[uh0], 0, %[b10]\n\t"
+        "v_subb_co_u32_e64 %[zh1], %[b1], %[uh1], 0, %[b11]"
+        : [zl0] "=&v"(zl0), [zh0] "=&v"(zh0), [zl1] "=&v"(zl1), [zh1] "=&v"(zh1), [b10] "=&s"(b10), [b0] "=&s"(b0),
+          [b11] "=&s"(b11), [b1] "=&s"(b1)
+        : [ul0] "v"(lo32(u0)), [uh0] "v"(hi32(u0)), [h10] "v"(hi32(hi0)), [ul1] "v"(lo32(u1)), [uh1] "v"(hi32(u1)),
+          [h11] "v"(hi32(hi1)), [ci0] "s"(cin0), [ci1] "s"(cin1));
+    uint64_t j0, j1;
+    asm("v_mad_u64_u32 %[r], %[j], %[cv], -1, %[z]"
+        : [r] "=&v"(r0), [j] "=&s"(j0)
+        : [cv] "v"(cv0), [z] "v"(pack(zl0, zh0)));
+    asm("v_mad_u64_u32 %[r], %[j], %[cv], -1, %[z]"
+        : [r] "=&v"(r1), [j] "=&s"(j1)
+        : [cv] "v"(cv1), [z] "v"(pack(zl1, zh1)));
+    bad |= b0 | b1;
+}
+
+__device__ __forceinline__ uint64_t mul_rare(uint64_t a, uint64_t b, uint64_t &bad)
+{
+    uint64_t lo, hi, c;
+    mul128c(a, b, lo, hi, c);
+    return reduce128_rare(lo, hi, c, bad);
+}
+
+__device__ __forceinline__ void mul_rare2(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_t &r0,
+                                          uint64_t &r1, uint64_t &bad)
+{
+    uint64_t lo0, hi0, c0, lo1, hi1, c1;
+    mul128c(a0, b0, lo0, hi0, c0);
+    mul128c(a1, b1, lo1, hi1, c1);
+    reduce128_rare2(lo0, hi0, c0, lo1, hi1, c1, r0, r1, bad);
+}
+
+// reduce96_lazy without its second step, which adds EPS in the lanes of
+// `carry`: a carry out of lo + top * EPS needs lo above 2^64 - top * 2^32
+// (for top < 2^16 one value in 2^16).  add_eps is that step.
+__device__ __forceinline__ uint64_t reduce96_rare(uint64_t lo, uint32_t top, uint64_t &carry)
+{
+    uint64_t u;
+    asm("v_mad_u64_u32 %[u], %[c], %[top], -1, %[lo]" : [u] "=&v"(u), [c] "=&s"(carry) : [top] "v"(top), [lo] "v"(lo));
+    return u;
+}
+__device__ __forceinline__ uint64_t add_eps(uint64_t u, uint64_t lanes)
+{
+    uint64_t r, j;
+    uint32_t cv;
+    asm("s_nop 1\n\t"
+        "v_cndmask_b32_e64 %[cv], 0, 1, %[m]\n\t"
+        "v_mad_u64_u32 %[r], %[j], %[cv], -1, %[u]"
+        : [r] "=&v"(r), [j] "=&s"(j), [cv] "=&v"(cv)
+        : [u] "v"(u), [m] "s"(lanes));
+    return r;
+}
+
+// x^7 of a wave whose branch is uniform: the products above, and the exact
+// ones for the whole wave if any lane borrowed.  `carry`: lanes in which x
+// still lacks an EPS (reduce96_rare).
+__device__ __forceinline__ uint64_t pow7_wave(uint64_t x, uint64_t carry = 0)
+{
+    uint64_t bad = carry, x3, x4;
+    const uint64_t x2 = mul_rare(x, x, bad);
+    mul_rare2(x2, x, x2, x2, x3, x4, bad);
+    uint64_t r = mul_rare(x3, x4, bad);
+    if (__builtin_expect(bad != 0, 0)) r = pow7_lazy(add_eps(x, carry));
+    return r;
+}
+
+// x^7 and y^7 in lockstep.
+__device__ __forceinline__ void pow7_wave2(uint64_t &x, uint64_t &y)
+{
+    uint64_t bad = 0, x2, y2, x3, y3, x4, y4, xr, yr;
+    mul_rare2(x, x, y, y, x2, y2, bad);
+    mul_rare2(x2, x, y2, y, x3, y3, bad);
+    mul_rare2(x2, x2, y2, y2, x4, y4, bad);
+    mul_rare2(x3, x4, y3, y4, xr, yr, bad);
+    if (__builtin_expect(bad != 0, 0)) {
+        pow7_lazy2(x, y);
+    } else {
+        x = xr;
+        y = yr;
+    }
+}
+
 // x^7, canonical.
 __device__ __forceinline__ uint64_t pow7(uint64_t x)
 {

@@ -25,12 +25,16 @@
 // elements per five rounds instead of one per round: 12 layers of vector
 // work instead of 30.
 //
-// Bound: VALU issue (1.07 of one wave instruction per 4 cycles per SIMD, the
-// MFMAs beside it).  Against one layer per round (the MDS on the matrix
+// Bound: VALU issue (1.03 of one wave instruction per 4 cycles per SIMD, the
+// MFMAs beside it; multiply-adds, carries and three-operand forms take 4
+// cycles, moves and plain adds 2).  Against one layer per round (the MDS on the matrix
 // cores for Poseidon, everything on the VALU for Poseidon2), wave
 // instructions per leaf permutation: Poseidon 205 -> 153 VALU, 8.4 -> 4.3
 // MFMA; Poseidon2 234 -> 162 VALU.  Leaf launch of 32 x 2^18 leaves of 135:
 // 56.4 -> 41.0 ms; of 2^21 leaves of 400 with Poseidon2: 36 -> 31.7 ms.
+// The S-boxes' products and the recombination then leave their rare corrections
+// to a branch (gl64.h): 153 -> 137 VALU and 41.0 -> 38.6 ms, Poseidon2 162 ->
+// 146 and 31.7 -> 29.7 ms.
 // Five rounds: the map of four leaves a K-chunk unused and costs as much; six
 // needs a fifth chunk and weights beyond 32 bits.
 //
@@ -137,6 +141,13 @@ __device__ __forceinline__ void hold_operands(const mf_v4i (&a)[NK], const mf_v4
     for (int kappa = 0; kappa < NK; kappa++) asm volatile("; hold %0 %1 %2" ::"v"(p), "v"(a[kappa]), "v"(b[kappa]));
 }
 
+// limb_combine for B < 2^48, less the EPS of the lanes of `carry`.
+__device__ __forceinline__ uint64_t limb_combine_rare(uint64_t A, uint64_t B, uint64_t &carry)
+{
+    const uint64_t T = gl::add_small(B, gl::hi32(A));
+    return gl::reduce96_rare(gl::pack(gl::lo32(A), gl::lo32(T)), gl::hi32(T), carry);
+}
+
 // p01 + 2^16 p23 + k, in signed multiply-adds.
 __device__ __forceinline__ uint64_t half_sum(uint32_t p01, uint32_t p23, uint64_t k)
 {
@@ -153,6 +164,7 @@ __device__ __forceinline__ void mfma_map(uint64_t s[2][6], const mf_v4i (&b)[2][
 {
     // one M-block and group at a time, recombined as soon as its chain is
     // done: 16 accumulator VGPRs live
+    uint64_t carry[2][6];
 #pragma unroll
     for (int beta = 0; beta < 3; beta++) {
         mf_v4i a[NK];
@@ -171,9 +183,20 @@ __device__ __forceinline__ void mfma_map(uint64_t s[2][6], const mf_v4i (&b)[2][
                 const uint64_t L = half_sum(digit_pair(dd[q], dd[q + 1]), digit_pair(dd[q + 2], dd[q + 3]), row[e][0]);
                 const uint64_t H =
                     half_sum(digit_pair(dd[q + 4], dd[q + 5]), digit_pair(dd[q + 6], dd[q + 7]), row[e][1]);
-                s[t][e] = limb_combine(L, H);
+                s[t][e] = limb_combine_rare(L, H, carry[t][e]);
             }
         }
+    }
+    uint64_t any = 0;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int e = 0; e < 6; e++) any |= carry[t][e];
+    if (__builtin_expect(any != 0, 0)) {
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int e = 0; e < 6; e++) s[t][e] = gl::add_eps(s[t][e], carry[t][e]);
     }
 }
 
@@ -210,16 +233,16 @@ constexpr uint64_t mfma_h(int m)
     return h.v[m];
 }
 
+// The sum of the weights up to h_last (2^32 if one of them is larger).
 template <int HT>
-constexpr uint64_t mfma_h_sum()
+constexpr uint64_t mfma_h_sum(int last)
 {
     uint64_t s = 0;
-    for (int m = 1; m < mfma::kGroupRounds; m++)
-        if (mfma_h<HT>(m) < (1ull << 32)) s += mfma_h<HT>(m);
-    return s;
+    for (int m = 1; m <= last; m++) s += mfma_h<HT>(m) < (1ull << 32) ? mfma_h<HT>(m) : 1ull << 32;
+    return s < (1ull << 32) ? s : 1ull << 32;
 }
-static_assert(mfma_h_sum<kPoseidon>() < (1ull << 30) && mfma_h_sum<kPoseidon2>() < (1ull << 30),
-              "2^47 + sum of weights * 2^32 stays below 2^63");
+static_assert(mfma_h_sum<kPoseidon>(mfma::kGroupRounds - 1) < (1ull << 30) && mfma_h<kPoseidon2>(2) < (1ull << 30),
+              "2^47 + sum of small weights * 2^32 stays below 2^63");
 
 template <int HT, int M, int I>
 __device__ __forceinline__ void add_earlier_small(uint64_t &L, uint64_t &H, const uint64_t *y)
@@ -269,12 +292,30 @@ __device__ __forceinline__ uint64_t sbox_input(const uint32_t (&d)[4], const mfm
     return x;
 }
 
+// The S-box output of that input, in the wave forms of gl64.h.
+template <int HT, int M>
+__device__ __forceinline__ uint64_t sbox_output(const uint32_t (&d)[4], const mfma::Pair &k, const uint64_t *y)
+{
+    uint64_t L = half_sum(d[0], d[1], k.l), H = half_sum(d[2], d[3], k.h);
+    add_earlier_small<HT, M, 0>(L, H, y);
+    // the weights of earlier outputs widen the sum: top < 2^15 + their sum, and
+    // a carry in one of 64 lanes once in 2^26 / top S-boxes
+    if constexpr (mfma_h_sum<HT>(M) < (1ull << 21)) {
+        uint64_t carry;
+        const uint64_t x = limb_combine_rare(L, H, carry);
+        return gl::pow7_wave(x, carry);
+    }
+    uint64_t x = limb_combine(L, H);
+    add_earlier_large<HT, M, 0>(x, y);
+    return gl::pow7_wave(x);
+}
+
 __device__ __forceinline__ void mfma_sboxes(uint64_t s[2][6])
 {
 #pragma unroll
     for (int t = 0; t < 2; t++)
 #pragma unroll
-        for (int e = 0; e < 6; e += 2) gl::pow7_lazy2(s[t][e], s[t][e + 1]);
+        for (int e = 0; e < 6; e += 2) gl::pow7_wave2(s[t][e], s[t][e + 1]);
 }
 
 // This lane's slots 0..11 as B operands.
@@ -337,8 +378,8 @@ __device__ __forceinline__ void permute_mfma(uint64_t s[2][6], const MfmaLds &m)
         uint32_t x[2][2][4];
         mfma_outputs(x, b3, eop + 64 * kOpEntryX);
         uint64_t y[2];
-        y[0] = gl::pow7_lazy(sbox_input<HT, 0>(x[0][0], c_mfma<HT>.x_entry[0], y));
-        y[1] = gl::pow7_lazy(sbox_input<HT, 1>(x[1][0], c_mfma<HT>.x_entry[1], y));
+        y[0] = sbox_output<HT, 0>(x[0][0], c_mfma<HT>.x_entry[0], y);
+        y[1] = sbox_output<HT, 1>(x[1][0], c_mfma<HT>.x_entry[1], y);
         uint64_t y1 = mfma_bytes(y[0]), y2 = mfma_bytes(y[1]);
         swap_halves(y1, y2);
         mf_v4i b[2][4];
@@ -364,11 +405,11 @@ __device__ __forceinline__ void permute_mfma(uint64_t s[2][6], const MfmaLds &m)
         swap_halves(x1, e6);
         const Pair *k = c_mfma<HT>.x_group[g];
         uint64_t y[5];
-        y[0] = gl::pow7_lazy(x1);
-        y[1] = gl::pow7_lazy(sbox_input<HT, 1>(x[0][0], k[0], y));
-        y[2] = gl::pow7_lazy(sbox_input<HT, 2>(x[0][1], k[1], y));
-        y[3] = gl::pow7_lazy(sbox_input<HT, 3>(x[1][0], k[2], y));
-        y[4] = gl::pow7_lazy(sbox_input<HT, 4>(x[1][1], k[3], y));
+        y[0] = gl::pow7_wave(x1);
+        y[1] = sbox_output<HT, 1>(x[0][0], k[0], y);
+        y[2] = sbox_output<HT, 2>(x[0][1], k[1], y);
+        y[3] = sbox_output<HT, 3>(x[1][0], k[2], y);
+        y[4] = sbox_output<HT, 4>(x[1][1], k[3], y);
 #pragma unroll
         for (int i = 0; i < 5; i++) y[i] = mfma_bytes(y[i]);
         e6 = mfma_bytes(e6);
