@@ -126,3 +126,42 @@ def test_invalid_lde_arguments(zk):
     with pytest.raises(zk.ZeknoxError) as e:
         zk.lde_batch(0, out, x, 3, zk.NTTConfig(batches=1, extension_rate_bits=0))
     assert e.value.code == 1
+
+
+# The passes compute on lazy values and leave out what a random operand needs
+# once in 2^32, doing a tile again exactly where it was needed after all.
+# Words at and above p, runs of -1 and multiples of 2^48 reach that in every
+# kernel: single tiles (ragged and whole), one- and two-round strided passes
+# of each stage count, in place, through the coset and from coefficients.
+def rare_words(count, seed):
+    rng = np.random.default_rng(seed)
+    special = np.array([0, 0, 1, 2, P - 2, P - 1, P - 1, P, P + 1, 2**64 - 2, 2**64 - 1, 2**32 - 1, 1 << 32, 1 << 48, 3 << 48,
+                        0xFFFF << 48, 1 << 63], dtype=np.uint64)
+    x = special[rng.integers(0, len(special), count)]
+    some = rng.random(count) < 0.05
+    x[some] = rng.integers(0, 2**64, int(some.sum()), dtype=np.uint64)
+    return x
+
+
+@pytest.mark.parametrize("lg,B", [(1, 5), (3, 3), (4, 7), (7, 2), (11, 3), (12, 2), (13, 3), (14, 2), (15, 1), (16, 2), (17, 1),
+                                  (18, 1), (19, 1), (20, 1), (21, 1)])
+@pytest.mark.parametrize("inverse", [False, True])
+@pytest.mark.parametrize("coset", [False, True])
+def test_ntt_of_rare_words_vs_oracle(zk, lg, B, inverse, coset):
+    print(f"ntt lg={lg} B={B} inverse={inverse} coset={coset}", flush=True)
+    x = rare_words(B << lg, 3 * lg + B + 2 * inverse + coset)
+    buf = x.copy()
+    (zk.intt_batch if inverse else zk.ntt_batch)(0, buf, lg, zk.NTTConfig(batches=B, with_coset=coset))
+    assert np.array_equal(buf, ob.ntt(x % np.uint64(P), lg, B, inverse, coset))
+
+
+@pytest.mark.parametrize("lg_n,rate,B", [(1, 1, 3), (4, 2, 3), (9, 1, 5), (12, 1, 3), (13, 2, 1), (14, 1, 1), (15, 1, 3), (16, 2, 1),
+                                         (17, 1, 1), (18, 1, 1), (19, 1, 1), (20, 1, 1)])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_lde_of_rare_words_vs_oracle(zk, lg_n, rate, B, inverse):
+    print(f"lde lg_n={lg_n} rate={rate} B={B} inverse={inverse}", flush=True)
+    x = rare_words(B << lg_n, 7 * lg_n + rate + B + inverse)
+    out = np.zeros(B << (lg_n + rate), np.uint64)
+    zk.lde_batch(0, out, x, lg_n, zk.NTTConfig(batches=B, extension_rate_bits=rate, with_coset=not inverse),
+                 direction=zk.INVERSE if inverse else zk.FORWARD)
+    assert np.array_equal(out, ob.lde(x % np.uint64(P), lg_n, rate, B, inverse=inverse, coset=not inverse))

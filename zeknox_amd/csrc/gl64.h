@@ -449,7 +449,11 @@ __device__ __forceinline__ void pow7_lazy2(uint64_t &x, uint64_t &y)
 // costs two of the seven instructions.  These forms leave it out,
 //   r = z + c * EPS   (exact unless b),
 // and or the borrow lanes into `bad`: a caller whose mask comes back nonzero
-// throws the results away and takes the exact form.  Per product 12
+// throws the results away and takes the exact form.  The masks are or-ed
+// where they are made, by the scalar unit, which waits for them: the compiler
+// could take them through a VGPR, whose move needs wait states that it does
+// not count after inline asm.  (A call with a mask that is not uniform does
+// not compile.)  Per product 12
 // instructions instead of 14; 32 commits of 135 x 2^15 51.4 -> 48.8 ms,
 // Poseidon2 400 x 2^20 40.1 -> 38.0 ms (alternating builds).  A wave alone on
 // its SIMD loses by it: it waits out the branches.
@@ -467,12 +471,13 @@ __device__ __forceinline__ uint64_t reduce128_rare(uint64_t lo, uint64_t hi, uin
     uint64_t b1, b;
     asm("v_subb_co_u32_e64 %[zlo], %[b1], %[ulo], %[h1], %[cin]\n\t"
         "s_nop 1\n\t"
-        "v_subb_co_u32_e64 %[zhi], %[b], %[uhi], 0, %[b1]"
-        : [zlo] "=&v"(zlo), [zhi] "=&v"(zhi), [b1] "=&s"(b1), [b] "=&s"(b)
-        : [ulo] "v"(lo32(u)), [uhi] "v"(hi32(u)), [h1] "v"(hi32(hi)), [cin] "s"(cin));
+        "v_subb_co_u32_e64 %[zhi], %[b], %[uhi], 0, %[b1]\n\t"
+        "s_or_b64 %[bad], %[bad], %[b]"
+        : [zlo] "=&v"(zlo), [zhi] "=&v"(zhi), [b1] "=&s"(b1), [b] "=&s"(b), [bad] "+s"(bad)
+        : [ulo] "v"(lo32(u)), [uhi] "v"(hi32(u)), [h1] "v"(hi32(hi)), [cin] "s"(cin)
+        : "scc");
     uint64_t r, j;
     asm("v_mad_u64_u32 %[r], %[j], %[cv], -1, %[z]" : [r] "=&v"(r), [j] "=&s"(j) : [cv] "v"(cv), [z] "v"(pack(zlo, zhi)));
-    bad |= b;
     return r;
 }
 
@@ -494,11 +499,14 @@ __device__ __forceinline__ void reduce128_rare2(uint64_t lo0, uint64_t hi0, uint
         "v_subb_co_u32_e64 %[zl1], %[b11], %[ul1], %[h11], %[ci1]\n\t"
         "s_nop 0\n\t"
         "v_subb_co_u32_e64 %[zh0], %[b0], %[uh0], 0, %[b10]\n\t"
-        "v_subb_co_u32_e64 %[zh1], %[b1], %[uh1], 0, %[b11]"
+        "v_subb_co_u32_e64 %[zh1], %[b1], %[uh1], 0, %[b11]\n\t"
+        "s_or_b64 %[bad], %[bad], %[b0]\n\t"
+        "s_or_b64 %[bad], %[bad], %[b1]"
         : [zl0] "=&v"(zl0), [zh0] "=&v"(zh0), [zl1] "=&v"(zl1), [zh1] "=&v"(zh1), [b10] "=&s"(b10), [b0] "=&s"(b0),
-          [b11] "=&s"(b11), [b1] "=&s"(b1)
+          [b11] "=&s"(b11), [b1] "=&s"(b1), [bad] "+s"(bad)
         : [ul0] "v"(lo32(u0)), [uh0] "v"(hi32(u0)), [h10] "v"(hi32(hi0)), [ul1] "v"(lo32(u1)), [uh1] "v"(hi32(u1)),
-          [h11] "v"(hi32(hi1)), [ci0] "s"(cin0), [ci1] "s"(cin1));
+          [h11] "v"(hi32(hi1)), [ci0] "s"(cin0), [ci1] "s"(cin1)
+        : "scc");
     uint64_t j0, j1;
     asm("v_mad_u64_u32 %[r], %[j], %[cv], -1, %[z]"
         : [r] "=&v"(r0), [j] "=&s"(j0)
@@ -506,7 +514,6 @@ __device__ __forceinline__ void reduce128_rare2(uint64_t lo0, uint64_t hi0, uint
     asm("v_mad_u64_u32 %[r], %[j], %[cv], -1, %[z]"
         : [r] "=&v"(r1), [j] "=&s"(j1)
         : [cv] "v"(cv1), [z] "v"(pack(zl1, zh1)));
-    bad |= b0 | b1;
 }
 
 __device__ __forceinline__ uint64_t mul_rare(uint64_t a, uint64_t b, uint64_t &bad)
@@ -544,6 +551,115 @@ __device__ __forceinline__ uint64_t add_eps(uint64_t u, uint64_t lanes)
         : [r] "=&v"(r), [j] "=&s"(j), [cv] "=&v"(cv)
         : [u] "v"(u), [m] "s"(lanes));
     return r;
+}
+
+// ---- butterflies of transforms: sums, differences and products of lazy values
+//
+// A sum whose carry or a difference whose borrow has been folded in as EPS
+// carries or borrows again only if an operand was not canonical (a random
+// lazy product is not once in 2^32).  Those lanes go to `bad` as above.  A
+// butterfly is 9 instructions here and its product 12, against 12 and 18 in
+// canonical form.
+
+// s = a + b, d = a - b, for two pairs at once: every lane mask is read at
+// least two instructions after its write.
+__device__ __forceinline__ void add_sub_rare2(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_t &s0,
+                                              uint64_t &d0, uint64_t &s1, uint64_t &d1, uint64_t &bad)
+{
+    uint32_t sl0, sh0, dl0, dh0, cv0, bv0, sl1, sh1, dl1, dh1, cv1, bv1;
+    uint64_t mc0, mb0, mc1, mb1;
+    asm("v_add_co_u32_e64 %[sl0], %[c0], %[al0], %[bl0]\n\t"
+        "v_sub_co_u32_e64 %[dl0], %[b0], %[al0], %[bl0]\n\t"
+        "v_add_co_u32_e64 %[sl1], %[c1], %[al1], %[bl1]\n\t"
+        "v_sub_co_u32_e64 %[dl1], %[b1], %[al1], %[bl1]\n\t"
+        "v_addc_co_u32_e64 %[sh0], %[c0], %[ah0], %[bh0], %[c0]\n\t"
+        "v_subb_co_u32_e64 %[dh0], %[b0], %[ah0], %[bh0], %[b0]\n\t"
+        "v_addc_co_u32_e64 %[sh1], %[c1], %[ah1], %[bh1], %[c1]\n\t"
+        "v_subb_co_u32_e64 %[dh1], %[b1], %[ah1], %[bh1], %[b1]\n\t"
+        "v_cndmask_b32_e64 %[cv0], 0, 1, %[c0]\n\t"
+        "v_cndmask_b32_e64 %[bv0], 0, -1, %[b0]\n\t"
+        "v_cndmask_b32_e64 %[cv1], 0, 1, %[c1]\n\t"
+        "v_cndmask_b32_e64 %[bv1], 0, -1, %[b1]\n\t"
+        "v_sub_co_u32_e64 %[dl0], %[b0], %[dl0], %[bv0]\n\t"
+        "v_sub_co_u32_e64 %[dl1], %[b1], %[dl1], %[bv1]\n\t"
+        "s_nop 0\n\t"
+        "v_subb_co_u32_e64 %[dh0], %[b0], %[dh0], 0, %[b0]\n\t"
+        "v_subb_co_u32_e64 %[dh1], %[b1], %[dh1], 0, %[b1]\n\t"
+        "s_or_b64 %[bad], %[bad], %[b0]\n\t"
+        "s_or_b64 %[bad], %[bad], %[b1]"
+        : [sl0] "=&v"(sl0), [sh0] "=&v"(sh0), [dl0] "=&v"(dl0), [dh0] "=&v"(dh0), [cv0] "=&v"(cv0), [bv0] "=&v"(bv0),
+          [sl1] "=&v"(sl1), [sh1] "=&v"(sh1), [dl1] "=&v"(dl1), [dh1] "=&v"(dh1), [cv1] "=&v"(cv1), [bv1] "=&v"(bv1),
+          [c0] "=&s"(mc0), [b0] "=&s"(mb0), [c1] "=&s"(mc1), [b1] "=&s"(mb1), [bad] "+s"(bad)
+        : [al0] "v"(lo32(a0)), [ah0] "v"(hi32(a0)), [bl0] "v"(lo32(b0)), [bh0] "v"(hi32(b0)), [al1] "v"(lo32(a1)),
+          [ah1] "v"(hi32(a1)), [bl1] "v"(lo32(b1)), [bh1] "v"(hi32(b1))
+        : "scc");
+    uint64_t k0, k1;
+    asm("v_mad_u64_u32 %[r0], %[k0], %[cv0], -1, %[s0]\n\t"
+        "v_mad_u64_u32 %[r1], %[k1], %[cv1], -1, %[s1]\n\t"
+        "s_or_b64 %[bad], %[bad], %[k0]\n\t"
+        "s_or_b64 %[bad], %[bad], %[k1]"
+        : [r0] "=&v"(s0), [k0] "=&s"(k0), [r1] "=&v"(s1), [k1] "=&s"(k1), [bad] "+s"(bad)
+        : [cv0] "v"(cv0), [s0] "v"(pack(sl0, sh0)), [cv1] "v"(cv1), [s1] "v"(pack(sl1, sh1))
+        : "scc");
+    d0 = pack(dl0, dh0);
+    d1 = pack(dl1, dh1);
+}
+
+// x * 2^E, lazy, for E < 96 and any x < 2^64: with x * 2^(E mod 32) =
+// x0 + x1 * 2^32 + x2 * 2^64 (x2 < 2^32),
+//   E < 32       x0 + x1 * 2^32 + x2 * EPS
+//   32 <= E < 64 x0 * 2^32 + x1 * EPS - x2
+//   64 <= E      x0 * EPS - (x1 + x2 * 2^32).
+template <int E>
+__device__ __forceinline__ uint64_t mul_pow2_rare(uint64_t x, uint64_t &bad)
+{
+    static_assert(E >= 0 && E < 96, "exponent below half the order of 2");
+    constexpr int s = E % 32;
+    const uint64_t l = x << s;
+    const uint32_t x2 = s ? (uint32_t)(x >> ((64 - s) & 63)) : 0u;
+    if constexpr (E == 0) return x;
+    else if constexpr (E < 32) return reduce96_lazy(l, x2);
+    else if constexpr (E == 32) return shl32_lazy(x);
+    else if constexpr (E < 64) {
+        // lo + hi * 2^64 with lo = x0 * 2^32, hi = (x1, x2): reduce128_rare without a borrow in
+        uint64_t u, sc;
+        uint32_t cv;
+        asm("v_mad_u64_u32 %[u], %[sc], %[h0], -1, %[lo]\n\t"
+            "s_nop 1\n\t"
+            "v_cndmask_b32_e64 %[cv], 0, 1, %[sc]"
+            : [u] "=&v"(u), [sc] "=&s"(sc), [cv] "=&v"(cv)
+            : [h0] "v"(hi32(l)), [lo] "v"(pack(0u, lo32(l))));
+        uint32_t zlo, zhi;
+        uint64_t b;
+        asm("v_sub_co_u32_e64 %[zlo], %[b], %[ulo], %[h1]\n\t"
+            "s_nop 1\n\t"
+            "v_subb_co_u32_e64 %[zhi], %[b], %[uhi], 0, %[b]\n\t"
+            "s_or_b64 %[bad], %[bad], %[b]"
+            : [zlo] "=&v"(zlo), [zhi] "=&v"(zhi), [b] "=&s"(b), [bad] "+s"(bad)
+            : [ulo] "v"(lo32(u)), [uhi] "v"(hi32(u)), [h1] "v"(x2)
+            : "scc");
+        uint64_t r, j;
+        asm("v_mad_u64_u32 %[r], %[j], %[cv], -1, %[z]" : [r] "=&v"(r), [j] "=&s"(j) : [cv] "v"(cv), [z] "v"(pack(zlo, zhi)));
+        return r;
+    } else {
+        // the subtrahend is below 2^62, so the second borrow cannot be: a
+        // first one leaves at least 2^64 - 2^62
+        static_assert(s <= 30, "x2 below 2^30");
+        const uint64_t y = mul_eps(lo32(l));
+        uint32_t dlo, dhi, bv;
+        uint64_t b;
+        asm("v_sub_co_u32_e64 %[dlo], %[b], %[yl], %[h0]\n\t"
+            "s_nop 1\n\t"
+            "v_subb_co_u32_e64 %[dhi], %[b], %[yh], %[h1], %[b]\n\t"
+            "s_nop 1\n\t"
+            "v_cndmask_b32_e64 %[bv], 0, -1, %[b]\n\t"
+            "v_sub_co_u32_e64 %[dlo], %[b], %[dlo], %[bv]\n\t"
+            "s_nop 1\n\t"
+            "v_subb_co_u32_e64 %[dhi], %[b], %[dhi], 0, %[b]"
+            : [dlo] "=&v"(dlo), [dhi] "=&v"(dhi), [bv] "=&v"(bv), [b] "=&s"(b)
+            : [yl] "v"(lo32(y)), [yh] "v"(hi32(y)), [h0] "v"(hi32(l)), [h1] "v"(x2));
+        return pack(dlo, dhi);
+    }
 }
 
 // x^7 of a wave whose branch is uniform: the products above, and the exact

@@ -88,17 +88,114 @@ __device__ __forceinline__ uint64_t tile_step(const NttPass &a, int i)
     return (uint64_t)i << (lt - a.c + a.s_lo);
 }
 
+// ---- arithmetic of the passes
+//
+// A butterfly is 21 instructions on lazy values (Lazy) rather than 30 on
+// canonical ones (Exact): what a random operand needs once in 2^32 is left
+// out and its lanes noted in `bad` (gl64.h).  A tile with such a lane is
+// computed again with Exact, from the source that nothing has overwritten
+// yet.  Words between the passes of a transform are lazy too; the contiguous
+// pass, the last, stores canonical ones.
+//
+// Bounds, 64 x 2^20 forward (1.07 GB of traffic a pass): the 12-stage
+// contiguous pass 375 -> 318 us, of which its loads and stores alone take
+// 273; the 8-stage strided pass 298 -> 294 us, bound by its loads and stores
+// (250 alone).  The whole transform 906 -> 854 us, alternating builds.
+
+struct Lazy {
+    uint64_t bad = 0;
+    static __device__ __forceinline__ uint64_t load(uint64_t x) { return x; }
+    static __device__ __forceinline__ uint64_t result(uint64_t x) { return gl::canon(x); }
+    __device__ __forceinline__ void add_sub2(uint64_t &x0, uint64_t &y0, uint64_t &x1, uint64_t &y1)
+    {
+        uint64_t s0, d0, s1, d1;
+        gl::add_sub_rare2(x0, y0, x1, y1, s0, d0, s1, d1, bad);
+        x0 = s0, y0 = d0, x1 = s1, y1 = d1;
+    }
+    __device__ __forceinline__ void mul2(uint64_t &x0, uint64_t w0, uint64_t &x1, uint64_t w1)
+    {
+        uint64_t r0, r1;
+        gl::mul_rare2(x0, w0, x1, w1, r0, r1, bad);
+        x0 = r0, x1 = r1;
+    }
+    __device__ __forceinline__ uint64_t mul(uint64_t x, uint64_t w) { return gl::mul_rare(x, w, bad); }
+    template <int E>
+    __device__ __forceinline__ uint64_t shift(uint64_t x)
+    {
+        return gl::mul_pow2_rare<E>(x, bad);
+    }
+};
+
+struct Exact {
+    static __device__ __forceinline__ uint64_t load(uint64_t x) { return gl::canon(x); }
+    static __device__ __forceinline__ uint64_t result(uint64_t x) { return x; }
+    __device__ __forceinline__ void add_sub2(uint64_t &x0, uint64_t &y0, uint64_t &x1, uint64_t &y1)
+    {
+        const uint64_t s0 = gl::add(x0, y0), d0 = gl::sub(x0, y0), s1 = gl::add(x1, y1), d1 = gl::sub(x1, y1);
+        x0 = s0, y0 = d0, x1 = s1, y1 = d1;
+    }
+    __device__ __forceinline__ void mul2(uint64_t &x0, uint64_t w0, uint64_t &x1, uint64_t w1)
+    {
+        x0 = mul(x0, w0);
+        x1 = mul(x1, w1);
+    }
+    // (the form with the fewest live registers)
+    __device__ __forceinline__ uint64_t mul(uint64_t x, uint64_t w) { return gl::mul_nc(x, w); }
+    template <int E>
+    __device__ __forceinline__ uint64_t shift(uint64_t x)
+    {
+        // (x is canonical; the compiler folds a canon() that directly follows a
+        // sub() into its carry chain and counts the wrap of that as its own)
+        if constexpr (E == 0) return x;
+        else return gl::mul_pow2<E>(x);
+    }
+};
+
+// The stage whose partners differ in bit b of the register index, w(e) the
+// twiddle of element e's butterfly.
+template <class A, class W>
+__device__ __forceinline__ void reg_stage(A &ar, uint64_t (&x)[kNttPerThread], int b, W &&w)
+{
+#pragma unroll
+    for (int k = 0; k < kNttPerThread / 2; k += 2) {
+        const int e0 = ((k >> b) << (b + 1)) | (k & ((1 << b) - 1));
+        const int e1 = (((k + 1) >> b) << (b + 1)) | ((k + 1) & ((1 << b) - 1));
+        const int f0 = e0 | (1 << b), f1 = e1 | (1 << b);
+        ar.add_sub2(x[e0], x[f0], x[e1], x[f1]);
+        ar.mul2(x[f0], w(e0), x[f1], w(e1));
+    }
+}
+
+// The lane and tile of the second computation, through values the compiler
+// cannot see through: nothing the first one loaded or computed stays in
+// registers for it.
+__device__ __forceinline__ void again(uint32_t &t, uint64_t &tile)
+{
+    asm volatile("; again %0 %1" : "+v"(t), "+s"(tile));
+}
+
+// Whether any wave of the work-group noted a lane; ends with every LDS write
+// before it visible.
+__device__ __forceinline__ bool barrier_any(uint32_t *flags, uint64_t bad)
+{
+    if ((threadIdx.x & 63) == 0) flags[threadIdx.x >> 6] = bad != 0 ? 1u : 0u;
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int i = 0; i < kNttThreads / 64; i++) any |= flags[i];
+    return __builtin_amdgcn_readfirstlane(any) != 0;
+}
+
 // One register round: stages on j-bits [b0, b0+K) (u-bits [RB, RB+K)).
 // Lane t holds the 2^K elements that differ in those bits, repeated over
 // 2^(4-K) groups taken from the extra element bits; the other u-bits come
 // from the lane id.  The twiddle of stage d for element e depends only on
 // (j mod 2^d) << s_lo | lo.
-template <bool CONTIG, int K>
-__device__ __forceinline__ void ntt_round(uint64_t *lds, const NttPass &a, uint32_t t, uint32_t b0, uint32_t jpos,
-                                          uint64_t lo_base)
+template <int K, class A>
+__device__ __forceinline__ void ntt_round(A &ar, uint64_t *lds, const NttPass &a, uint32_t t, uint64_t lo_base)
 {
     constexpr int E = kNttPerThread;
-    const uint32_t RB = jpos + b0;
+    const uint32_t RB = a.c;
     uint64_t x[E];
     uint32_t uu[E];
 #pragma unroll
@@ -111,27 +208,13 @@ __device__ __forceinline__ void ntt_round(uint64_t *lds, const NttPass &a, uint3
     }
 #pragma unroll
     for (int dd = K - 1; dd >= 0; dd--) {
-        const uint32_t d = b0 + (uint32_t)dd;
-        const uint32_t lg = a.s_lo + d + 1;
-        const uint64_t *tab = !CONTIG ? stage_table(a, lg) : nullptr;
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            if ((e >> dd) & 1) continue;
-            const int f = e | (1 << dd);
-            const uint32_t u = uu[e];
-            const uint32_t j = !CONTIG ? (u >> a.c) : (u & ((1u << a.m) - 1));
-            uint64_t w;
-            if constexpr (CONTIG) {
-                w = tw12_at(a, (j & ((1u << d) - 1)) << (kNttTileLog - 1 - d));
-            } else {
-                const uint64_t lo_part = lo_base + (u & ((1u << a.c) - 1));
-                const uint64_t ex = (((uint64_t)(j & ((1u << d) - 1))) << a.s_lo) | lo_part;
-                w = tw_at(tab, lg, ex, a.inverse);
-            }
-            const uint64_t y0 = x[e], y1 = x[f];
-            x[e] = gl::add(y0, y1);
-            x[f] = gl::mul(gl::sub(y0, y1), w);
-        }
+        const uint32_t lg = a.s_lo + (uint32_t)dd + 1;
+        const uint64_t *tab = stage_table(a, lg);
+        reg_stage(ar, x, dd, [&](int e) {
+            const uint32_t u = uu[e], j = u >> a.c;
+            const uint64_t lo_part = lo_base + (u & ((1u << a.c) - 1));
+            return tw_at(tab, lg, ((uint64_t)(j & ((1u << dd) - 1)) << a.s_lo) | lo_part, a.inverse);
+        });
     }
 #pragma unroll
     for (int e = 0; e < E; e++) lds[lds_slot(uu[e])] = x[e];
@@ -139,9 +222,9 @@ __device__ __forceinline__ void ntt_round(uint64_t *lds, const NttPass &a, uint3
 
 // Full-width round (K = 4, no extra element bits): the lane's other u-bits
 // are its id, so the 15 distinct twiddles of the round are loaded once.
-template <bool CONTIG>
-__device__ __forceinline__ void ntt_round4(uint64_t *lds, const NttPass &a, uint32_t t, uint32_t b0, uint32_t jpos,
-                                           uint64_t lo_base)
+template <bool CONTIG, class A>
+__device__ __forceinline__ void ntt_round4(A &ar, uint64_t *lds, const NttPass &a, uint32_t t, uint32_t b0,
+                                           uint32_t jpos, uint64_t lo_base)
 {
     constexpr int E = kNttPerThread;
     const uint32_t RB = jpos + b0;
@@ -168,14 +251,7 @@ __device__ __forceinline__ void ntt_round4(uint64_t *lds, const NttPass &a, uint
 #pragma unroll
             for (int v = 0; v < (1 << dd); v++) w[v] = tw_at(tab, lg, base + ((uint64_t)v << (b0 + a.s_lo)), a.inverse);
         }
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            if ((e >> dd) & 1) continue;
-            const int f = e | (1 << dd);
-            const uint64_t y0 = x[e], y1 = x[f];
-            x[e] = gl::add(y0, y1);
-            x[f] = gl::mul(gl::sub(y0, y1), w[e & ((1 << dd) - 1)]);
-        }
+        reg_stage(ar, x, dd, [&](int e) { return w[e & ((1 << dd) - 1)]; });
     }
 #pragma unroll
     for (int e = 0; e < E; e++) lds[lds_slot(ubase | ((uint32_t)e << RB))] = x[e];
@@ -185,7 +261,8 @@ __device__ __forceinline__ void ntt_round4(uint64_t *lds, const NttPass &a, uint
 //
 // With b0 = 0 the round covers the K lowest stages; stage d's twiddle for
 // element e is w_{2^(d+1)}^v with v = e mod 2^d, a root of order <= 16:
-// w = 1 (no product) or a power of two (a shift, mul_pow2).
+// w = 1 (no product) or a power of two (a shift; 2^96 = -1 is the difference
+// taken the other way round).
 
 template <int I, int N, class F>
 __device__ __forceinline__ void static_for(F &&f)
@@ -196,38 +273,41 @@ __device__ __forceinline__ void static_for(F &&f)
     }
 }
 
-// x * w_{2^(D+1)}^V (w^-V for the inverse), x canonical
+// e with 2^e = w_{2^(D+1)}^V (w^-V for the inverse)
 template <int D, int V, bool INV>
-__device__ __forceinline__ uint64_t small_root_mul(uint64_t x)
+constexpr int small_root_log()
 {
     constexpr int L = gl::clog2(gl::comega(D + 1));
     static_assert(L >= 0, "the 2^(D+1)-th root of unity of the transform is a power of two");
     constexpr int E0 = (V * L) % 192;
-    constexpr int E = INV ? (192 - E0) % 192 : E0;
-    if constexpr (E == 0) return x;
-    else return gl::mul_pow2<E>(x);
+    return INV ? (192 - E0) % 192 : E0;
 }
 
-template <int DD, bool INV>
-__device__ __forceinline__ void last_stages(uint64_t (&x)[kNttPerThread])
+template <int DD, bool INV, class A>
+__device__ __forceinline__ void last_stages(A &ar, uint64_t (&x)[kNttPerThread])
 {
-    static_for<0, kNttPerThread>([&](auto ec) {
-        constexpr int e = decltype(ec)::value;
-        if constexpr (!((e >> DD) & 1)) {
-            constexpr int f = e | (1 << DD);
-            const uint64_t y0 = x[e], y1 = x[f];
-            x[e] = gl::add(y0, y1);
-            x[f] = small_root_mul<DD, (e & ((1 << DD) - 1)), INV>(gl::sub(y0, y1));
-        }
+    static_for<0, kNttPerThread / 4>([&](auto kc) {
+        constexpr int k = 2 * decltype(kc)::value;
+        constexpr int e0 = ((k >> DD) << (DD + 1)) | (k & ((1 << DD) - 1)), f0 = e0 | (1 << DD);
+        constexpr int e1 = (((k + 1) >> DD) << (DD + 1)) | ((k + 1) & ((1 << DD) - 1)), f1 = e1 | (1 << DD);
+        constexpr int E0 = small_root_log<DD, (e0 & ((1 << DD) - 1)), INV>();
+        constexpr int E1 = small_root_log<DD, (e1 & ((1 << DD) - 1)), INV>();
+        uint64_t a0 = E0 >= 96 ? x[f0] : x[e0], b0 = E0 >= 96 ? x[e0] : x[f0];
+        uint64_t a1 = E1 >= 96 ? x[f1] : x[e1], b1 = E1 >= 96 ? x[e1] : x[f1];
+        ar.add_sub2(a0, b0, a1, b1);
+        x[e0] = a0;
+        x[e1] = a1;
+        x[f0] = ar.template shift<E0 % 96>(b0);
+        x[f1] = ar.template shift<E1 % 96>(b1);
     });
-    if constexpr (DD > 0) last_stages<DD - 1, INV>(x);
+    if constexpr (DD > 0) last_stages<DD - 1, INV>(ar, x);
 }
 
 // The round on stages K-1..0 of a contiguous pass (lane t holds the 2^K
-// elements u = (other << K) | rb, other = t | group << 8): ntt_round /
-// ntt_round4 with b0 = 0, twiddles folded in at compile time.
-template <int K, bool INV>
-__device__ __forceinline__ void ntt_round_last(uint64_t *lds, uint32_t t)
+// elements u = (other << K) | rb, other = t | group << 8): ntt_round4 with
+// b0 = 0, twiddles folded in at compile time.
+template <int K, bool INV, class A>
+__device__ __forceinline__ void ntt_round_last(A &ar, uint64_t *lds, uint32_t t)
 {
     constexpr int E = kNttPerThread;
     uint64_t x[E];
@@ -239,126 +319,35 @@ __device__ __forceinline__ void ntt_round_last(uint64_t *lds, uint32_t t)
         uu[e] = (other << K) | rb;
         x[e] = lds[lds_slot(uu[e])];
     }
-    last_stages<K - 1, INV>(x);
+    last_stages<K - 1, INV>(ar, x);
 #pragma unroll
-    for (int e = 0; e < E; e++) lds[lds_slot(uu[e])] = x[e];
+    for (int e = 0; e < E; e++) lds[lds_slot(uu[e])] = A::result(x[e]);
 }
 
-template <int K>
-__device__ __forceinline__ void ntt_round_last(uint64_t *lds, uint32_t t, bool inverse)
+template <int K, class A>
+__device__ __forceinline__ void ntt_round_last(A &ar, uint64_t *lds, uint32_t t, bool inverse)
 {
-    if (inverse) ntt_round_last<K, true>(lds, t);
-    else ntt_round_last<K, false>(lds, t);
+    if (inverse) ntt_round_last<K, true>(ar, lds, t);
+    else ntt_round_last<K, false>(ar, lds, t);
 }
 
-// `passes` (npasses > 0, device memory) lists independent passes sorted by
-// tile_begin; with npasses == 0 the launch runs the single pass `one`.
-// CONTIG: every pass of the launch is contiguous (s_lo == 0), else strided.
-// Work-group k runs tile first + k of the list (a launch may cover a range).
-// Four work-groups per CU: 33 KB of LDS and at most 128 VGPRs each.
-template <bool CONTIG>
-__global__ void __launch_bounds__(kNttThreads) __attribute__((amdgpu_waves_per_eu(4)))
-k_ntt_tiles(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
+// Stages rem-1..0 of a contiguous pass, whose words are in LDS; the last
+// round's writes are left to the caller's barrier.
+template <class A>
+__device__ __forceinline__ void contig_rounds(A &ar, uint64_t *lds, const NttPass &a, uint32_t t, uint32_t rem)
 {
-    __shared__ uint64_t lds[(1 << kNttTileLog) + (1 << kNttTileLog) / 32];
-
-    // locate this work-group's pass (uniform)
-    const uint64_t bid = first + blockIdx.x;
-    uint32_t lo = 0, hi = npasses;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (passes[mid].tile_begin <= bid) lo = mid;
-        else hi = mid;
-    }
-    const NttPass a = npasses ? passes[lo] : one;
-    const uint64_t tile = bid - a.tile_begin;
-    const uint32_t t = threadIdx.x;
-
-    // ---- load, coalesced: lane t takes positions t + 256 i, all 16 in flight,
-    // at its own index plus a uniform step.  Only a contiguous pass over
-    // blocks shorter than a tile can end inside a tile (strided passes have
-    // L > 12, so every tile is full).
-    const uint64_t ibase = tile_index(a, tile, t);
-    const bool ragged = CONTIG && (a.total & ((1ull << kNttTileLog) - 1)) != 0;
-    const gptr<uint64_t> bufp = gmem(a.buf) + ibase;
-    // A strided pass reading through a mode is the first pass (s_lo + m = L):
-    // its tile lies in one block of 2^L, so the LDE source row and the factor
-    // (or coset) row follow the index at fixed offsets.
-    gptr<const uint64_t> srcp = nullptr, facp = nullptr;
-    if (!CONTIG && a.mode != kSrcInPlace) {
-        const uint64_t blk = ibase >> a.L;
-        const uint64_t pos0 = ibase - (blk << a.L);
-        if (a.mode == kSrcLde) {
-            // first `rate` DIF stages of the zero-padded column: block b of
-            // column col holds a_i * F[b*n + i], F the resident factor table
-            srcp = gmem(a.src) + ((blk >> a.rate) << a.L) + pos0;
-            facp = gmem(a.coset) + ((blk & ((1ull << a.rate) - 1)) << a.L) + pos0;
-        } else {
-            facp = gmem(a.coset) + pos0;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < kNttPerThread; i++) {
-        const uint32_t u = t + kNttThreads * i;
-        const uint64_t st = tile_step(a, i);
-        uint64_t v = 0;
-        if constexpr (CONTIG) {
-            const uint64_t idx = ibase + st;
-            if (!ragged || idx < a.total) {
-                if (a.mode == kSrcLde) {
-                    const uint64_t n = 1ull << a.L;
-                    const uint64_t col = idx >> (a.L + a.rate), pos = idx & (n - 1);
-                    v = gl::mul(gmem(a.src)[(col << a.L) + pos], gmem(a.coset)[idx & ((n << a.rate) - 1)]);
-                } else {
-                    v = bufp[st];
-                    if (a.mode == kSrcCoset) v = gl::mul(v, gmem(a.coset)[idx & ((1ull << a.L) - 1)]);
-                }
-            }
-        } else {
-            if (a.mode == kSrcLde) {
-                v = gl::mul(srcp[st], facp[st]);
-            } else {
-                v = bufp[st];
-                if (a.mode == kSrcCoset) v = gl::mul(v, facp[st]);
-            }
-        }
-        lds[lds_slot(u)] = v;
-    }
-    __syncthreads();
-
-    // low in-block bits shared by the tile's columns (strided passes)
-    const uint64_t lo_base = !CONTIG ? ((tile & ((1ull << (a.s_lo - a.c)) - 1)) << a.c) : 0;
-    const uint32_t jpos = !CONTIG ? a.c : 0;  // u-bit of j-bit 0
-
-    // ---- register rounds, top j-bits first: 4 stages each, then the rest
-    uint32_t rem = a.m;
-    while (rem >= 4) {
+    while (rem > 4) {
         rem -= 4;
-        if (CONTIG && rem == 0) ntt_round_last<4>(lds, t, a.inverse);
-        else ntt_round4<CONTIG>(lds, a, t, rem, jpos, lo_base);
+        ntt_round4<true>(ar, lds, a, t, rem, 0, 0);
         __syncthreads();
     }
-    if constexpr (CONTIG) {
-        if (rem == 3) ntt_round_last<3>(lds, t, a.inverse);
-        else if (rem == 2) ntt_round_last<2>(lds, t, a.inverse);
-        else if (rem == 1) ntt_round_last<1>(lds, t, a.inverse);
-    } else {
-        if (rem == 3) ntt_round<CONTIG, 3>(lds, a, t, 0, jpos, lo_base);
-        else if (rem == 2) ntt_round<CONTIG, 2>(lds, a, t, 0, jpos, lo_base);
-        else if (rem == 1) ntt_round<CONTIG, 1>(lds, a, t, 0, jpos, lo_base);
-    }
-    if (rem) __syncthreads();
-
-    // ---- store, coalesced
-#pragma unroll
-    for (int i = 0; i < kNttPerThread; i++) {
-        const uint32_t u = t + kNttThreads * i;
-        const uint64_t st = tile_step(a, i);
-        if (!ragged || ibase + st < a.total) bufp[st] = lds[lds_slot(u)];
-    }
+    if (rem == 4) ntt_round_last<4>(ar, lds, t, a.inverse);
+    else if (rem == 3) ntt_round_last<3>(ar, lds, t, a.inverse);
+    else if (rem == 2) ntt_round_last<2>(ar, lds, t, a.inverse);
+    else if (rem == 1) ntt_round_last<1>(ar, lds, t, a.inverse);
 }
 
-// ---- descriptors of the one-tile-per-work-group kernels
+// ---- descriptors
 //
 // A launch's descriptor list is read through the constant address space
 // (scalar loads into SGPRs; as vector loads they cost 32 VGPRs).
@@ -384,6 +373,130 @@ __device__ __forceinline__ NttPass pass_at(const NttPass *passes, uint32_t npass
     return r;
 }
 
+// The tile of k_ntt_tiles from its source to its results in LDS (a barrier
+// is left to the caller).
+template <bool CONTIG, class A>
+__device__ __forceinline__ void tile_transform(A &ar, uint64_t *lds, const NttPass &a, uint64_t tile, uint32_t t)
+{
+    // ---- load, coalesced: lane t takes positions t + 256 i, all 16 in flight,
+    // at its own index plus a uniform step.  Only a contiguous pass over
+    // blocks shorter than a tile can end inside a tile (strided passes have
+    // L > 12, so every tile is full); its lanes past the end read the last
+    // word, in blocks of their own.
+    const uint64_t ibase = tile_index(a, tile, t);
+    const gptr<const uint64_t> bufp = gmem(a.buf) + ibase;
+    // A strided pass reading through a mode is the first pass (s_lo + m = L):
+    // its tile lies in one block of 2^L, so the LDE source row and the factor
+    // (or coset) row follow the index at fixed offsets.
+    gptr<const uint64_t> srcp = nullptr, facp = nullptr;
+    if (!CONTIG && a.mode != kSrcInPlace) {
+        const uint64_t blk = ibase >> a.L;
+        const uint64_t pos0 = ibase - (blk << a.L);
+        if (a.mode == kSrcLde) {
+            // first `rate` DIF stages of the zero-padded column: block b of
+            // column col holds a_i * F[b*n + i], F the resident factor table
+            srcp = gmem(a.src) + ((blk >> a.rate) << a.L) + pos0;
+            facp = gmem(a.coset) + ((blk & ((1ull << a.rate) - 1)) << a.L) + pos0;
+        } else {
+            facp = gmem(a.coset) + pos0;
+        }
+    }
+    uint64_t x[kNttPerThread], f[kNttPerThread];
+    auto index = [&](int i) {
+        const uint64_t idx = (tile << kNttTileLog) + (t + kNttThreads * i);
+        return idx < a.total ? idx : a.total - 1;
+    };
+    if (a.mode == kSrcLde) {
+        const uint64_t n = 1ull << a.L;
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i++) {
+            if constexpr (CONTIG) {
+                const uint64_t idx = index(i), col = idx >> (a.L + a.rate), pos = idx & (n - 1);
+                x[i] = gmem(a.src)[(col << a.L) + pos];
+                f[i] = gmem(a.coset)[idx & ((n << a.rate) - 1)];
+            } else {
+                x[i] = srcp[tile_step(a, i)];
+                f[i] = facp[tile_step(a, i)];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i++) {
+            if constexpr (CONTIG) x[i] = A::load(gmem(a.buf)[index(i)]);
+            else x[i] = A::load(bufp[tile_step(a, i)]);
+        }
+        if (a.mode == kSrcCoset) {
+#pragma unroll
+            for (int i = 0; i < kNttPerThread; i++) {
+                if constexpr (CONTIG) f[i] = gmem(a.coset)[index(i) & ((1ull << a.L) - 1)];
+                else f[i] = facp[tile_step(a, i)];
+            }
+        }
+    }
+    if (a.mode != kSrcInPlace) {
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i += 2) ar.mul2(x[i], f[i], x[i + 1], f[i + 1]);
+    }
+#pragma unroll
+    for (int i = 0; i < kNttPerThread; i++) lds[lds_slot(t + kNttThreads * i)] = x[i];
+    __syncthreads();
+
+    // ---- register rounds, top j-bits first: 4 stages each, then the rest
+    if constexpr (CONTIG) {
+        contig_rounds(ar, lds, a, t, a.m);
+    } else {
+        // low in-block bits shared by the tile's columns
+        const uint64_t lo_base = (tile & ((1ull << (a.s_lo - a.c)) - 1)) << a.c;
+        uint32_t rem = a.m;
+        while (rem >= 4) {
+            rem -= 4;
+            ntt_round4<false>(ar, lds, a, t, rem, a.c, lo_base);
+            if (rem) __syncthreads();
+        }
+        if (rem == 3) ntt_round<3>(ar, lds, a, t, lo_base);
+        else if (rem == 2) ntt_round<2>(ar, lds, a, t, lo_base);
+        else if (rem == 1) ntt_round<1>(ar, lds, a, t, lo_base);
+    }
+}
+
+// `passes` (npasses > 0, device memory) lists independent passes sorted by
+// tile_begin; with npasses == 0 the launch runs the single pass `one`.
+// CONTIG: every pass of the launch is contiguous (s_lo == 0), else strided.
+// Work-group k runs tile first + k of the list (a launch may cover a range).
+// Four work-groups per CU: 33 KB of LDS and at most 128 VGPRs each.
+template <bool CONTIG>
+__global__ void __launch_bounds__(kNttThreads) __attribute__((amdgpu_waves_per_eu(4)))
+k_ntt_tiles(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
+{
+    __shared__ uint64_t lds[(1 << kNttTileLog) + (1 << kNttTileLog) / 32];
+    __shared__ uint32_t flags[kNttThreads / 64];
+
+    const uint64_t bid = first + blockIdx.x;
+    const NttPass a = pass_at(passes, npasses, one, bid);
+    uint64_t tile = bid - a.tile_begin;
+    uint32_t t = threadIdx.x;
+
+    Lazy lazy;
+    tile_transform<CONTIG>(lazy, lds, a, tile, t);
+    if (__builtin_expect(barrier_any(flags, lazy.bad), 0)) {
+        Exact exact;
+        again(t, tile);
+        tile_transform<CONTIG>(exact, lds, a, tile, t);
+        __syncthreads();
+    }
+
+    // ---- store, coalesced
+    const uint64_t ibase = CONTIG ? (tile << kNttTileLog) + t : tile_index(a, tile, t);
+    const bool ragged = CONTIG && (a.total & ((1ull << kNttTileLog) - 1)) != 0;
+    const gptr<uint64_t> bufp = gmem(a.buf) + ibase;
+#pragma unroll
+    for (int i = 0; i < kNttPerThread; i++) {
+        const uint32_t u = t + kNttThreads * i;
+        const uint64_t st = CONTIG ? (uint64_t)kNttThreads * i : tile_step(a, i);
+        if (!ragged || ibase + st < a.total) bufp[st] = lds[lds_slot(u)];
+    }
+}
+
 // ---- contiguous in-place passes over whole tiles, one tile per work-group
 //
 // Lane t loads the tile's words t + 256 i, which are, for the stages 8..m-1
@@ -393,54 +506,52 @@ __device__ __forceinline__ NttPass pass_at(const NttPass *passes, uint32_t npass
 // w_4096^(that << (3 - dd)) from the global table (16 KB of it in use).  So
 // those stages run on the loaded registers and only the stages below 8 go
 // through LDS (two register rounds, the last with its small roots as
-// shifts).  Four work-groups per CU at 127 VGPRs.  This replaced a
+// shifts).  Four work-groups per CU.  This replaced a
 // persistent kernel that prefetched the next tile and staged the stage
 // twiddles in LDS (three waves per SIMD, 164-168 VGPRs): batched LDE NTT
 // 5.13 -> 4.75 ms per 16 commits, the plain 12-stage pass 0.216 -> 0.198 ms,
 // same GPU, alternating builds.  The kernel takes in-place passes over whole
 // tiles only (ntt_kernel_kind 1); ragged, coset and LDE-source contiguous passes
 // run on k_ntt_tiles.
-__global__ void __launch_bounds__(kNttThreads) __attribute__((amdgpu_waves_per_eu(4)))
-k_ntt_contig_reg(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
+template <class A>
+__device__ __forceinline__ void contig_transform(A &ar, uint64_t *lds, const NttPass &a, uint64_t tile, uint32_t t)
 {
-    __shared__ uint64_t lds[(1 << kNttTileLog) + (1 << kNttTileLog) / 32];
-    const uint32_t t = threadIdx.x;
-    const uint64_t b = first + blockIdx.x;
-    const NttPass a = pass_at(passes, npasses, one, b);
-    const uint64_t tile = b - a.tile_begin;
-    const gptr<uint64_t> p = gmem(a.buf) + (tile << kNttTileLog) + t;
+    const gptr<const uint64_t> p = gmem(a.buf) + (tile << kNttTileLog) + t;
     uint64_t x[kNttPerThread];
 #pragma unroll
-    for (int i = 0; i < kNttPerThread; i++) x[i] = p[i << 8];
+    for (int i = 0; i < kNttPerThread; i++) x[i] = A::load(p[i << 8]);
 #pragma unroll
     for (int dd = 3; dd >= 0; dd--) {
         if ((uint32_t)dd + 8 >= a.m) continue;
         uint64_t w[8];
 #pragma unroll
         for (int v = 0; v < (1 << dd); v++) w[v] = tw12_at(a, (((uint32_t)v << 8) | t) << (3 - dd));
-#pragma unroll
-        for (int e = 0; e < kNttPerThread; e++) {
-            if ((e >> dd) & 1) continue;
-            const int f = e | (1 << dd);
-            const uint64_t y0 = x[e], y1 = x[f];
-            x[e] = gl::add(y0, y1);
-            x[f] = gl::mul(gl::sub(y0, y1), w[e & ((1 << dd) - 1)]);
-        }
+        reg_stage(ar, x, dd, [&](int e) { return w[e & ((1 << dd) - 1)]; });
     }
 #pragma unroll
     for (int i = 0; i < kNttPerThread; i++) lds[lds_slot(t + kNttThreads * i)] = x[i];
     __syncthreads();
-    uint32_t rem = a.m < 8 ? a.m : 8u;
-    while (rem >= 4) {
-        rem -= 4;
-        if (rem == 0) ntt_round_last<4>(lds, t, a.inverse);
-        else ntt_round4<true>(lds, a, t, rem, 0, 0);
+    contig_rounds(ar, lds, a, t, a.m < 8 ? a.m : 8u);
+}
+
+__global__ void __launch_bounds__(kNttThreads) __attribute__((amdgpu_waves_per_eu(4)))
+k_ntt_contig_reg(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
+{
+    __shared__ uint64_t lds[(1 << kNttTileLog) + (1 << kNttTileLog) / 32];
+    __shared__ uint32_t flags[kNttThreads / 64];
+    uint32_t t = threadIdx.x;
+    const uint64_t b = first + blockIdx.x;
+    const NttPass a = pass_at(passes, npasses, one, b);
+    uint64_t tile = b - a.tile_begin;
+    Lazy lazy;
+    contig_transform(lazy, lds, a, tile, t);
+    if (__builtin_expect(barrier_any(flags, lazy.bad), 0)) {
+        Exact exact;
+        again(t, tile);
+        contig_transform(exact, lds, a, tile, t);
         __syncthreads();
     }
-    if (rem == 3) ntt_round_last<3>(lds, t, a.inverse);
-    else if (rem == 2) ntt_round_last<2>(lds, t, a.inverse);
-    else if (rem == 1) ntt_round_last<1>(lds, t, a.inverse);
-    if (rem) __syncthreads();
+    const gptr<uint64_t> p = gmem(a.buf) + (tile << kNttTileLog) + t;
 #pragma unroll
     for (int i = 0; i < kNttPerThread; i++) p[i << 8] = lds[lds_slot(t + kNttThreads * i)];
 }
@@ -529,39 +640,50 @@ __device__ __forceinline__ StridedRows strided_rows(const NttPass &a, uint64_t t
     return r;
 }
 
-// Work-group k runs tile first + k of the list.
+template <int MODE, int K, class A>
+__device__ __forceinline__ void strided1_transform(A &ar, uint64_t (&x)[kNttPerThread], const NttPass &a,
+                                                   uint64_t tile, uint32_t t)
+{
+    constexpr int CB = 4 - K;
+    uint64_t w[strided_ntw<K>()];
+    strided_tw_load<K>(a, tile, t, w);
+    const StridedRows r = strided_rows<MODE>(a, tile, t);
+    if constexpr (MODE == kSrcLde) {
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i++) x[i] = r.src[strided_step<K>(a, i)];
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i += 2)
+            ar.mul2(x[i], r.fac[strided_step<K>(a, i)], x[i + 1], r.fac[strided_step<K>(a, i + 1)]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i++) x[i] = A::load(r.src[strided_step<K>(a, i)]);
+    }
+#pragma unroll
+    for (int dd = K - 1; dd >= 0; dd--)
+        reg_stage(ar, x, dd + CB, [&](int i) {
+            const int rb = i >> CB, g = i & ((1 << CB) - 1);
+            return w[strided_tw_off<K>(dd) + (g << dd) + (rb & ((1 << dd) - 1))];
+        });
+}
+
+// Work-group k runs tile first + k of the list.  A wave redoes its own words.
 template <int MODE, int K>
 __global__ void __launch_bounds__(kNttThreads)
 k_ntt_strided1_tiles(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
 {
-    constexpr int CB = 4 - K;
-    const uint32_t t = threadIdx.x;
+    uint32_t t = threadIdx.x;
     const uint64_t b = first + blockIdx.x;
     const NttPass a = pass_at(passes, npasses, one, b);
-    const uint64_t tile = b - a.tile_begin;
-    uint64_t w[strided_ntw<K>()];
-    strided_tw_load<K>(a, tile, t, w);
-    const StridedRows r = strided_rows<MODE>(a, tile, t);
+    uint64_t tile = b - a.tile_begin;
     uint64_t x[kNttPerThread];
-#pragma unroll
-    for (int i = 0; i < kNttPerThread; i++) x[i] = r.src[strided_step<K>(a, i)];
-    if constexpr (MODE == kSrcLde) {
-#pragma unroll
-        for (int i = 0; i < kNttPerThread; i++) x[i] = gl::mul(x[i], r.fac[strided_step<K>(a, i)]);
+    Lazy lazy;
+    strided1_transform<MODE, K>(lazy, x, a, tile, t);
+    if (__builtin_expect(lazy.bad != 0, 0)) {
+        Exact exact;
+        again(t, tile);
+        strided1_transform<MODE, K>(exact, x, a, tile, t);
     }
-#pragma unroll
-    for (int dd = K - 1; dd >= 0; dd--) {
-#pragma unroll
-        for (int i = 0; i < kNttPerThread; i++) {
-            const int rb = i >> CB, g = i & ((1 << CB) - 1);
-            if ((rb >> dd) & 1) continue;
-            const int f = i | (1 << (dd + CB));
-            const uint64_t wv = w[strided_tw_off<K>(dd) + (g << dd) + (rb & ((1 << dd) - 1))];
-            const uint64_t y0 = x[i], y1 = x[f];
-            x[i] = gl::add(y0, y1);
-            x[f] = gl::mul(gl::sub(y0, y1), wv);
-        }
-    }
+    const StridedRows r = strided_rows<MODE>(a, tile, t);
 #pragma unroll
     for (int i = 0; i < kNttPerThread; i++) r.buf[strided_step<K>(a, i)] = x[i];
 }
@@ -626,37 +748,19 @@ __device__ __forceinline__ void strided2_tw_load(const NttPass &a, uint64_t tile
     }
 }
 
-// Butterfly product of the two-round kernels: the carry form (gl::mul) but
-// in the in-place 8-stage kernel, where its schedule exceeds the 128 VGPRs
-// of four waves per SIMD (20 VGPRs spilled, against 6 with gl::mul_nc; the
-// 64 x 2^20 forward NTT took 1.03 against 0.95 ms).
-template <bool NC>
-__device__ __forceinline__ uint64_t strided2_mul(uint64_t a, uint64_t b)
-{
-    if constexpr (NC) return gl::mul_nc(a, b);
-    else return gl::mul(a, b);
-}
-
 // First round: stages K+3..K on the registers (element i = top j-bits).
-template <bool NC>
-__device__ __forceinline__ void strided2_round1(uint64_t (&x)[kNttPerThread], const uint64_t (&wa)[15])
+template <class A>
+__device__ __forceinline__ void strided2_round1(A &ar, uint64_t (&x)[kNttPerThread], const uint64_t (&wa)[15])
 {
 #pragma unroll
-    for (int dd = 3; dd >= 0; dd--) {
-#pragma unroll
-        for (int e = 0; e < kNttPerThread; e++) {
-            if ((e >> dd) & 1) continue;
-            const int f = e | (1 << dd);
-            const uint64_t y0 = x[e], y1 = x[f];
-            x[e] = gl::add(y0, y1);
-            x[f] = strided2_mul<NC>(gl::sub(y0, y1), wa[stage_off(4, dd) + (e & ((1 << dd) - 1))]);
-        }
-    }
+    for (int dd = 3; dd >= 0; dd--)
+        reg_stage(ar, x, dd, [&](int e) { return wa[stage_off(4, dd) + (e & ((1 << dd) - 1))]; });
 }
 
 // Second round: stages K-1..0 through LDS (ntt_round with b0 = 0, RB = c).
-template <int M, bool NC>
-__device__ __forceinline__ void strided2_round2(uint64_t *lds, uint32_t t, const uint64_t (&wb)[strided2_nwb<M>()])
+template <int M, class A>
+__device__ __forceinline__ void strided2_round2(A &ar, uint64_t *lds, uint32_t t,
+                                                const uint64_t (&wb)[strided2_nwb<M>()])
 {
     constexpr int K = M - 4, C = kNttTileLog - M, E = kNttPerThread;
     uint64_t x[E];
@@ -669,16 +773,8 @@ __device__ __forceinline__ void strided2_round2(uint64_t *lds, uint32_t t, const
         x[e] = lds[sl[e]];
     }
 #pragma unroll
-    for (int dd = K - 1; dd >= 0; dd--) {
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            if ((e >> dd) & 1) continue;
-            const int f = e | (1 << dd);
-            const uint64_t y0 = x[e], y1 = x[f];
-            x[e] = gl::add(y0, y1);
-            x[f] = strided2_mul<NC>(gl::sub(y0, y1), wb[stage_off(K, dd) + (e & ((1 << dd) - 1))]);
-        }
-    }
+    for (int dd = K - 1; dd >= 0; dd--)
+        reg_stage(ar, x, dd, [&](int e) { return wb[stage_off(K, dd) + (e & ((1 << dd) - 1))]; });
 #pragma unroll
     for (int e = 0; e < E; e++) lds[sl[e]] = x[e];
 }
@@ -725,6 +821,32 @@ __device__ __forceinline__ uint32_t strided2_off(const NttPass &a, uint32_t t)
     return ((t >> C) << a.s_lo) + (t & ((1u << C) - 1));
 }
 
+template <int MODE, int M, class A>
+__device__ __forceinline__ void strided2_transform(A &ar, uint64_t *lds, const NttPass &a, uint64_t tile, uint32_t t)
+{
+    const Strided2Rows r = strided2_rows<MODE, M>(a, tile);
+    const uint32_t off = strided2_off<M>(a, t);
+    uint64_t wa[15], wb[strided2_nwb<M>()];
+    strided2_tw_load<M>(a, tile, t, wa, wb);
+    uint64_t x[kNttPerThread];
+    if constexpr (MODE == kSrcLde) {
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i++) x[i] = gmem(r.src + strided2_step<M>(a, i))[off];
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i += 2)
+            ar.mul2(x[i], gmem(r.fac + strided2_step<M>(a, i))[off], x[i + 1],
+                    gmem(r.fac + strided2_step<M>(a, i + 1))[off]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < kNttPerThread; i++) x[i] = A::load(gmem(r.src + strided2_step<M>(a, i))[off]);
+    }
+    strided2_round1(ar, x, wa);
+#pragma unroll
+    for (int i = 0; i < kNttPerThread; i++) lds[lds_slot(t + kNttThreads * i)] = x[i];
+    __syncthreads();
+    strided2_round2<M>(ar, lds, t, wb);
+}
+
 // Work-group k runs tile first + k of the list (passes of one source mode
 // and M stages; grid = the tiles of the range).
 template <int MODE, int M>
@@ -732,28 +854,21 @@ __global__ void __launch_bounds__(kNttThreads) __attribute__((amdgpu_waves_per_e
 k_ntt_strided2_tiles(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
 {
     __shared__ uint64_t lds[(1 << kNttTileLog) + (1 << kNttTileLog) / 32];
-    const uint32_t t = threadIdx.x;
+    __shared__ uint32_t flags[kNttThreads / 64];
+    uint32_t t = threadIdx.x;
     const uint64_t b = first + blockIdx.x;
     const NttPass a = pass_at(passes, npasses, one, b);
-    const uint64_t tile = b - a.tile_begin;
-    uint64_t wa[15], wb[strided2_nwb<M>()];
-    strided2_tw_load<M>(a, tile, t, wa, wb);
-    uint64_t x[kNttPerThread];
+    uint64_t tile = b - a.tile_begin;
+    Lazy lazy;
+    strided2_transform<MODE, M>(lazy, lds, a, tile, t);
+    if (__builtin_expect(barrier_any(flags, lazy.bad), 0)) {
+        Exact exact;
+        again(t, tile);
+        strided2_transform<MODE, M>(exact, lds, a, tile, t);
+        __syncthreads();
+    }
     const Strided2Rows r = strided2_rows<MODE, M>(a, tile);
     const uint32_t off = strided2_off<M>(a, t);
-#pragma unroll
-    for (int i = 0; i < kNttPerThread; i++) x[i] = gmem(r.src + strided2_step<M>(a, i))[off];
-    if constexpr (MODE == kSrcLde) {
-#pragma unroll
-        for (int i = 0; i < kNttPerThread; i++) x[i] = gl::mul(x[i], gmem(r.fac + strided2_step<M>(a, i))[off]);
-    }
-    constexpr bool NC = MODE == kSrcInPlace && M == 8;
-    strided2_round1<NC>(x, wa);
-#pragma unroll
-    for (int i = 0; i < kNttPerThread; i++) lds[lds_slot(t + kNttThreads * i)] = x[i];
-    __syncthreads();
-    strided2_round2<M, NC>(lds, t, wb);
-    __syncthreads();
 #pragma unroll
     for (int i = 0; i < kNttPerThread; i++)
         gmem(r.buf + strided2_step<M>(a, i))[off] = lds[lds_slot(t + kNttThreads * i)];
