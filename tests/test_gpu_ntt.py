@@ -1,4 +1,6 @@
 """GPU NTT / LDE / transpose through the C ABI vs the oracle. Bit-exact."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -144,7 +146,7 @@ def rare_words(count, seed):
 
 
 @pytest.mark.parametrize("lg,B", [(1, 5), (3, 3), (4, 7), (7, 2), (11, 3), (12, 2), (13, 3), (14, 2), (15, 1), (16, 2), (17, 1),
-                                  (18, 1), (19, 1), (20, 1), (21, 1)])
+                                  (18, 1), (19, 1), (20, 1), (21, 1), (2, 1500), (9, 17), (13, 48), (14, 48)])
 @pytest.mark.parametrize("inverse", [False, True])
 @pytest.mark.parametrize("coset", [False, True])
 def test_ntt_of_rare_words_vs_oracle(zk, lg, B, inverse, coset):
@@ -156,12 +158,32 @@ def test_ntt_of_rare_words_vs_oracle(zk, lg, B, inverse, coset):
 
 
 @pytest.mark.parametrize("lg_n,rate,B", [(1, 1, 3), (4, 2, 3), (9, 1, 5), (12, 1, 3), (13, 2, 1), (14, 1, 1), (15, 1, 3), (16, 2, 1),
-                                         (17, 1, 1), (18, 1, 1), (19, 1, 1), (20, 1, 1)])
+                                         (17, 1, 1), (18, 1, 1), (19, 1, 1), (20, 1, 1), (1, 5, 3), (8, 4, 3), (7, 5, 2),
+                                         (9, 4, 2), (10, 3, 3), (11, 2, 1), (12, 1, 50), (10, 4, 48), (11, 3, 48),
+                                         (12, 2, 48), (13, 1, 48), (13, 3, 2)])
 @pytest.mark.parametrize("inverse", [False, True])
-def test_lde_of_rare_words_vs_oracle(zk, lg_n, rate, B, inverse):
-    print(f"lde lg_n={lg_n} rate={rate} B={B} inverse={inverse}", flush=True)
+@pytest.mark.parametrize("coset", [False, True])
+def test_lde_of_rare_words_vs_oracle(zk, lg_n, rate, B, inverse, coset):
+    print(f"lde lg_n={lg_n} rate={rate} B={B} inverse={inverse} coset={coset}", flush=True)
     x = rare_words(B << lg_n, 7 * lg_n + rate + B + inverse)
     out = np.zeros(B << (lg_n + rate), np.uint64)
-    zk.lde_batch(0, out, x, lg_n, zk.NTTConfig(batches=B, extension_rate_bits=rate, with_coset=not inverse),
+    zk.lde_batch(0, out, x, lg_n, zk.NTTConfig(batches=B, extension_rate_bits=rate, with_coset=coset),
                  direction=zk.INVERSE if inverse else zk.FORWARD)
-    assert np.array_equal(out, ob.lde(x % np.uint64(P), lg_n, rate, B, inverse=inverse, coset=not inverse))
+    assert np.array_equal(out, ob.lde(x % np.uint64(P), lg_n, rate, B, inverse=inverse, coset=coset))
+
+
+# Commits of degrees whose LDE is one launch, jobs of one list sharing it or
+# not: a ragged last tile, blocks of 2^13, columns of mixed degrees.
+def test_commit_of_one_launch_degrees_vs_oracle(zk):
+    shapes = [(3, 1, 1), (2, 4, 2), (5, 9, 1), (20, 10, 3), (7, 12, 1), (3, 13, 1), (2, 13, 2), (1, 13, 5), (2, 14, 1), (4, 10, 1)]
+    jobs, keep = [], []
+    for c, n, r in shapes:
+        x = rare_words(c << n, 100 * c + n + r)
+        N = 1 << (n + r)
+        d = [zk.DeviceBuffer.from_host(x), zk.DeviceBuffer(c * N), zk.DeviceBuffer(8 * N), zk.DeviceBuffer(4)]
+        jobs.append(zk.CommitJob(d[0].ptr, d[1].ptr, d[2].ptr, d[3].ptr, c, n, r, 0, zk.HASH_KECCAK, 0))
+        keep.append((x, d))
+    zk.commit_batch([SimpleNamespace(job=lambda j=j: j) for j in jobs])
+    for (c, n, r), (x, d) in zip(shapes, keep):
+        rows = ob.transpose_rev(ob.lde(x % np.uint64(P), n, r, c), n + r, c)
+        assert np.array_equal(d[1].to_host(), rows), (c, n, r)

@@ -47,7 +47,9 @@ std::vector<uint32_t> ntt_pass_sizes(uint32_t L, const Tuning &tun);
 // 2 + 4 * lde + (m - 1) strided single-round (every pass strided with the
 // same m <= 4 stages and the same source, in place or LDE; registers only);
 // 10 + 4 * lde + (m - 5) strided two-round (the same with 5 <= m <= 8, the
-// first round in registers).
+// first round in registers); kColumnKind + m whole blocks of 2^m <= 2^13 from
+// coefficients, forward, every pass with the same m (ntt_columns.h).
+constexpr int kColumnKind = 18;
 int ntt_kernel_kind(const NttPass *host_list, size_t n);
 
 // One launch over n pass descriptors in device memory (sorted by
@@ -57,6 +59,25 @@ int ntt_kernel_kind(const NttPass *host_list, size_t n);
 // dispatched between them).
 void launch_ntt_list(hipStream_t stream, const NttPass *dev_list, uint32_t n, uint64_t blocks, bool contiguous,
                      int kernel_kind, const char *name, uint64_t chunk = 0);
+
+// log2 words of the tile in which one launch does a whole transform of stages
+// L into `cols` columns of 2^lg in natural order, 0 where passes and a bit
+// reversal are used.  Rates above 3 have no kernel at 2^13 and 2^14.  A
+// column of 2^14 takes a CU to itself, so few of them leave the chip to 31 us
+// of passes that spread over it (inverse, one launch / passes, us: 2^14 x 20
+// 37 / 34, x 101 39 / 54, x 400 71 / 98; 2^13 x 1 25 / 30, x 101 27 / 39,
+// x 400 39 / 65; 2^12 x 1 20 / 27, x 400 27 / 44).
+inline uint32_t column_tile_log(uint32_t L, uint32_t lg, uint32_t cols)
+{
+    if (L == 0 || L > lg) return 0;
+    if (lg <= 12) return 12;
+    if (lg > 14 || lg - L > 3) return 0;
+    return lg == 13 || cols >= 48 ? lg : 0;
+}
+// That launch over the tiles [first, end) of the passes (device list, or
+// `one` when n == 0): s_lo == 0, m == L, every mode.
+void launch_columns(hipStream_t s, uint32_t L, uint32_t tile_log, const NttPass *list, uint32_t n, const NttPass &one,
+                    const ColumnPost &post, bool inverse, uint64_t first, uint64_t end);
 
 // table[i] = base^i, i < n.
 void fill_powers(uint64_t *dst, uint64_t n, uint64_t base, hipStream_t s);

@@ -63,6 +63,13 @@ bool launch_kind(int kind, hipStream_t stream, const NttPass *dev_list, uint32_t
         else launch_strided2<kSrcInPlace>(m, stream, dev_list, n, one, first, end);
         return true;
     }
+    if (kind > kColumnKind) {
+        const uint32_t L = (uint32_t)(kind - kColumnKind);
+        ColumnPost post{};
+        post.lg = L;
+        launch_columns(stream, L, std::max<uint32_t>(L, kNttTileLog), dev_list, n, one, post, false, first, end);
+        return true;
+    }
     return false;
 }
 
@@ -101,6 +108,12 @@ int ntt_kernel_kind(const NttPass *host_list, size_t n)
     if (n == 0) return 0;
     const NttPass &p0 = host_list[0];
     if (p0.s_lo == 0) {
+        bool columns = p0.m >= 1 && p0.m <= 13;
+        for (size_t i = 0; i < n; i++) {
+            const NttPass &p = host_list[i];
+            columns &= p.s_lo == 0 && p.mode == kSrcLde && !p.inverse && p.m == p0.m;
+        }
+        if (columns) return kColumnKind + (int)p0.m;
         for (size_t i = 0; i < n; i++) {
             const NttPass &p = host_list[i];
             if (p.s_lo != 0 || p.mode != kSrcInPlace || (p.total & ((1ull << kNttTileLog) - 1)) != 0) return 0;
@@ -181,8 +194,15 @@ uint64_t plan_dif(std::vector<NttPass> &out, uint64_t *buf, uint64_t nblk, uint3
                   const Tuning &tun)
 {
     const uint64_t total = nblk << L;
-    const uint64_t tiles = (total + (1ull << kNttTileLog) - 1) >> kNttTileLog;
-    const std::vector<uint32_t> sizes = ntt_pass_sizes(L, tun);
+    // an LDE of 2^13-word blocks fits the one-launch kernel (ntt_columns.h)
+    // with two work-groups per CU: 8 commits of 135 x 2^13 rate 3, Keccak-256,
+    // 2.01 -> 1.86 ms against a strided and a contiguous pass.  At 2^14, one
+    // work-group per CU, nothing overlaps its loads and the two passes are as
+    // fast (3.70 against 3.72 ms).
+    const bool whole = mode0 == kSrcLde && !inverse && L == kNttTileLog + 1;
+    const uint32_t tile_log = whole ? L : (uint32_t)kNttTileLog;
+    const uint64_t tiles = (total + (1ull << tile_log) - 1) >> tile_log;
+    const std::vector<uint32_t> sizes = whole ? std::vector<uint32_t>{L} : ntt_pass_sizes(L, tun);
     uint32_t hi = L;  // stages [0, hi) not yet planned
     for (size_t k = 0; k < sizes.size(); k++) {
         NttPass a{};
@@ -201,7 +221,7 @@ uint64_t plan_dif(std::vector<NttPass> &out, uint64_t *buf, uint64_t nblk, uint3
         a.mode = k == 0 ? mode0 : (uint32_t)kSrcInPlace;
         a.m = sizes[k];
         a.s_lo = hi - a.m;  // 0 exactly for the last (contiguous) pass
-        a.c = kNttTileLog - a.m;
+        a.c = tile_log - a.m;
         if (a.s_lo > 0 && a.s_lo < a.c) invalid("internal: NTT pass plan with stride below its column count");
         out.push_back(a);
         hi = a.s_lo;
@@ -262,6 +282,40 @@ const uint64_t *lde_factor_table(Device &d, uint32_t lg_n, uint32_t rate, bool i
     return F;
 }
 
+namespace {
+
+// A whole transform into natural order in one launch, where there is one:
+// cols blocks-of-2^rate columns of 2^(L + rate), read through `mode`.
+bool columns(Device &d, uint64_t *buf, uint32_t L, uint32_t rate, uint32_t cols, bool inverse, uint32_t mode,
+             const uint64_t *src, const uint64_t *factors, const uint64_t *coset_after)
+{
+    const uint32_t lg = L + rate, tile_log = column_tile_log(L, lg, cols);
+    if (!tile_log) return false;
+    NttPass a{};
+    a.buf = buf;
+    a.src = src;
+    a.coset = factors;
+    a.tw_lg = d.twiddle_tables_upto(L);
+    a.total = (uint64_t)cols << lg;
+    a.L = a.m = L;
+    a.rate = rate;
+    a.mode = mode;
+    a.inverse = inverse ? 1u : 0u;
+    ColumnPost post{};
+    post.coset = coset_after;
+    post.scale = inverse ? host_inv(1ull << lg) : 1;
+    post.lg = lg;
+    post.natural = 1;
+    const uint64_t tiles = (a.total + (1ull << tile_log) - 1) >> tile_log;
+    if (tiles > 0x7FFFFFFFull) invalid("transform too large for one launch");
+    ProfScope ps(mode == kSrcLde ? "ntt_pass_lde" : "ntt_pass", d.stream);
+    launch_columns(d.stream, L, tile_log, nullptr, 0, a, post, inverse, 0, tiles);
+    ZKX_HIP(hipGetLastError());
+    return true;
+}
+
+}  // namespace
+
 void lde_bitrev(Device &d, uint64_t *out, const uint64_t *in, uint32_t lg_n, uint32_t rate, uint32_t cols,
                 bool inverse, bool with_coset)
 {
@@ -277,6 +331,10 @@ void lde(Device &d, uint64_t *out, const uint64_t *in, uint32_t lg_n, uint32_t r
     const uint32_t lg = lg_n + rate;
     if (with_coset && inverse && (!d.coset || d.coset_lg < lg))
         invalid("coset table not initialised for log size " + std::to_string(lg));
+    if (column_tile_log(lg_n, lg, cols) &&
+        columns(d, out, lg_n, rate, cols, inverse, kSrcLde, in, lde_factor_table(d, lg_n, rate, inverse, with_coset),
+                (inverse && with_coset) ? d.coset : nullptr))
+        return;
     lde_bitrev(d, out, in, lg_n, rate, cols, inverse, with_coset);
     // natural order; inverse transforms are scaled by N^-1 and (reference
     // semantics, ntt.cu:137-139) by g^t when with_coset
@@ -288,8 +346,10 @@ void ntt(Device &d, uint64_t *inout, uint32_t lg, uint32_t cols, bool inverse, b
 {
     if (with_coset && (!d.coset || d.coset_lg < lg))
         invalid("coset table not initialised for log size " + std::to_string(lg));
-    const uint64_t *tw = d.twiddle_table(lg);
     const uint32_t mode = (with_coset && !inverse) ? kSrcCoset : kSrcInPlace;
+    if (columns(d, inout, lg, 0, cols, inverse, mode, nullptr, d.coset, (inverse && with_coset) ? d.coset : nullptr))
+        return;
+    const uint64_t *tw = d.twiddle_table(lg);
     run_dif(d, inout, cols, lg, lg, tw, inverse, mode, nullptr, 0, false, d.coset);
     bitrev_columns(d, inout, lg, cols, inverse, inverse ? host_inv((1ull << lg) % 0xFFFFFFFF00000001ull) : 1,
                    (inverse && with_coset) ? d.coset : nullptr);

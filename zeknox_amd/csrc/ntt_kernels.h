@@ -21,11 +21,7 @@
 // coefficients directly and multiplies by the resident factor table F, so
 // the zero half is never read, written or butterflied.
 #pragma once
-#include <type_traits>
-
-#include "gl64.h"
-#include "gmem.h"
-#include "ntt_types.h"
+#include "ntt_lanes.h"
 
 namespace zkx {
 
@@ -56,9 +52,6 @@ __device__ __forceinline__ uint32_t brev_bits(uint32_t x, uint32_t bits)
     return bits ? (__builtin_bitreverse32(x) >> (32 - bits)) : 0u;
 }
 
-// LDS slot of tile position u (one pad word per 32 breaks power-of-two strides)
-__device__ __forceinline__ uint32_t lds_slot(uint32_t u) { return u + (u >> 5); }
-
 // Tile positions are numbered u in memory order: u = j*2^c + q when the
 // pass is strided (s_lo > 0: column q of the stride, butterfly index j),
 // u = q*2^m + j when it is contiguous (s_lo == 0: group q, index j).
@@ -88,69 +81,6 @@ __device__ __forceinline__ uint64_t tile_step(const NttPass &a, int i)
     return (uint64_t)i << (lt - a.c + a.s_lo);
 }
 
-// ---- arithmetic of the passes
-//
-// A butterfly is 21 instructions on lazy values (Lazy) rather than 30 on
-// canonical ones (Exact): what a random operand needs once in 2^32 is left
-// out and its lanes noted in `bad` (gl64.h).  A tile with such a lane is
-// computed again with Exact, from the source that nothing has overwritten
-// yet.  Words between the passes of a transform are lazy too; the contiguous
-// pass, the last, stores canonical ones.
-//
-// Bounds, 64 x 2^20 forward (1.07 GB of traffic a pass): the 12-stage
-// contiguous pass 375 -> 318 us, of which its loads and stores alone take
-// 273; the 8-stage strided pass 298 -> 294 us, bound by its loads and stores
-// (250 alone).  The whole transform 906 -> 854 us, alternating builds.
-
-struct Lazy {
-    uint64_t bad = 0;
-    static __device__ __forceinline__ uint64_t load(uint64_t x) { return x; }
-    static __device__ __forceinline__ uint64_t result(uint64_t x) { return gl::canon(x); }
-    __device__ __forceinline__ void add_sub2(uint64_t &x0, uint64_t &y0, uint64_t &x1, uint64_t &y1)
-    {
-        uint64_t s0, d0, s1, d1;
-        gl::add_sub_rare2(x0, y0, x1, y1, s0, d0, s1, d1, bad);
-        x0 = s0, y0 = d0, x1 = s1, y1 = d1;
-    }
-    __device__ __forceinline__ void mul2(uint64_t &x0, uint64_t w0, uint64_t &x1, uint64_t w1)
-    {
-        uint64_t r0, r1;
-        gl::mul_rare2(x0, w0, x1, w1, r0, r1, bad);
-        x0 = r0, x1 = r1;
-    }
-    __device__ __forceinline__ uint64_t mul(uint64_t x, uint64_t w) { return gl::mul_rare(x, w, bad); }
-    template <int E>
-    __device__ __forceinline__ uint64_t shift(uint64_t x)
-    {
-        return gl::mul_pow2_rare<E>(x, bad);
-    }
-};
-
-struct Exact {
-    static __device__ __forceinline__ uint64_t load(uint64_t x) { return gl::canon(x); }
-    static __device__ __forceinline__ uint64_t result(uint64_t x) { return x; }
-    __device__ __forceinline__ void add_sub2(uint64_t &x0, uint64_t &y0, uint64_t &x1, uint64_t &y1)
-    {
-        const uint64_t s0 = gl::add(x0, y0), d0 = gl::sub(x0, y0), s1 = gl::add(x1, y1), d1 = gl::sub(x1, y1);
-        x0 = s0, y0 = d0, x1 = s1, y1 = d1;
-    }
-    __device__ __forceinline__ void mul2(uint64_t &x0, uint64_t w0, uint64_t &x1, uint64_t w1)
-    {
-        x0 = mul(x0, w0);
-        x1 = mul(x1, w1);
-    }
-    // (the form with the fewest live registers)
-    __device__ __forceinline__ uint64_t mul(uint64_t x, uint64_t w) { return gl::mul_nc(x, w); }
-    template <int E>
-    __device__ __forceinline__ uint64_t shift(uint64_t x)
-    {
-        // (x is canonical; the compiler folds a canon() that directly follows a
-        // sub() into its carry chain and counts the wrap of that as its own)
-        if constexpr (E == 0) return x;
-        else return gl::mul_pow2<E>(x);
-    }
-};
-
 // The stage whose partners differ in bit b of the register index, w(e) the
 // twiddle of element e's butterfly.
 template <class A, class W>
@@ -164,26 +94,6 @@ __device__ __forceinline__ void reg_stage(A &ar, uint64_t (&x)[kNttPerThread], i
         ar.add_sub2(x[e0], x[f0], x[e1], x[f1]);
         ar.mul2(x[f0], w(e0), x[f1], w(e1));
     }
-}
-
-// The lane and tile of the second computation, through values the compiler
-// cannot see through: nothing the first one loaded or computed stays in
-// registers for it.
-__device__ __forceinline__ void again(uint32_t &t, uint64_t &tile)
-{
-    asm volatile("; again %0 %1" : "+v"(t), "+s"(tile));
-}
-
-// Whether any wave of the work-group noted a lane; ends with every LDS write
-// before it visible.
-__device__ __forceinline__ bool barrier_any(uint32_t *flags, uint64_t bad)
-{
-    if ((threadIdx.x & 63) == 0) flags[threadIdx.x >> 6] = bad != 0 ? 1u : 0u;
-    __syncthreads();
-    uint32_t any = 0;
-#pragma unroll
-    for (int i = 0; i < kNttThreads / 64; i++) any |= flags[i];
-    return __builtin_amdgcn_readfirstlane(any) != 0;
 }
 
 // One register round: stages on j-bits [b0, b0+K) (u-bits [RB, RB+K)).
@@ -260,48 +170,8 @@ __device__ __forceinline__ void ntt_round4(A &ar, uint64_t *lds, const NttPass &
 // ---- last register round of a contiguous pass
 //
 // With b0 = 0 the round covers the K lowest stages; stage d's twiddle for
-// element e is w_{2^(d+1)}^v with v = e mod 2^d, a root of order <= 16:
-// w = 1 (no product) or a power of two (a shift; 2^96 = -1 is the difference
-// taken the other way round).
-
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F &&f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
-// e with 2^e = w_{2^(D+1)}^V (w^-V for the inverse)
-template <int D, int V, bool INV>
-constexpr int small_root_log()
-{
-    constexpr int L = gl::clog2(gl::comega(D + 1));
-    static_assert(L >= 0, "the 2^(D+1)-th root of unity of the transform is a power of two");
-    constexpr int E0 = (V * L) % 192;
-    return INV ? (192 - E0) % 192 : E0;
-}
-
-template <int DD, bool INV, class A>
-__device__ __forceinline__ void last_stages(A &ar, uint64_t (&x)[kNttPerThread])
-{
-    static_for<0, kNttPerThread / 4>([&](auto kc) {
-        constexpr int k = 2 * decltype(kc)::value;
-        constexpr int e0 = ((k >> DD) << (DD + 1)) | (k & ((1 << DD) - 1)), f0 = e0 | (1 << DD);
-        constexpr int e1 = (((k + 1) >> DD) << (DD + 1)) | ((k + 1) & ((1 << DD) - 1)), f1 = e1 | (1 << DD);
-        constexpr int E0 = small_root_log<DD, (e0 & ((1 << DD) - 1)), INV>();
-        constexpr int E1 = small_root_log<DD, (e1 & ((1 << DD) - 1)), INV>();
-        uint64_t a0 = E0 >= 96 ? x[f0] : x[e0], b0 = E0 >= 96 ? x[e0] : x[f0];
-        uint64_t a1 = E1 >= 96 ? x[f1] : x[e1], b1 = E1 >= 96 ? x[e1] : x[f1];
-        ar.add_sub2(a0, b0, a1, b1);
-        x[e0] = a0;
-        x[e1] = a1;
-        x[f0] = ar.template shift<E0 % 96>(b0);
-        x[f1] = ar.template shift<E1 % 96>(b1);
-    });
-    if constexpr (DD > 0) last_stages<DD - 1, INV>(ar, x);
-}
+// element e is w_{2^(d+1)}^v with v = e mod 2^d, a root of order <= 16
+// (last_stages).
 
 // The round on stages K-1..0 of a contiguous pass (lane t holds the 2^K
 // elements u = (other << K) | rb, other = t | group << 8): ntt_round4 with
@@ -319,7 +189,7 @@ __device__ __forceinline__ void ntt_round_last(A &ar, uint64_t *lds, uint32_t t)
         uu[e] = (other << K) | rb;
         x[e] = lds[lds_slot(uu[e])];
     }
-    last_stages<K - 1, INV>(ar, x);
+    last_stages<K - 1, INV, E>(ar, x);
 #pragma unroll
     for (int e = 0; e < E; e++) lds[lds_slot(uu[e])] = A::result(x[e]);
 }
@@ -345,32 +215,6 @@ __device__ __forceinline__ void contig_rounds(A &ar, uint64_t *lds, const NttPas
     else if (rem == 3) ntt_round_last<3>(ar, lds, t, a.inverse);
     else if (rem == 2) ntt_round_last<2>(ar, lds, t, a.inverse);
     else if (rem == 1) ntt_round_last<1>(ar, lds, t, a.inverse);
-}
-
-// ---- descriptors
-//
-// A launch's descriptor list is read through the constant address space
-// (scalar loads into SGPRs; as vector loads they cost 32 VGPRs).
-
-__device__ __forceinline__ NttPass pass_at(const NttPass *passes, uint32_t npasses, const NttPass &one, uint64_t b)
-{
-    if (!npasses) return one;
-    const cptr<NttPass> cp = cmem(passes);
-    uint32_t lo = 0, hi = npasses;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (cp[mid].tile_begin <= b) lo = mid;
-        else hi = mid;
-    }
-    static_assert(sizeof(NttPass) % 8 == 0, "descriptor copied as 64-bit words");
-    constexpr int W = sizeof(NttPass) / 8;
-    const cptr<uint64_t> src = (cptr<uint64_t>)(cp + lo);
-    uint64_t w[W];
-#pragma unroll
-    for (int i = 0; i < W; i++) w[i] = src[i];
-    NttPass r;
-    __builtin_memcpy(&r, w, sizeof r);
-    return r;
 }
 
 // The tile of k_ntt_tiles from its source to its results in LDS (a barrier

@@ -41,4 +41,12 @@ struct NttPass {
     const uint64_t *const *tw_lg;
 };
 
+// What follows the stages of a one-launch transform.
+struct ColumnPost {
+    const uint64_t *coset;  // inverse: times g^t at natural index t (null: not)
+    uint64_t scale;         // inverse: times this
+    uint32_t lg;            // log2 column length
+    uint32_t natural;       // 1: columns bit-reversed into natural order; 0: left in DIF order
+};
+
 }  // namespace zkx
