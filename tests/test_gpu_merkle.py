@@ -182,3 +182,38 @@ def test_lone_schedules_agree_at_switch_sizes(zk, ht, lg_l):
     for name in ("fused", "by_level"):
         assert np.array_equal(out[name][1], out["default"][1]), name
         assert np.array_equal(out[name][0], out["default"][0]), name
+
+
+# Keccak on lane pairs: levels inside the leaf launch, and the top of a tree
+# whose wide levels are launched apart (from 2^16 children, and caps above,
+# at and below that level).
+@pytest.mark.parametrize("lg,leaf,cap", [(1, 5, 0), (2, 3, 1), (8, 20, 0), (9, 4, 0), (11, 17, 2), (18, 4, 0), (18, 4, 4), (18, 1, 8),
+                                         (18, 2, 9), (18, 4, 15), (18, 4, 16), (18, 4, 17), (18, 3, 18), (19, 4, 1)])
+def test_keccak_tops_vs_oracle(zk, lg, leaf, cap):
+    print(f"keccak lg={lg} leaf={leaf} cap={cap}", flush=True)
+    n, nc = 1 << lg, 1 << cap
+    x = ob.canonical(n * leaf, 31 * lg + leaf + cap)
+    d, dig, caps = zk.DeviceBuffer.from_host(x), zk.DeviceBuffer(max(8 * (n - nc), 1)), zk.DeviceBuffer(4 * nc)
+    zk.fill_digests_buf_linear_gpu_with_gpu_ptr(dig, caps, d, 2 * (n - nc), nc, n, leaf, cap, zk.HASH_KECCAK, 0)
+    edig, ecap = ob.merkle(x, leaf, cap, zk.HASH_KECCAK)
+    assert np.array_equal(caps.to_host(), ecap)
+    if n > nc:
+        assert np.array_equal(dig.to_host(), edig)
+
+
+def test_keccak_top_in_a_batch(zk):
+    """Two forests of one batch whose levels are launched apart, one of them narrow from the start."""
+    from types import SimpleNamespace
+    jobs, keep = [], []
+    for c, n, r, h in [(3, 16, 1, 2), (2, 16, 1, 14), (4, 5, 1, 0)]:
+        x = ob.canonical(c << n, c + n)
+        N = 1 << (n + r)
+        d = [zk.DeviceBuffer.from_host(x), zk.DeviceBuffer(c * N), zk.DeviceBuffer(8 * (N - (1 << h))), zk.DeviceBuffer(4 << h)]
+        jobs.append(zk.CommitJob(*[b.ptr for b in d], c, n, r, h, zk.HASH_KECCAK, 0))
+        keep.append((c, h, d))
+    zk.init_coset_rs(0, 17, 7)
+    for _ in range(4):  # the last replays a captured launch list
+        zk.commit_batch([SimpleNamespace(job=lambda j=j: j) for j in jobs])
+    for c, h, d in keep:
+        dig, cap = ob.merkle(d[1].to_host(), c, h, zk.HASH_KECCAK)
+        assert np.array_equal(d[2].to_host(), dig) and np.array_equal(d[3].to_host(), cap), (c, h)

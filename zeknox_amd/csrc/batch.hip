@@ -212,8 +212,8 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
     };
     // levels launched apart, by hash kind: level k above the leaves of every
     // tree that has it in one launch each, and for the hashes with the
-    // 16-permutations-per-wave kernel every level from the first one whose
-    // children are few enough in one launch of that
+    // 16-permutations-per-wave kernel (or a top of tiles) every level from the
+    // first one whose children are few enough in one launch of that
     struct LevelLaunch {
         int hash;
         bool narrow;
@@ -235,7 +235,7 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
                 for (size_t i = 0; i < n; i++)
                     if (apart(i, k)) children += specs[i].num_caps << (mk[i].lg_w - k + 1);
                 if (!children) break;
-                l.narrow = has_narrow_kernel((uint64_t)ht) && children <= kNarrowNodes;
+                l.narrow = (has_narrow_kernel((uint64_t)ht) || has_tile_top((uint64_t)ht)) && children <= kNarrowNodes;
                 for (size_t i = 0; i < n; i++) {
                     if (!apart(i, k)) continue;
                     MerkleArgs a;
@@ -313,7 +313,9 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
     for (LevelLaunch &l : levels) {
         for (size_t i = 0; l.narrow && i < l.list.size(); i++) l.list[i].ctr = ctr_.as<uint32_t>() + l.first_ctr[i];
         const size_t off = push(l.list.data(), l.list.size() * sizeof(MerkleArgs));
-        launches.push_back({off, (uint32_t)l.list.size(), l.blocks, l.narrow ? 3 : 2, l.hash, 0, 0});
+        const bool tiles = l.narrow && has_tile_top((uint64_t)l.hash);
+        launches.push_back({off, (uint32_t)l.list.size(), l.blocks, tiles ? 1 : l.narrow ? 3 : 2, l.hash, 0,
+                            tiles ? (uint32_t)kMerkleMinTileLog : 0});
         host.resize(align_up(host.size()));
     }
     size_t off0 = 0;

@@ -48,7 +48,8 @@ void launch_merkle_level(hipStream_t stream, int hash_type, const MerkleArgs *de
 // The passes of a tree (written null: leaves in tiles of 2^6), or of what lies
 // above its level of width 2^*written per subtree (nodes in tiles of 2^7),
 // fused into one descriptor for launch_merkle_narrow; returns the arrival
-// counters it needs.
+// counters it needs.  Keccak-256 (has_tile_top): what lies above a written
+// level, in tiles of 2^8, for launch_merkle_pass with 2^8 lanes.
 uint64_t plan_merkle_narrow(const MerkleSpec &s, const uint32_t *written, MerkleArgs &out);
 // One launch of the 16-permutations-per-wave kernel (merkle_narrow.h; Poseidon
 // and Poseidon2) over n such descriptors in device memory, or over `one`

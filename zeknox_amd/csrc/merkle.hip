@@ -79,8 +79,8 @@ uint32_t plan_merkle(const MerkleSpec &s, MerkleArgs (&passes)[kMerkleMaxPasses]
 uint64_t plan_merkle_narrow(const MerkleSpec &s, const uint32_t *written, MerkleArgs &out)
 {
     MerkleArgs passes[kMerkleMaxPasses];
-    const uint32_t n = plan_passes(s, passes, written ? kMerkleNarrowNodesLog : kMerkleNarrowTileLog,
-                                   kMerkleNarrowNodesLog,
+    const uint32_t nodes_log = has_tile_top(s.hash_type) ? kMerkleMinTileLog : kMerkleNarrowNodesLog;
+    const uint32_t n = plan_passes(s, passes, written ? nodes_log : kMerkleNarrowTileLog, nodes_log,
                                    written ? *written : log2u(s.num_leaves) - log2u(s.num_caps));
     if (written) passes[0].leaves = nullptr;
     return fuse_merkle_passes(passes, n, out);
@@ -206,6 +206,11 @@ void build_narrow(Device &d, const MerkleSpec &s, const uint32_t *written, const
     MerkleArgs f;
     const uint64_t nctr = plan_merkle_narrow(s, written, f);
     if (nctr) f.ctr = scratch.counters(d, nctr);
+    if (has_tile_top(s.hash_type)) {
+        const MerkleArgs *dj = scratch.descriptor(d, f);
+        launch_merkle_pass(d.stream, (int)s.hash_type, dj, 1, MerkleArgs{}, f.count >> f.tile_log, kMerkleMinTileLog);
+        return;
+    }
     launch_merkle_narrow(d.stream, (int)s.hash_type, nullptr, 0, f, f.count >> f.tile_log,
                          f.leaves ? "merkle_leaves" : "merkle_levels");
 }
@@ -235,7 +240,7 @@ void merkle_build(Device &d, const MerkleSpec &s, const MerkleScratch &scratch)
         leaf.leaves_only = 1;
         launch_merkle_pass(d.stream, (int)s.hash_type, nullptr, 0, leaf, leaf.count >> leaf.tile_log, tl);
         for (uint32_t w = leaf.lg_w; w-- > 0;) {
-            if (narrow && s.num_caps << (w + 1) <= kNarrowNodes) {
+            if ((narrow || has_tile_top(s.hash_type)) && s.num_caps << (w + 1) <= kNarrowNodes) {
                 const uint32_t written = w + 1;
                 build_narrow(d, s, &written, scratch);
                 break;

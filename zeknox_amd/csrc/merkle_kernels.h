@@ -42,6 +42,7 @@
 #include "gmem.h"
 #include "hash.h"
 #include "merkle_types.h"
+#include "tuning.h"
 #include "poseidon_mfma.h"
 
 namespace zkx {
@@ -143,11 +144,22 @@ k_merkle_tile(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs on
     uint32_t lg_w = a.lg_w;           // log2 per-subtree width of the current level
     uint64_t first = ((uint64_t)bid - a.tile_begin) << a.tile_log;  // first node of the tile
 
+    // the tile's nodes (of a level that is written) into LDS
+    auto load_nodes = [&] {
+        if (t < cur) {
+            const uint64_t g = first + t;
+            const gptr<uint64_t> src = node_ptr(a, g >> lg_w, lg_w, g & ((1ull << lg_w) - 1));
+#pragma unroll
+            for (int i = 0; i < 4; i++) lds[t][i] = src[i];
+        }
+    };
     uint64_t h[4];
     const bool mfma = has_mfma(HT) && cur >= 64 && a.leaf_size > 4 && !(HT == kPoseidon && a.leaf_valu);
     if constexpr (has_mfma(HT))
         if (mfma) leaf_hash_mfma<HT, TPB>(a, first, cur, lds, tables);
-    if (t < cur) {
+    if (has_tile_top(HT) && !a.leaves) {
+        load_nodes();
+    } else if (t < cur) {
         const uint64_t g = first + t;
         const uint64_t sub = g >> lg_w, idx = g & ((1ull << lg_w) - 1);
         if (mfma) {
@@ -204,21 +216,16 @@ k_merkle_tile(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs on
             up++;
             cur = 1u << tl;
             first = grp << tl;
-            if (t < cur) {
-                const uint64_t g = first + t;
-                const gptr<uint64_t> src = node_ptr(a, g >> lg_w, lg_w, g & ((1ull << lg_w) - 1));
-#pragma unroll
-                for (int i = 0; i < 4; i++) lds[t][i] = src[i];
-            }
+            load_nodes();
             __syncthreads();
             continue;
         }
-        // Nodes of a level: with PAIR (Poseidon, Poseidon2) lanes 2n and 2n+1
+        // Nodes of a level: with PAIR (Poseidon, Poseidon2, Keccak) lanes 2n and 2n+1
         // hash node n together (a level never has more than TPB / 2 nodes)
         // and lane 2n writes the digest; a Poseidon level of at most TPB / 16
         // nodes runs on rows (ROW: lanes 16n .. 16n + 15, lane 16n + k
         // writes digest element k < 4); otherwise lane n hashes node n.
-        constexpr bool PAIR = HT == kPoseidon || HT == kPoseidon2;
+        constexpr bool PAIR = HT == kPoseidon || HT == kPoseidon2 || HT == kKeccak;
         const bool ROW = HT == kPoseidon && (cur >> 1) * 16 <= TPB;
         const uint32_t k = t & 15;
         const uint32_t n = ROW ? t >> 4 : PAIR ? t >> 1 : t;
@@ -226,6 +233,7 @@ k_merkle_tile(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs on
         auto hash_node = [&](uint64_t out[4]) {
             if constexpr (HT == kPoseidon) poseidon_hash_two_pair(lds[2 * n], lds[2 * n + 1], out, (t & 1) != 0);
             else if constexpr (HT == kPoseidon2) poseidon2_hash_two_pair(lds[2 * n], lds[2 * n + 1], out, (t & 1) != 0);
+            else if constexpr (HT == kKeccak) keccak_hash_two_pair(lds[2 * n], lds[2 * n + 1], out, (t & 1) != 0);
             else hash_two<HT>(lds[2 * n], lds[2 * n + 1], out);
         };
         if (lg_w == 1) {

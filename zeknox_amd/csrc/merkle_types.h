@@ -23,7 +23,7 @@ constexpr int kMerkleNarrowLanes = 256;
 constexpr int kMerkleLevelLanes = 256;
 
 struct MerkleArgs {
-    const uint64_t *leaves;  // first pass: leaf source (null, k_merkle_narrow only: the level lg_w is written)
+    const uint64_t *leaves;  // first pass: leaf source (null: the level lg_w is written)
     uint64_t *leaves_out;    // first pass, optional: leaf rows [t][leaf_size]
     uint64_t *dig;
     uint64_t *cap;

@@ -67,6 +67,12 @@ constexpr uint64_t kNarrowLeaves = 1ull << 15;
 // (over all trees of one hash): every tile of 128 is resident at once.
 constexpr uint64_t kNarrowNodes = 1ull << 16;
 
+// Keccak-256's trees finish in one launch of the leaf kernel, on tiles of 256
+// nodes of a written level, from the same number of children: there a level
+// is a permutation on a lane pair, 6 us, against 9.4 in a launch of its own.
+// (Forest of 2^18 leaves of 135, cap 0, 484 -> 423 us; 2^20 1239 -> 1179.)
+constexpr bool has_tile_top(uint64_t hash_type) { return hash_type == 1; }
+
 // Whether one tree through the C-ABI Merkle entry points builds its levels
 // with one launch per level (after a leaf-digests-only launch; Poseidon and
 // Poseidon2 finish with one launch of the 16-per-wave kernel) rather than
@@ -75,17 +81,19 @@ constexpr uint64_t kNarrowNodes = 1ull << 16;
 // and Monolith at min_leaves / 4, Poseidon-BN128 at min_leaves / 32 (0:
 // always).  Measured, fused against apart, 135-element leaves, cap 4, ms:
 //   leaves  Poseidon      Poseidon2     Keccak-256     Monolith       Poseidon-BN128
-//   2^15                                0.248 / 0.251  0.540 / 0.533  36.2 / 33.5
-//   2^16                  0.92 / 0.76
-//   2^17                  1.11 / 0.96   0.330 / 0.333  0.695 / 0.697  48.5 / 46.2
-//   2^18    1.74 / 1.53   1.86 / 1.65   0.503 / 0.485  1.078 / 1.056  75.3 / 72.8
-//   2^19                  3.66 / 3.25   1.095 / 0.779  2.069 / 1.760
-//   2^20    6.36 / 5.67   7.01 / 6.02   1.928 / 1.344  3.639 / 3.143
+//   2^15                                0.215 / 0.219  0.540 / 0.533  36.2 / 33.5
+//   2^16                  0.92 / 0.76   0.225 / 0.234
+//   2^17                  1.11 / 0.96   0.299 / 0.295  0.695 / 0.697  48.5 / 46.2
+//   2^18    1.74 / 1.53   1.86 / 1.65         / 0.423  1.078 / 1.056  75.3 / 72.8
+//   2^19                  3.66 / 3.25         / 0.688  2.069 / 1.760
+//   2^20    6.36 / 5.67   7.01 / 6.02         / 1.179  3.639 / 3.143
+// (Keccak-256 above 2^17 before its lane pairs and top of tiles: 0.503 / 0.485,
+// 1.095 / 0.779, 1.928 / 1.344.)
 // Poseidon's and Poseidon2's narrow levels cost 12 us each in the 16-per-wave
 // kernel against 25-36 us on lane pairs and rows inside the leaf launch, so
 // every tree that is not built whole by that kernel gains.  Keccak's and
-// Monolith's permutations are short, so their fused trees' tops, one
-// permutation's latency per level on ever fewer lanes, weigh more;
+// Monolith's permutations are short, so what their fused trees' lower levels
+// lose on ever fewer lanes weighs more;
 // Poseidon-BN128's levels are slow enough that a full-GPU launch per level
 // pays at every size measured.
 inline bool lone_tree_levels_apart(uint64_t num_leaves, uint64_t hash_type, uint64_t min_leaves)
