@@ -187,3 +187,28 @@ def test_commit_of_one_launch_degrees_vs_oracle(zk):
     for (c, n, r), (x, d) in zip(shapes, keep):
         rows = ob.transpose_rev(ob.lde(x % np.uint64(P), n, r, c), n + r, c)
         assert np.array_equal(d[1].to_host(), rows), (c, n, r)
+
+
+# The two-launch transforms: every split of the stages, whole and partial
+# chunks of columns, the smallest batch that takes them and the one below,
+# rates whose blocks share an output run; then with the scratch given back.
+@pytest.mark.parametrize("lg,B", [(15, 7), (15, 8), (16, 4), (17, 3), (18, 1), (19, 3), (20, 1), (20, 17)])
+@pytest.mark.parametrize("inverse,coset", [(False, False), (False, True), (True, False), (True, True)])
+def test_two_launch_ntt_vs_oracle(zk, lg, B, inverse, coset):
+    print(f"ntt lg={lg} B={B} inverse={inverse} coset={coset}", flush=True)
+    x = rare_words(B << lg, 5 * lg + B) if lg < 18 else ob.canonical(B << lg, 5 * lg + B)
+    buf = x.copy()
+    (zk.intt_batch if inverse else zk.ntt_batch)(0, buf, lg, zk.NTTConfig(batches=B, with_coset=coset))
+    assert np.array_equal(buf, ob.ntt(x % np.uint64(P), lg, B, inverse, coset))
+
+
+@pytest.mark.parametrize("lg_n,rate,B", [(15, 3, 1), (15, 5, 3), (16, 2, 2), (17, 3, 1), (18, 1, 2), (19, 1, 1), (20, 2, 1), (20, 4, 1)])
+@pytest.mark.parametrize("inverse,coset", [(False, True), (True, False), (True, True)])
+def test_two_launch_lde_vs_oracle(zk, lg_n, rate, B, inverse, coset):
+    print(f"lde lg_n={lg_n} rate={rate} B={B} inverse={inverse} coset={coset}", flush=True)
+    x = ob.canonical(B << lg_n, lg_n + 11 * rate + B)
+    out = np.zeros(B << (lg_n + rate), np.uint64)
+    zk._check(zk.lib.zkx_commit_trim(0))
+    zk.lde_batch(0, out, x, lg_n, zk.NTTConfig(batches=B, extension_rate_bits=rate, with_coset=coset),
+                 direction=zk.INVERSE if inverse else zk.FORWARD)
+    assert np.array_equal(out, ob.lde(x, lg_n, rate, B, inverse=inverse, coset=coset))

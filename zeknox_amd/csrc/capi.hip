@@ -360,9 +360,13 @@ RustError zkx_commit_batch_pieces(size_t device_id, const ZkxCommitJob *jobs, si
 RustError zkx_commit_trim(size_t device_id)
 {
     return guarded([&] {
-        Engine &e = default_engine(device(device_id));
+        Device &d = device(device_id);
+        Engine &e = default_engine(d);
         std::lock_guard<std::mutex> g(e.mu);
         e.trim();
+        std::lock_guard<std::mutex> gd(d.mu);
+        d.sync();
+        d.ntt_scratch = DevBuf();
     });
 }
 

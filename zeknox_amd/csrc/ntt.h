@@ -79,6 +79,12 @@ inline uint32_t column_tile_log(uint32_t L, uint32_t lg, uint32_t cols)
 void launch_columns(hipStream_t s, uint32_t L, uint32_t tile_log, const NttPass *list, uint32_t n, const NttPass &one,
                     const ColumnPost &post, bool inverse, uint64_t first, uint64_t end);
 
+// The two launches of ntt_two.h over a.total words (whole columns): the top
+// a.m stages from a.src into a.buf, and the low a.m stages from a.src into
+// natural order in a.buf.
+void launch_two_first(hipStream_t s, const NttPass &a);
+void launch_two_second(hipStream_t s, const NttPass &a, const ColumnPost &post);
+
 // table[i] = base^i, i < n.
 void fill_powers(uint64_t *dst, uint64_t n, uint64_t base, hipStream_t s);
 // `count` pseudo-random field elements from `seed` (LDE salt columns).

@@ -314,6 +314,73 @@ bool columns(Device &d, uint64_t *buf, uint32_t L, uint32_t rate, uint32_t cols,
     return true;
 }
 
+constexpr size_t kTwoScratch = 128ull << 20;
+
+// Columns of a chunk of the two-launch transform (ntt_two.h) of stages L into
+// `cols` columns of 2^lg, 0 where passes and a bit reversal are used.
+// Below 2^18 words in all both ways are a few tiles' latency and the passes, on
+// smaller tiles, win (2^15 x 4 30.5 / 29.9 us, 2^16 x 1 31.3 / 30.0; 2^16 x 4
+// 30.7 / 31.9, 2^18 x 1 31.7 / 33.6).  A chunk of 64 MiB costs 5% (too few
+// tiles a launch), one of 512 gains nothing.
+uint64_t two_launch_chunk(uint32_t L, uint32_t lg, uint64_t cols)
+{
+    if (L < 15 || L > 20 || (cols << lg) < (1ull << 18) || (sizeof(uint64_t) << lg) > kTwoScratch) return 0;
+    return std::min<uint64_t>(cols, kTwoScratch / (sizeof(uint64_t) << lg));
+}
+
+// A transform into natural order in two launches a chunk, where there is one
+// and its scratch can be had: from src (cols x 2^L; buf itself in place).
+bool two_launches(Device &d, uint64_t *buf, uint32_t L, uint32_t rate, uint32_t cols, bool inverse, uint32_t mode,
+                  const uint64_t *src, const uint64_t *factors, const uint64_t *coset_after)
+{
+    const uint32_t lg = L + rate;
+    const uint64_t chunk = two_launch_chunk(L, lg, cols);
+    if (!chunk) return false;
+    const size_t bytes = (size_t)(chunk * sizeof(uint64_t)) << lg;
+    if (d.ntt_scratch.bytes < bytes) {
+        d.sync();
+        d.ntt_scratch = DevBuf();
+        try {
+            d.ntt_scratch = DevBuf(bytes);
+        } catch (const Error &) {
+            (void)hipGetLastError();  // no memory left for it: the passes need none
+            return false;
+        }
+    }
+    NttPass a{};
+    a.coset = factors;
+    a.tw_lg = d.twiddle_tables_upto(L);
+    a.L = L;
+    a.rate = rate;
+    a.mode = mode;
+    a.inverse = inverse ? 1u : 0u;
+    ColumnPost post{};
+    post.coset = coset_after;
+    post.scale = inverse ? host_inv((1ull << lg) % 0xFFFFFFFF00000001ull) : 1;
+    post.lg = lg;
+    post.natural = 1;
+    for (uint64_t c = 0; c < cols; c += chunk) {
+        a.total = std::min<uint64_t>(chunk, cols - c) << lg;
+        {
+            ProfScope ps(mode == kSrcLde ? "ntt_pass_lde" : "ntt_pass", d.stream);
+            a.src = src + (c << L);
+            a.buf = d.ntt_scratch.as<uint64_t>();
+            a.m = (L + 1) / 2;
+            a.s_lo = L - a.m;
+            launch_two_first(d.stream, a);
+            ZKX_HIP(hipGetLastError());
+        }
+        ProfScope ps("ntt_pass", d.stream);
+        a.src = d.ntt_scratch.as<uint64_t>();
+        a.buf = buf + (c << lg);
+        a.m = L / 2;
+        a.s_lo = 0;
+        launch_two_second(d.stream, a, post);
+        ZKX_HIP(hipGetLastError());
+    }
+    return true;
+}
+
 }  // namespace
 
 void lde_bitrev(Device &d, uint64_t *out, const uint64_t *in, uint32_t lg_n, uint32_t rate, uint32_t cols,
@@ -335,6 +402,10 @@ void lde(Device &d, uint64_t *out, const uint64_t *in, uint32_t lg_n, uint32_t r
         columns(d, out, lg_n, rate, cols, inverse, kSrcLde, in, lde_factor_table(d, lg_n, rate, inverse, with_coset),
                 (inverse && with_coset) ? d.coset : nullptr))
         return;
+    if (two_launch_chunk(lg_n, lg, cols) &&
+        two_launches(d, out, lg_n, rate, cols, inverse, kSrcLde, in, lde_factor_table(d, lg_n, rate, inverse, with_coset),
+                     (inverse && with_coset) ? d.coset : nullptr))
+        return;
     lde_bitrev(d, out, in, lg_n, rate, cols, inverse, with_coset);
     // natural order; inverse transforms are scaled by N^-1 and (reference
     // semantics, ntt.cu:137-139) by g^t when with_coset
@@ -347,8 +418,9 @@ void ntt(Device &d, uint64_t *inout, uint32_t lg, uint32_t cols, bool inverse, b
     if (with_coset && (!d.coset || d.coset_lg < lg))
         invalid("coset table not initialised for log size " + std::to_string(lg));
     const uint32_t mode = (with_coset && !inverse) ? kSrcCoset : kSrcInPlace;
-    if (columns(d, inout, lg, 0, cols, inverse, mode, nullptr, d.coset, (inverse && with_coset) ? d.coset : nullptr))
-        return;
+    const uint64_t *after = (inverse && with_coset) ? d.coset : nullptr;
+    if (columns(d, inout, lg, 0, cols, inverse, mode, nullptr, d.coset, after)) return;
+    if (two_launches(d, inout, lg, 0, cols, inverse, mode, inout, d.coset, after)) return;
     const uint64_t *tw = d.twiddle_table(lg);
     run_dif(d, inout, cols, lg, lg, tw, inverse, mode, nullptr, 0, false, d.coset);
     bitrev_columns(d, inout, lg, cols, inverse, inverse ? host_inv((1ull << lg) % 0xFFFFFFFF00000001ull) : 1,

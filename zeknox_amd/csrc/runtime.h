@@ -69,6 +69,10 @@ struct Device {
     hipDeviceProp_t prop{};
     std::mutex mu;                 // serialises table builds and compute calls
 
+    // Scratch of the transforms in two launches (ntt.hip), at most 128 MiB;
+    // used under `mu` on `stream`, given back by zkx_commit_trim.
+    DevBuf ntt_scratch;
+
     // Resident tables (twiddles per log size, coset powers).
     uint64_t *twiddles[33] = {};   // twiddles[k][i] = w_{2^k}^i, i < 2^k
     // The same 33 table pointers in device memory (null where not built),
