@@ -34,7 +34,8 @@
 // 56.4 -> 41.0 ms; of 2^21 leaves of 400 with Poseidon2: 36 -> 31.7 ms.
 // The S-boxes' products and the recombination then leave their rare corrections
 // to a branch (gl64.h): 153 -> 137 VALU and 41.0 -> 38.6 ms, Poseidon2 162 ->
-// 146 and 31.7 -> 29.7 ms.
+// 146 and 31.7 -> 29.7 ms.  With a chunk's loads together (merkle_kernels.h) 133
+// VALU and 36.8 ms, Poseidon2 28.5 ms.
 // Five rounds: the map of four leaves a K-chunk unused and costs as much; six
 // needs a fifth chunk and weights beyond 32 bits.
 //
