@@ -55,7 +55,7 @@ MFMA_WAVE_INSTS_PER_PERM = {(8, 0): 4.3125, (9, 0): 4.3125, (10, 0): 4.3125, (9,
 #   SHA-256 (first 16 hex digits) of the leaf kernel's sources those counts
 #   were measured on (leaf_kernel_digest()); a build whose sources differ is
 #   flagged in the JSON ("counters_match_build": false)
-LEAF_COUNTERS_SOURCES = "a738f73fbbf4d93b"
+LEAF_COUNTERS_SOURCES = "e57c836782a8f862"
 #   issue slots (one per 4 cycles) that one such MFMA takes from the vector
 #   issue of its SIMD beside full-rate VALU work: measured live by the
 #   "issue" leg (zkx_issue_probe); this value only when that leg is skipped
@@ -71,9 +71,9 @@ NTT_TRAFFIC_BYTES_PER_COMMIT = 8.855e8
 #   VALU wave-instructions of the NTT launches per commit (both passes,
 #   SQ_INSTS_VALU), keyed by the LDE's pass split (stages per pass), measured
 #   on the sources NTT_COUNTERS_SOURCES
-NTT_VALU_WAVE_INSTS_PER_COMMIT = {(3, 12): 1.062e8, (4, 11): 1.068e8, (5, 10): 1.146e8, (6, 9): 1.150e8,
-                                  (7, 8): 1.162e8, (8, 7): 1.216e8}
-NTT_COUNTERS_SOURCES = "49be5e50bc433eb1"
+NTT_VALU_WAVE_INSTS_PER_COMMIT = {(3, 12): 1.069e8, (4, 11): 1.065e8, (5, 10): 1.113e8, (6, 9): 1.119e8,
+                                  (7, 8): 1.131e8, (8, 7): 1.184e8}
+NTT_COUNTERS_SOURCES = "e7fd9ac3372ff032"
 # 32-bit VALU issue peak: 256 CUs x 4 SIMDs x one wave64 instruction per 4
 # cycles x 2.4 GHz = 39.3 T lane-ops/s (MI355X's published 78.6 TFLOP/s
 # vector FP64 counts an FMA as 2 flops on the same issue rate)

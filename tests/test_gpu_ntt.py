@@ -131,7 +131,7 @@ def test_invalid_lde_arguments(zk):
 
 
 # The passes compute on lazy values and leave out what a random operand needs
-# once in 2^32, doing a tile again exactly where it was needed after all.
+# once in 2^32, fixing the lanes where it was needed after all.
 # Words at and above p, runs of -1 and multiples of 2^48 reach that in every
 # kernel: single tiles (ragged and whole), one- and two-round strided passes
 # of each stage count, in place, through the coset and from coefficients.

@@ -482,7 +482,8 @@ __device__ __forceinline__ uint64_t reduce128_rare(uint64_t lo, uint64_t hi, uin
 }
 
 __device__ __forceinline__ void reduce128_rare2(uint64_t lo0, uint64_t hi0, uint64_t cin0, uint64_t lo1, uint64_t hi1,
-                                                uint64_t cin1, uint64_t &r0, uint64_t &r1, uint64_t &bad)
+                                                uint64_t cin1, uint64_t &r0, uint64_t &r1, uint64_t &bad, uint64_t &b0,
+                                                uint64_t &b1)
 {
     uint64_t u0, u1, sc0, sc1;
     uint32_t cv0, cv1;
@@ -494,7 +495,7 @@ __device__ __forceinline__ void reduce128_rare2(uint64_t lo0, uint64_t hi0, uint
         : [u0] "=&v"(u0), [u1] "=&v"(u1), [sc0] "=&s"(sc0), [sc1] "=&s"(sc1), [cv0] "=&v"(cv0), [cv1] "=&v"(cv1)
         : [a0] "v"(lo32(hi0)), [l0] "v"(lo0), [a1] "v"(lo32(hi1)), [l1] "v"(lo1));
     uint32_t zl0, zh0, zl1, zh1;
-    uint64_t b10, b0, b11, b1;
+    uint64_t b10, b11;
     asm("v_subb_co_u32_e64 %[zl0], %[b10], %[ul0], %[h10], %[ci0]\n\t"
         "v_subb_co_u32_e64 %[zl1], %[b11], %[ul1], %[h11], %[ci1]\n\t"
         "s_nop 0\n\t"
@@ -526,10 +527,10 @@ __device__ __forceinline__ uint64_t mul_rare(uint64_t a, uint64_t b, uint64_t &b
 __device__ __forceinline__ void mul_rare2(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_t &r0,
                                           uint64_t &r1, uint64_t &bad)
 {
-    uint64_t lo0, hi0, c0, lo1, hi1, c1;
+    uint64_t lo0, hi0, c0, lo1, hi1, c1, m0, m1;
     mul128c(a0, b0, lo0, hi0, c0);
     mul128c(a1, b1, lo1, hi1, c1);
-    reduce128_rare2(lo0, hi0, c0, lo1, hi1, c1, r0, r1, bad);
+    reduce128_rare2(lo0, hi0, c0, lo1, hi1, c1, r0, r1, bad, m0, m1);
 }
 
 // reduce96_lazy without its second step, which adds EPS in the lanes of
@@ -556,18 +557,36 @@ __device__ __forceinline__ uint64_t add_eps(uint64_t u, uint64_t lanes)
 // ---- butterflies of transforms: sums, differences and products of lazy values
 //
 // A sum whose carry or a difference whose borrow has been folded in as EPS
-// carries or borrows again only if an operand was not canonical (a random
-// lazy product is not once in 2^32).  Those lanes go to `bad` as above.  A
-// butterfly is 9 instructions here and its product 12, against 12 and 18 in
-// canonical form.
+// carries or borrows again only if an operand was not canonical, and a product
+// borrows (reduce128_rare) once in 2^32 for random operands; but values of a
+// trace are often small numbers, and small negative ones times the negative
+// powers of two among the twiddles do it every time.  So the lanes are fixed in
+// place behind a uniform branch, by one EPS: what was left out is added to (or
+// taken from) the wrapped result, which is then exact.  A butterfly is 9
+// instructions here and its product 12, against 12 and 18 in canonical form.
+
+// x - EPS in the lanes of the mask.
+__device__ __forceinline__ uint64_t sub_eps(uint64_t x, uint64_t lanes)
+{
+    uint32_t dlo, dhi, bv;
+    uint64_t b;
+    asm("s_nop 1\n\t"
+        "v_cndmask_b32_e64 %[bv], 0, -1, %[m]\n\t"
+        "v_sub_co_u32_e64 %[dlo], %[b], %[xl], %[bv]\n\t"
+        "s_nop 1\n\t"
+        "v_subb_co_u32_e64 %[dhi], %[b], %[xh], 0, %[b]"
+        : [dlo] "=&v"(dlo), [dhi] "=&v"(dhi), [bv] "=&v"(bv), [b] "=&s"(b)
+        : [xl] "v"(lo32(x)), [xh] "v"(hi32(x)), [m] "s"(lanes));
+    return pack(dlo, dhi);
+}
 
 // s = a + b, d = a - b, for two pairs at once: every lane mask is read at
 // least two instructions after its write.
-__device__ __forceinline__ void add_sub_rare2(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_t &s0,
-                                              uint64_t &d0, uint64_t &s1, uint64_t &d1, uint64_t &bad)
+__device__ __forceinline__ void add_sub_lazy2(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_t &s0,
+                                              uint64_t &d0, uint64_t &s1, uint64_t &d1)
 {
     uint32_t sl0, sh0, dl0, dh0, cv0, bv0, sl1, sh1, dl1, dh1, cv1, bv1;
-    uint64_t mc0, mb0, mc1, mb1;
+    uint64_t mc0, mb0, mc1, mb1, any;
     asm("v_add_co_u32_e64 %[sl0], %[c0], %[al0], %[bl0]\n\t"
         "v_sub_co_u32_e64 %[dl0], %[b0], %[al0], %[bl0]\n\t"
         "v_add_co_u32_e64 %[sl1], %[c1], %[al1], %[bl1]\n\t"
@@ -585,24 +604,42 @@ __device__ __forceinline__ void add_sub_rare2(uint64_t a0, uint64_t b0, uint64_t
         "s_nop 0\n\t"
         "v_subb_co_u32_e64 %[dh0], %[b0], %[dh0], 0, %[b0]\n\t"
         "v_subb_co_u32_e64 %[dh1], %[b1], %[dh1], 0, %[b1]\n\t"
-        "s_or_b64 %[bad], %[bad], %[b0]\n\t"
-        "s_or_b64 %[bad], %[bad], %[b1]"
+        "s_or_b64 %[any], %[b0], %[b1]"
         : [sl0] "=&v"(sl0), [sh0] "=&v"(sh0), [dl0] "=&v"(dl0), [dh0] "=&v"(dh0), [cv0] "=&v"(cv0), [bv0] "=&v"(bv0),
           [sl1] "=&v"(sl1), [sh1] "=&v"(sh1), [dl1] "=&v"(dl1), [dh1] "=&v"(dh1), [cv1] "=&v"(cv1), [bv1] "=&v"(bv1),
-          [c0] "=&s"(mc0), [b0] "=&s"(mb0), [c1] "=&s"(mc1), [b1] "=&s"(mb1), [bad] "+s"(bad)
+          [c0] "=&s"(mc0), [b0] "=&s"(mb0), [c1] "=&s"(mc1), [b1] "=&s"(mb1), [any] "=&s"(any)
         : [al0] "v"(lo32(a0)), [ah0] "v"(hi32(a0)), [bl0] "v"(lo32(b0)), [bh0] "v"(hi32(b0)), [al1] "v"(lo32(a1)),
           [ah1] "v"(hi32(a1)), [bl1] "v"(lo32(b1)), [bh1] "v"(hi32(b1))
         : "scc");
     uint64_t k0, k1;
     asm("v_mad_u64_u32 %[r0], %[k0], %[cv0], -1, %[s0]\n\t"
         "v_mad_u64_u32 %[r1], %[k1], %[cv1], -1, %[s1]\n\t"
-        "s_or_b64 %[bad], %[bad], %[k0]\n\t"
-        "s_or_b64 %[bad], %[bad], %[k1]"
-        : [r0] "=&v"(s0), [k0] "=&s"(k0), [r1] "=&v"(s1), [k1] "=&s"(k1), [bad] "+s"(bad)
+        "s_or_b64 %[any], %[any], %[k0]\n\t"
+        "s_or_b64 %[any], %[any], %[k1]"
+        : [r0] "=&v"(s0), [k0] "=&s"(k0), [r1] "=&v"(s1), [k1] "=&s"(k1), [any] "+s"(any)
         : [cv0] "v"(cv0), [s0] "v"(pack(sl0, sh0)), [cv1] "v"(cv1), [s1] "v"(pack(sl1, sh1))
         : "scc");
     d0 = pack(dl0, dh0);
     d1 = pack(dl1, dh1);
+    if (__builtin_expect(any != 0, 0)) {
+        s0 = add_eps(s0, k0);
+        s1 = add_eps(s1, k1);
+        d0 = sub_eps(d0, mb0);
+        d1 = sub_eps(d1, mb1);
+    }
+}
+
+// Two products, exact (lazy).
+__device__ __forceinline__ void mul_fix2(uint64_t a0, uint64_t w0, uint64_t a1, uint64_t w1, uint64_t &r0, uint64_t &r1)
+{
+    uint64_t lo0, hi0, c0, lo1, hi1, c1, b0, b1, any = 0;
+    mul128c(a0, w0, lo0, hi0, c0);
+    mul128c(a1, w1, lo1, hi1, c1);
+    reduce128_rare2(lo0, hi0, c0, lo1, hi1, c1, r0, r1, any, b0, b1);
+    if (__builtin_expect(any != 0, 0)) {
+        r0 = sub_eps(r0, b0);
+        r1 = sub_eps(r1, b1);
+    }
 }
 
 // x * 2^E, lazy, for E < 96 and any x < 2^64: with x * 2^(E mod 32) =
@@ -611,7 +648,7 @@ __device__ __forceinline__ void add_sub_rare2(uint64_t a0, uint64_t b0, uint64_t
 //   32 <= E < 64 x0 * 2^32 + x1 * EPS - x2
 //   64 <= E      x0 * EPS - (x1 + x2 * 2^32).
 template <int E>
-__device__ __forceinline__ uint64_t mul_pow2_rare(uint64_t x, uint64_t &bad)
+__device__ __forceinline__ uint64_t mul_pow2_lazy(uint64_t x)
 {
     static_assert(E >= 0 && E < 96, "exponent below half the order of 2");
     constexpr int s = E % 32;
@@ -621,26 +658,8 @@ __device__ __forceinline__ uint64_t mul_pow2_rare(uint64_t x, uint64_t &bad)
     else if constexpr (E < 32) return reduce96_lazy(l, x2);
     else if constexpr (E == 32) return shl32_lazy(x);
     else if constexpr (E < 64) {
-        // lo + hi * 2^64 with lo = x0 * 2^32, hi = (x1, x2): reduce128_rare without a borrow in
-        uint64_t u, sc;
-        uint32_t cv;
-        asm("v_mad_u64_u32 %[u], %[sc], %[h0], -1, %[lo]\n\t"
-            "s_nop 1\n\t"
-            "v_cndmask_b32_e64 %[cv], 0, 1, %[sc]"
-            : [u] "=&v"(u), [sc] "=&s"(sc), [cv] "=&v"(cv)
-            : [h0] "v"(hi32(l)), [lo] "v"(pack(0u, lo32(l))));
-        uint32_t zlo, zhi;
-        uint64_t b;
-        asm("v_sub_co_u32_e64 %[zlo], %[b], %[ulo], %[h1]\n\t"
-            "s_nop 1\n\t"
-            "v_subb_co_u32_e64 %[zhi], %[b], %[uhi], 0, %[b]\n\t"
-            "s_or_b64 %[bad], %[bad], %[b]"
-            : [zlo] "=&v"(zlo), [zhi] "=&v"(zhi), [b] "=&s"(b), [bad] "+s"(bad)
-            : [ulo] "v"(lo32(u)), [uhi] "v"(hi32(u)), [h1] "v"(x2)
-            : "scc");
-        uint64_t r, j;
-        asm("v_mad_u64_u32 %[r], %[j], %[cv], -1, %[z]" : [r] "=&v"(r), [j] "=&s"(j) : [cv] "v"(cv), [z] "v"(pack(zlo, zhi)));
-        return r;
+        // lo + hi * 2^64 with lo = x0 * 2^32, hi = (x1, x2)
+        return reduce128_lazy(pack(0u, lo32(l)), pack(hi32(l), x2));
     } else {
         // the subtrahend is below 2^62, so the second borrow cannot be: a
         // first one leaves at least 2^64 - 2^62

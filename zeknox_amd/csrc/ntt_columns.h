@@ -144,19 +144,13 @@ k_ntt_columns(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one,
 {
     constexpr int N = ColumnShape<LT, LE>::kLanes;
     __shared__ uint64_t lds[ColumnShape<LT, LE>::kSlots];
-    __shared__ uint32_t flags[N / 64];
-    uint32_t t = threadIdx.x;
+    const uint32_t t = threadIdx.x;
     const uint64_t b = first + blockIdx.x;
     const NttPass a = pass_at(passes, npasses, one, b);
-    uint64_t tile = b - a.tile_begin;
+    const uint64_t tile = b - a.tile_begin;
     Lazy lazy;
     column_transform<LT, LE, L, INV>(lazy, lds, a, post, tile, t);
-    if (__builtin_expect(barrier_any<N>(flags, lazy.bad), 0)) {
-        Exact exact;
-        again(t, tile);
-        column_transform<LT, LE, L, INV>(exact, lds, a, post, tile, t);
-        __syncthreads();
-    }
+    __syncthreads();
     const uint64_t base = (tile << LT) + t;
     const gptr<uint64_t> p = gmem(a.buf) + base;
 #pragma unroll

@@ -313,21 +313,15 @@ __global__ void __launch_bounds__(kNttThreads) __attribute__((amdgpu_waves_per_e
 k_ntt_tiles(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
 {
     __shared__ uint64_t lds[(1 << kNttTileLog) + (1 << kNttTileLog) / 32];
-    __shared__ uint32_t flags[kNttThreads / 64];
 
     const uint64_t bid = first + blockIdx.x;
     const NttPass a = pass_at(passes, npasses, one, bid);
-    uint64_t tile = bid - a.tile_begin;
-    uint32_t t = threadIdx.x;
+    const uint64_t tile = bid - a.tile_begin;
+    const uint32_t t = threadIdx.x;
 
     Lazy lazy;
     tile_transform<CONTIG>(lazy, lds, a, tile, t);
-    if (__builtin_expect(barrier_any(flags, lazy.bad), 0)) {
-        Exact exact;
-        again(t, tile);
-        tile_transform<CONTIG>(exact, lds, a, tile, t);
-        __syncthreads();
-    }
+    __syncthreads();
 
     // ---- store, coalesced
     const uint64_t ibase = CONTIG ? (tile << kNttTileLog) + t : tile_index(a, tile, t);
@@ -382,19 +376,13 @@ __global__ void __launch_bounds__(kNttThreads) __attribute__((amdgpu_waves_per_e
 k_ntt_contig_reg(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
 {
     __shared__ uint64_t lds[(1 << kNttTileLog) + (1 << kNttTileLog) / 32];
-    __shared__ uint32_t flags[kNttThreads / 64];
-    uint32_t t = threadIdx.x;
+    const uint32_t t = threadIdx.x;
     const uint64_t b = first + blockIdx.x;
     const NttPass a = pass_at(passes, npasses, one, b);
-    uint64_t tile = b - a.tile_begin;
+    const uint64_t tile = b - a.tile_begin;
     Lazy lazy;
     contig_transform(lazy, lds, a, tile, t);
-    if (__builtin_expect(barrier_any(flags, lazy.bad), 0)) {
-        Exact exact;
-        again(t, tile);
-        contig_transform(exact, lds, a, tile, t);
-        __syncthreads();
-    }
+    __syncthreads();
     const gptr<uint64_t> p = gmem(a.buf) + (tile << kNttTileLog) + t;
 #pragma unroll
     for (int i = 0; i < kNttPerThread; i++) p[i << 8] = lds[lds_slot(t + kNttThreads * i)];
@@ -493,11 +481,15 @@ __device__ __forceinline__ void strided1_transform(A &ar, uint64_t (&x)[kNttPerT
     strided_tw_load<K>(a, tile, t, w);
     const StridedRows r = strided_rows<MODE>(a, tile, t);
     if constexpr (MODE == kSrcLde) {
+        // (every load before the products: their branches would hold it back)
+        uint64_t f[kNttPerThread];
 #pragma unroll
-        for (int i = 0; i < kNttPerThread; i++) x[i] = r.src[strided_step<K>(a, i)];
+        for (int i = 0; i < kNttPerThread; i++) {
+            x[i] = r.src[strided_step<K>(a, i)];
+            f[i] = r.fac[strided_step<K>(a, i)];
+        }
 #pragma unroll
-        for (int i = 0; i < kNttPerThread; i += 2)
-            ar.mul2(x[i], r.fac[strided_step<K>(a, i)], x[i + 1], r.fac[strided_step<K>(a, i + 1)]);
+        for (int i = 0; i < kNttPerThread; i += 2) ar.mul2(x[i], f[i], x[i + 1], f[i + 1]);
     } else {
 #pragma unroll
         for (int i = 0; i < kNttPerThread; i++) x[i] = A::load(r.src[strided_step<K>(a, i)]);
@@ -510,23 +502,18 @@ __device__ __forceinline__ void strided1_transform(A &ar, uint64_t (&x)[kNttPerT
         });
 }
 
-// Work-group k runs tile first + k of the list.  A wave redoes its own words.
+// Work-group k runs tile first + k of the list.
 template <int MODE, int K>
 __global__ void __launch_bounds__(kNttThreads)
 k_ntt_strided1_tiles(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
 {
-    uint32_t t = threadIdx.x;
+    const uint32_t t = threadIdx.x;
     const uint64_t b = first + blockIdx.x;
     const NttPass a = pass_at(passes, npasses, one, b);
-    uint64_t tile = b - a.tile_begin;
+    const uint64_t tile = b - a.tile_begin;
     uint64_t x[kNttPerThread];
     Lazy lazy;
     strided1_transform<MODE, K>(lazy, x, a, tile, t);
-    if (__builtin_expect(lazy.bad != 0, 0)) {
-        Exact exact;
-        again(t, tile);
-        strided1_transform<MODE, K>(exact, x, a, tile, t);
-    }
     const StridedRows r = strided_rows<MODE>(a, tile, t);
 #pragma unroll
     for (int i = 0; i < kNttPerThread; i++) r.buf[strided_step<K>(a, i)] = x[i];
@@ -674,12 +661,14 @@ __device__ __forceinline__ void strided2_transform(A &ar, uint64_t *lds, const N
     strided2_tw_load<M>(a, tile, t, wa, wb);
     uint64_t x[kNttPerThread];
     if constexpr (MODE == kSrcLde) {
+        uint64_t f[kNttPerThread];
 #pragma unroll
-        for (int i = 0; i < kNttPerThread; i++) x[i] = gmem(r.src + strided2_step<M>(a, i))[off];
+        for (int i = 0; i < kNttPerThread; i++) {
+            x[i] = gmem(r.src + strided2_step<M>(a, i))[off];
+            f[i] = gmem(r.fac + strided2_step<M>(a, i))[off];
+        }
 #pragma unroll
-        for (int i = 0; i < kNttPerThread; i += 2)
-            ar.mul2(x[i], gmem(r.fac + strided2_step<M>(a, i))[off], x[i + 1],
-                    gmem(r.fac + strided2_step<M>(a, i + 1))[off]);
+        for (int i = 0; i < kNttPerThread; i += 2) ar.mul2(x[i], f[i], x[i + 1], f[i + 1]);
     } else {
 #pragma unroll
         for (int i = 0; i < kNttPerThread; i++) x[i] = A::load(gmem(r.src + strided2_step<M>(a, i))[off]);
@@ -698,19 +687,13 @@ __global__ void __launch_bounds__(kNttThreads) __attribute__((amdgpu_waves_per_e
 k_ntt_strided2_tiles(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, uint64_t first)
 {
     __shared__ uint64_t lds[(1 << kNttTileLog) + (1 << kNttTileLog) / 32];
-    __shared__ uint32_t flags[kNttThreads / 64];
-    uint32_t t = threadIdx.x;
+    const uint32_t t = threadIdx.x;
     const uint64_t b = first + blockIdx.x;
     const NttPass a = pass_at(passes, npasses, one, b);
-    uint64_t tile = b - a.tile_begin;
+    const uint64_t tile = b - a.tile_begin;
     Lazy lazy;
     strided2_transform<MODE, M>(lazy, lds, a, tile, t);
-    if (__builtin_expect(barrier_any(flags, lazy.bad), 0)) {
-        Exact exact;
-        again(t, tile);
-        strided2_transform<MODE, M>(exact, lds, a, tile, t);
-        __syncthreads();
-    }
+    __syncthreads();
     const Strided2Rows r = strided2_rows<MODE, M>(a, tile);
     const uint32_t off = strided2_off<M>(a, t);
 #pragma unroll

@@ -1,5 +1,5 @@
 // What the transform kernels share: their arithmetic on lazy values, the
-// second computation of a tile, the small-root stages, descriptors.
+// small-root stages, descriptors.
 #pragma once
 #include <type_traits>
 
@@ -14,90 +14,36 @@ __device__ __forceinline__ uint32_t lds_slot(uint32_t u) { return u + (u >> 5); 
 
 // ---- arithmetic of the passes
 //
-// A butterfly is 21 instructions on lazy values (Lazy) rather than 30 on
-// canonical ones (Exact): what a random operand needs once in 2^32 is left
-// out and its lanes noted in `bad` (gl64.h).  A tile with such a lane is
-// computed again with Exact, from the source that nothing has overwritten
-// yet.  Words between the passes of a transform are lazy too; the contiguous
-// pass, the last, stores canonical ones.
+// Words are lazy (below 2^64) inside a transform and between its passes; a
+// butterfly is 21 instructions and a test of two lane masks (gl64.h) rather
+// than 30 on canonical words.  The last pass stores canonical ones.
 //
-// Bounds, 64 x 2^20 forward (1.07 GB of traffic a pass): the 12-stage
-// contiguous pass 375 -> 318 us, of which its loads and stores alone take
-// 273; the 8-stage strided pass 298 -> 294 us, bound by its loads and stores
-// (250 alone).  The whole transform 906 -> 854 us, alternating builds.
-
+// Bounds, 32 commits of 135 x 2^15 rate 3: the first pass, bound by its loads
+// and stores (3.2 ms alone), 3.55 -> 3.53 ms; the 12-stage contiguous pass, of
+// which they take 4.4, 5.93 -> 5.57.  (Redoing a whole tile exactly instead of
+// fixing the lanes took 3.33 and 5.26 on random words, but 41 us against 27 for
+// the inverse of 101 x 2^13 bits, as for any trace of small numbers.)
 struct Lazy {
-    uint64_t bad;
-    // (zero from the scalar unit: as a constant it may join the masks of
-    // another branch in a VGPR)
-    __device__ __forceinline__ Lazy() { asm("s_mov_b64 %0, 0" : "=s"(bad)); }
     static __device__ __forceinline__ uint64_t load(uint64_t x) { return x; }
     static __device__ __forceinline__ uint64_t result(uint64_t x) { return gl::canon(x); }
     __device__ __forceinline__ void add_sub2(uint64_t &x0, uint64_t &y0, uint64_t &x1, uint64_t &y1)
     {
         uint64_t s0, d0, s1, d1;
-        gl::add_sub_rare2(x0, y0, x1, y1, s0, d0, s1, d1, bad);
+        gl::add_sub_lazy2(x0, y0, x1, y1, s0, d0, s1, d1);
         x0 = s0, y0 = d0, x1 = s1, y1 = d1;
     }
     __device__ __forceinline__ void mul2(uint64_t &x0, uint64_t w0, uint64_t &x1, uint64_t w1)
     {
         uint64_t r0, r1;
-        gl::mul_rare2(x0, w0, x1, w1, r0, r1, bad);
+        gl::mul_fix2(x0, w0, x1, w1, r0, r1);
         x0 = r0, x1 = r1;
     }
-    __device__ __forceinline__ uint64_t mul(uint64_t x, uint64_t w) { return gl::mul_rare(x, w, bad); }
     template <int E>
     __device__ __forceinline__ uint64_t shift(uint64_t x)
     {
-        return gl::mul_pow2_rare<E>(x, bad);
+        return gl::mul_pow2_lazy<E>(x);
     }
 };
-
-struct Exact {
-    static __device__ __forceinline__ uint64_t load(uint64_t x) { return gl::canon(x); }
-    static __device__ __forceinline__ uint64_t result(uint64_t x) { return x; }
-    __device__ __forceinline__ void add_sub2(uint64_t &x0, uint64_t &y0, uint64_t &x1, uint64_t &y1)
-    {
-        const uint64_t s0 = gl::add(x0, y0), d0 = gl::sub(x0, y0), s1 = gl::add(x1, y1), d1 = gl::sub(x1, y1);
-        x0 = s0, y0 = d0, x1 = s1, y1 = d1;
-    }
-    __device__ __forceinline__ void mul2(uint64_t &x0, uint64_t w0, uint64_t &x1, uint64_t w1)
-    {
-        x0 = mul(x0, w0);
-        x1 = mul(x1, w1);
-    }
-    // (the form with the fewest live registers)
-    __device__ __forceinline__ uint64_t mul(uint64_t x, uint64_t w) { return gl::mul_nc(x, w); }
-    template <int E>
-    __device__ __forceinline__ uint64_t shift(uint64_t x)
-    {
-        // (x is canonical; the compiler folds a canon() that directly follows a
-        // sub() into its carry chain and counts the wrap of that as its own)
-        if constexpr (E == 0) return x;
-        else return gl::mul_pow2<E>(x);
-    }
-};
-
-// The lane and tile of the second computation, through values the compiler
-// cannot see through: nothing the first one loaded or computed stays in
-// registers for it.
-__device__ __forceinline__ void again(uint32_t &t, uint64_t &tile)
-{
-    asm volatile("; again %0 %1" : "+v"(t), "+s"(tile));
-}
-
-// Whether any wave of the work-group noted a lane; ends with every LDS write
-// before it visible.
-template <int LANES = kNttThreads>
-__device__ __forceinline__ bool barrier_any(uint32_t *flags, uint64_t bad)
-{
-    if ((threadIdx.x & 63) == 0) flags[threadIdx.x >> 6] = bad != 0 ? 1u : 0u;
-    __syncthreads();
-    uint32_t any = 0;
-#pragma unroll
-    for (int i = 0; i < LANES / 64; i++) any |= flags[i];
-    return __builtin_amdgcn_readfirstlane(any) != 0;
-}
 
 // ---- stages whose twiddles are roots of order <= 16: w = 1 (no product) or
 // a power of two (a shift; 2^96 = -1 is the difference taken the other way

@@ -148,17 +148,11 @@ k_ntt_first(NttPass a)
 {
     constexpr int LE = kTwoWords, C = kTwoTile - M1;
     __shared__ uint64_t lds[TwoShape::kSlots];
-    __shared__ uint32_t flags[kTwoLanes / 64];
-    uint32_t t = threadIdx.x;
-    uint64_t tile = two_tile<C>(blockIdx.x);
+    const uint32_t t = threadIdx.x;
+    const uint64_t tile = two_tile<C>(blockIdx.x);
     uint64_t x[1 << LE];
     Lazy lazy;
     first_transform<M1, INV>(lazy, lds, x, a, tile, t);
-    if (__builtin_expect(barrier_any<kTwoLanes>(flags, lazy.bad), 0)) {
-        Exact exact;
-        again(t, tile);
-        first_transform<M1, INV>(exact, lds, x, a, tile, t);
-    }
     const uint32_t s = a.s_lo, ch = (uint32_t)tile & ((1u << (s - C)) - 1);
     const gptr<uint64_t> row = gmem(a.buf) + ((tile >> (s - C)) << a.L);
 #pragma unroll
@@ -248,17 +242,11 @@ k_ntt_second(NttPass a, ColumnPost post)
 {
     constexpr int LE = kTwoWords, C = kTwoTile - M2;
     __shared__ uint64_t lds[TwoShape::kSlots];
-    __shared__ uint32_t flags[kTwoLanes / 64];
-    uint32_t t = threadIdx.x;
-    uint64_t tile = two_tile<C>(blockIdx.x);
+    const uint32_t t = threadIdx.x;
+    const uint64_t tile = two_tile<C>(blockIdx.x);
     Lazy lazy;
     second_transform<M2, INV>(lazy, lds, a, post, tile, t);
-    if (__builtin_expect(barrier_any<kTwoLanes>(flags, lazy.bad), 0)) {
-        Exact exact;
-        again(t, tile);
-        second_transform<M2, INV>(exact, lds, a, post, tile, t);
-        __syncthreads();
-    }
+    __syncthreads();
     const uint32_t gb = post.lg - kTwoTile, gr = (uint32_t)tile & ((1u << gb) - 1);
     const gptr<uint64_t> col = gmem(a.buf) + ((tile >> gb) << post.lg) + (gr << C);
 #pragma unroll
