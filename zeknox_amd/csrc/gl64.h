@@ -112,10 +112,14 @@ __device__ __forceinline__ uint64_t reduce96(uint64_t lo, uint32_t top) { return
 // through inline asm.  gfx950 needs two wait states between a VALU write of
 // a lane mask and a VALU read of it (the compiler inserts the same for its
 // own carry chains): every mask is created and consumed inside one asm
-// block, behind an s_nop 1 -- except the product carry of mul128c, which is
-// read by the second asm block of reduce128c_lazy(2): that block depends on
+// block, behind an s_nop 1, or leaves it two wait states after its write --
+// except the product carry of mul128c, which is read by the second asm block
+// of the reductions that take it: that block depends on
 // the first one, whose inputs depend on the multiply-add writing the mask,
-// so at least the first block's three instructions lie between them.  The
+// so at least the first block's three instructions lie between them (a wait
+// of its own would cost every product an issue slot; that the compiler does
+// not spill it in between is checked in the machine code:
+// tests/test_wait_states.py).  The
 // inline constant -1 is 0xFFFFFFFF = EPS as the 32-bit multiplicand.
 
 // Lazy residue (below 2^64, congruent mod p) of top * 2^64 + lo, top < 2^32:
@@ -535,11 +539,16 @@ __device__ __forceinline__ void mul_rare2(uint64_t a0, uint64_t b0, uint64_t a1,
 
 // reduce96_lazy without its second step, which adds EPS in the lanes of
 // `carry`: a carry out of lo + top * EPS needs lo above 2^64 - top * 2^32
-// (for top < 2^16 one value in 2^16).  add_eps is that step.
+// (for top < 2^16 one value in 2^16).  add_eps is that step.  The mask leaves
+// the block, so its two wait states are in it: whatever the compiler reads it
+// with next (the scalar unit, or a v_writelane_b32 that spills it) finds it.
 __device__ __forceinline__ uint64_t reduce96_rare(uint64_t lo, uint32_t top, uint64_t &carry)
 {
     uint64_t u;
-    asm("v_mad_u64_u32 %[u], %[c], %[top], -1, %[lo]" : [u] "=&v"(u), [c] "=&s"(carry) : [top] "v"(top), [lo] "v"(lo));
+    asm("v_mad_u64_u32 %[u], %[c], %[top], -1, %[lo]\n\t"
+        "s_nop 1"
+        : [u] "=&v"(u), [c] "=&s"(carry)
+        : [top] "v"(top), [lo] "v"(lo));
     return u;
 }
 __device__ __forceinline__ uint64_t add_eps(uint64_t u, uint64_t lanes)
@@ -580,8 +589,8 @@ __device__ __forceinline__ uint64_t sub_eps(uint64_t x, uint64_t lanes)
     return pack(dlo, dhi);
 }
 
-// s = a + b, d = a - b, for two pairs at once: every lane mask is read at
-// least two instructions after its write.
+// s = a + b, d = a - b, for two pairs at once: every lane mask is read, or
+// leaves its block, at least two instructions after its write.
 __device__ __forceinline__ void add_sub_lazy2(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_t &s0,
                                               uint64_t &d0, uint64_t &s1, uint64_t &d1)
 {
@@ -604,7 +613,8 @@ __device__ __forceinline__ void add_sub_lazy2(uint64_t a0, uint64_t b0, uint64_t
         "s_nop 0\n\t"
         "v_subb_co_u32_e64 %[dh0], %[b0], %[dh0], 0, %[b0]\n\t"
         "v_subb_co_u32_e64 %[dh1], %[b1], %[dh1], 0, %[b1]\n\t"
-        "s_or_b64 %[any], %[b0], %[b1]"
+        "s_or_b64 %[any], %[b0], %[b1]\n\t"
+        "s_nop 0"
         : [sl0] "=&v"(sl0), [sh0] "=&v"(sh0), [dl0] "=&v"(dl0), [dh0] "=&v"(dh0), [cv0] "=&v"(cv0), [bv0] "=&v"(bv0),
           [sl1] "=&v"(sl1), [sh1] "=&v"(sh1), [dl1] "=&v"(dl1), [dh1] "=&v"(dh1), [cv1] "=&v"(cv1), [bv1] "=&v"(bv1),
           [c0] "=&s"(mc0), [b0] "=&s"(mb0), [c1] "=&s"(mc1), [b1] "=&s"(mb1), [any] "=&s"(any)
