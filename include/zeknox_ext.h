@@ -126,7 +126,9 @@ RustError zkx_commit_batch_pieces(size_t device_id, const ZkxCommitJob *jobs, si
 /* Device working memory zkx_commit_batch needs for these jobs, in bytes.
  * The library keeps it between calls (one buffer per device, grown as
  * needed); zkx_commit_trim frees it, and the scratch of at most 128 MiB that
- * the natural-order transforms keep. */
+ * the natural-order transforms keep (they run without it, slower, where there
+ * is no memory for it; an allocation of the library that finds no memory left
+ * frees it and tries again). */
 size_t zkx_commit_scratch_bytes(const ZkxCommitJob *jobs, size_t njobs);
 RustError zkx_commit_trim(size_t device_id);
 

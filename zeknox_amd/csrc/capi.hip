@@ -364,9 +364,7 @@ RustError zkx_commit_trim(size_t device_id)
         Engine &e = default_engine(d);
         std::lock_guard<std::mutex> g(e.mu);
         e.trim();
-        std::lock_guard<std::mutex> gd(d.mu);
-        d.sync();
-        d.ntt_scratch = DevBuf();
+        d.drop_spare();
     });
 }
 

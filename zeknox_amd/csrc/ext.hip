@@ -106,7 +106,7 @@ RustError zkx_device_malloc(size_t device_id, void **ptr, size_t bytes)
         if (!ptr) invalid("null pointer");
         device(device_id);
         *ptr = nullptr;
-        if (bytes) ZKX_HIP(hipMalloc(ptr, bytes));
+        if (bytes) *ptr = device_alloc(bytes);
     });
 }
 

@@ -271,8 +271,7 @@ const uint64_t *lde_factor_table(Device &d, uint32_t lg_n, uint32_t rate, bool i
         fb.c[b] = host_mul(gen, host_pow(w, rb));
     }
     const uint64_t total = 1ull << lg;
-    uint64_t *F = nullptr;
-    ZKX_HIP(hipMalloc(&F, total * sizeof(uint64_t)));
+    uint64_t *F = static_cast<uint64_t *>(device_alloc(total * sizeof(uint64_t)));
     const uint64_t chunk = lg_n < 6 ? (1ull << lg_n) : 64;
     const uint64_t threads = total / chunk;
     hipLaunchKernelGGL(k_lde_factors, dim3((uint32_t)((threads + kNttThreads - 1) / kNttThreads)),
@@ -315,16 +314,17 @@ bool columns(Device &d, uint64_t *buf, uint32_t L, uint32_t rate, uint32_t cols,
 }
 
 constexpr size_t kTwoScratch = 128ull << 20;
+constexpr uint64_t kTwoLeast = 1ull << 18;  // words
 
 // Columns of a chunk of the two-launch transform (ntt_two.h) of stages L into
 // `cols` columns of 2^lg, 0 where passes and a bit reversal are used.
-// Below 2^18 words in all both ways are a few tiles' latency and the passes, on
+// Below kTwoLeast words in all both ways are a few tiles' latency and the passes, on
 // smaller tiles, win (2^15 x 4 30.5 / 29.9 us, 2^16 x 1 31.3 / 30.0; 2^16 x 4
 // 30.7 / 31.9, 2^18 x 1 31.7 / 33.6).  A chunk of 64 MiB costs 5% (too few
 // tiles a launch), one of 512 gains nothing.
 uint64_t two_launch_chunk(uint32_t L, uint32_t lg, uint64_t cols)
 {
-    if (L < 15 || L > 20 || (cols << lg) < (1ull << 18) || (sizeof(uint64_t) << lg) > kTwoScratch) return 0;
+    if (L < 15 || L > 20 || (cols << lg) < kTwoLeast || (sizeof(uint64_t) << lg) > kTwoScratch) return 0;
     return std::min<uint64_t>(cols, kTwoScratch / (sizeof(uint64_t) << lg));
 }
 
@@ -334,22 +334,16 @@ bool two_launches(Device &d, uint64_t *buf, uint32_t L, uint32_t rate, uint32_t 
                   const uint64_t *src, const uint64_t *factors, const uint64_t *coset_after)
 {
     const uint32_t lg = L + rate;
-    const uint64_t chunk = two_launch_chunk(L, lg, cols);
+    uint64_t chunk = two_launch_chunk(L, lg, cols);
     if (!chunk) return false;
-    const size_t bytes = (size_t)(chunk * sizeof(uint64_t)) << lg;
-    if (d.ntt_scratch.bytes < bytes) {
-        d.sync();
-        d.ntt_scratch = DevBuf();
-        try {
-            d.ntt_scratch = DevBuf(bytes);
-        } catch (const Error &) {
-            (void)hipGetLastError();  // no memory left for it: the passes need none
-            return false;
-        }
-    }
     NttPass a{};
     a.coset = factors;
     a.tw_lg = d.twiddle_tables_upto(L);
+    // until the launches are queued; no memory left for it, or only for chunks
+    // below the rule's size: the passes need none
+    std::lock_guard<std::mutex> g(d.spare_mu);
+    chunk = d.ntt_scratch.hold(chunk, sizeof(uint64_t) << lg);
+    if ((chunk << lg) < kTwoLeast) return false;
     a.L = L;
     a.rate = rate;
     a.mode = mode;
@@ -364,14 +358,14 @@ bool two_launches(Device &d, uint64_t *buf, uint32_t L, uint32_t rate, uint32_t 
         {
             ProfScope ps(mode == kSrcLde ? "ntt_pass_lde" : "ntt_pass", d.stream);
             a.src = src + (c << L);
-            a.buf = d.ntt_scratch.as<uint64_t>();
+            a.buf = static_cast<uint64_t *>(d.ntt_scratch.get());
             a.m = (L + 1) / 2;
             a.s_lo = L - a.m;
             launch_two_first(d.stream, a);
             ZKX_HIP(hipGetLastError());
         }
         ProfScope ps("ntt_pass", d.stream);
-        a.src = d.ntt_scratch.as<uint64_t>();
+        a.src = static_cast<uint64_t *>(d.ntt_scratch.get());
         a.buf = buf + (c << lg);
         a.m = L / 2;
         a.s_lo = 0;

@@ -16,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "spare.h"
 #include "tuning.h"
 
 namespace zkx {
@@ -37,6 +38,14 @@ struct Error : std::runtime_error {
         hipError_t zkx_e_ = (call);                                           \
         if (zkx_e_ != hipSuccess) ::zkx::throw_hip(zkx_e_, #call, __FILE__, __LINE__); \
     } while (0)
+
+// Memory on the current device.  Where there is none left, the device's spare
+// memory is given back and the allocation tried once more: nothing that fits
+// without that memory fails because of it.
+void *device_alloc(size_t bytes);
+// The same without that second try; null when there is none.
+void *device_alloc_spare(size_t bytes);
+void device_free(void *p);
 
 // A device buffer owned by the library; freed on destruction.
 struct DevBuf {
@@ -69,9 +78,14 @@ struct Device {
     hipDeviceProp_t prop{};
     std::mutex mu;                 // serialises table builds and compute calls
 
-    // Scratch of the transforms in two launches (ntt.hip), at most 128 MiB;
-    // used under `mu` on `stream`, given back by zkx_commit_trim.
-    DevBuf ntt_scratch;
+    // Scratch of the transforms in two launches (ntt.hip), at most 128 MiB.
+    // A transform holds spare_mu until its launches on `stream` are queued;
+    // given back by zkx_commit_trim and by an allocation that finds no memory
+    // left, which both wait for the device.  Taken last: whoever holds it
+    // allocates nothing else and takes no other lock.
+    std::mutex spare_mu;
+    SpareMemory ntt_scratch{device_alloc_spare, device_free};
+    bool drop_spare();
 
     // Resident tables (twiddles per log size, coset powers).
     uint64_t *twiddles[33] = {};   // twiddles[k][i] = w_{2^k}^i, i < 2^k

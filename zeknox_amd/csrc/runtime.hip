@@ -21,7 +21,7 @@ void throw_hip(hipError_t e, const char *what, const char *file, int line)
 
 DevBuf::DevBuf(size_t n) : bytes(n)
 {
-    if (n) ZKX_HIP(hipMalloc(&p, n));
+    if (n) p = device_alloc(n);
 }
 
 DevBuf::~DevBuf()
@@ -70,6 +70,43 @@ Device &device(size_t id)
     // a throwing creation leaves the flag unset for the next caller
     std::call_once(d.stream_once, [&] { ZKX_HIP(hipStreamCreate(&d.stream)); });
     return d;
+}
+
+void *device_alloc_spare(size_t bytes)
+{
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();  // answered here, not by the next launch
+    return nullptr;
+}
+
+// (hipFree waits for everything on the device)
+void device_free(void *p) { (void)hipFree(p); }
+
+void *device_alloc(size_t bytes)
+{
+    void *p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        int id = 0;
+        bool dropped = false;
+        if (hipGetDevice(&id) == hipSuccess)
+            for (auto &d : registry().devs)
+                if (d->id == id) dropped = d->drop_spare();
+        if (dropped) e = hipMalloc(&p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        throw_hip(e, "hipMalloc", __FILE__, __LINE__);
+    }
+    return p;
+}
+
+bool Device::drop_spare()
+{
+    std::lock_guard<std::mutex> g(spare_mu);
+    return ntt_scratch.drop();
 }
 
 void Device::sync() { ZKX_HIP(hipStreamSynchronize(stream)); }
@@ -128,8 +165,7 @@ const uint64_t *Device::twiddle_table(uint32_t lg)
     if (lg > 32) invalid("log size " + std::to_string(lg) + " exceeds 32");
     if (!twiddles[lg]) {
         const uint64_t n = 1ull << lg;
-        uint64_t *p = nullptr;
-        ZKX_HIP(hipMalloc(&p, n * sizeof(uint64_t)));
+        uint64_t *p = static_cast<uint64_t *>(device_alloc(n * sizeof(uint64_t)));
         fill_powers(p, n, omega(lg), stream);
         twiddles[lg] = p;
         if (twiddle_ptrs.p)
@@ -159,7 +195,7 @@ void Device::build_coset(uint32_t lg, uint64_t gen)
         coset = nullptr;
     }
     if (!coset) {
-        ZKX_HIP(hipMalloc(&coset, n * sizeof(uint64_t)));
+        coset = static_cast<uint64_t *>(device_alloc(n * sizeof(uint64_t)));
         coset_lg = lg;
     }
     coset_gen = gen;
