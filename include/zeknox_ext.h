@@ -138,7 +138,11 @@ RustError zkx_commit_trim(size_t device_id);
  * (1..9; greedy or spread evenly), the leaves per Merkle work-group
  * (2^8..2^10) and, for Poseidon leaves, whether the permutations' MDS layers
  * run on the matrix cores or every step on the VALU.  No setting changes a
- * result.  Shapes without an entry use
+ * result.  A schedule that zkx_set_tuning set runs as it stands; otherwise the
+ * library builds Poseidon and Poseidon2 forests of at most 2^15 leaves (all of
+ * one hash in a batch) with a kernel of 2^6-leaf work-groups, and transforms of
+ * 2^13 to 2^20 in one or two launches, where that is faster, and schedules
+ * that it tuned itself are those of the rest.  Shapes without an entry use
  * the default, which the C-ABI entry points (compute_batched_lde,
  * fill_digests_buf_linear_gpu_with_gpu_ptr) use as well, except that until
  * zkx_set_tuning sets a default the Merkle entry points size the work-groups
@@ -203,7 +207,8 @@ int zkx_merkle_plan(uint64_t nl, uint64_t nc, uint32_t tile_log, uint64_t *count
                     uint32_t *tile_logs, uint32_t *first_ctr, int cap, uint64_t *counters);
 /* Forget every shape entry and restore the built-in default. */
 RustError zkx_tuning_clear(size_t device_id);
-/* The shape table as text, one shape per line. */
+/* The shape table as text, one shape per line (with a mark on those that
+ * zkx_set_tuning set). */
 RustError zkx_tuning_save(size_t device_id, const char *path);
 RustError zkx_tuning_load(size_t device_id, const char *path);
 

@@ -454,7 +454,8 @@ def get_tuning(commit=None, device_id=0):
 
 
 def set_tuning(tuning, commit=None, device_id=0):
-    """Schedule of the commit's shape, or the default (commit None)."""
+    """Schedule of the commit's shape, or the default (commit None); it runs as
+    it stands, where the library would otherwise choose kernels by size."""
     job = ctypes.byref(commit.job()) if commit is not None else None
     _check(lib.zkx_set_tuning(device_id, job, ctypes.byref(tuning)))
 

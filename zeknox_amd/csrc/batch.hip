@@ -148,14 +148,18 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
     for (size_t i = 0; i < n; i++)
         if (jobs[i].cap_height < jobs[i].lg_n + jobs[i].rate) tree_leaves += 1ull << (jobs[i].lg_n + jobs[i].rate);
     // (Poseidon and Poseidon2 forests small enough for it run on the
-    // 16-permutations-per-wave kernel, whatever the others of the batch do)
-    std::map<int, uint64_t> hash_leaves;
-    for (size_t i = 0; i < n; i++) hash_leaves[(int)jobs[i].hash_type] += 1ull << (jobs[i].lg_n + jobs[i].rate);
-    auto narrow_trees = [&](uint64_t ht) { return has_narrow_kernel(ht) && hash_leaves[(int)ht] <= kNarrowLeaves; };
+    // 16-permutations-per-wave kernel, whatever the others of the batch do,
+    // unless the caller set their schedule)
+    std::map<uint64_t, uint64_t> hash_leaves;
+    for (size_t i = 0; i < n; i++)
+        if (!tun[i].by_caller) hash_leaves[jobs[i].hash_type] += 1ull << (jobs[i].lg_n + jobs[i].rate);
     const uint64_t apart_from = dev_.level_launch_leaves.load();
-    auto by_level = [&](uint64_t ht) {
-        return !narrow_trees(ht) && batch_levels_apart(tree_leaves, ht, apart_from);
-    };
+    std::vector<char> narrow_tree(n), by_level(n);
+    for (size_t i = 0; i < n; i++) {
+        const uint64_t ht = jobs[i].hash_type;
+        narrow_tree[i] = has_narrow_kernel(ht) && !tun[i].by_caller && hash_leaves[ht] <= kNarrowLeaves;
+        by_level[i] = !narrow_tree[i] && batch_levels_apart(tree_leaves, ht, apart_from);
+    }
 
     // ---- plans
     std::vector<std::vector<NttPass>> ntt_plan(n);
@@ -188,14 +192,14 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
         specs[i] = s;
         mk_ctr[i] = total_ctr;
         uint64_t nctr = 0;
-        if (narrow_trees(j.hash_type)) {
+        if (narrow_tree[i]) {
             nctr = plan_merkle_narrow(s, nullptr, mk[i]);
         } else {
             std::vector<MerkleArgs> passes;
             plan_merkle(s, passes, tun[i].merkle_tile_log);
             nctr = fuse_merkle_passes(passes, mk[i]);
         }
-        if (by_level(j.hash_type)) mk[i].leaves_only = 1;  // the leaf pass alone: its levels are launched apart
+        if (by_level[i]) mk[i].leaves_only = 1;  // the leaf pass alone: its levels are launched apart
         else total_ctr += nctr;
         max_ntt = std::max(max_ntt, ntt_plan[i].size());
     }
@@ -222,40 +226,39 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
         uint64_t blocks = 0;
     };
     std::vector<LevelLaunch> levels;
-    for (int ht : {kPoseidon, kKeccak, kPoseidonBN128, kPoseidon2, kMonolith})
-        if (by_level((uint64_t)ht)) {
-            auto apart = [&](size_t i, uint32_t k) {
-                return (int)jobs[i].hash_type == ht && mk[i].lg_w >= k;
-            };
-            // mk[i].lg_w is the log2 width of tree i's leaf level per subtree
-            // (0: caps == leaves, no levels)
-            for (uint32_t k = 1;; k++) {
-                LevelLaunch l{ht, false, {}, {}};
-                uint64_t children = 0;
-                for (size_t i = 0; i < n; i++)
-                    if (apart(i, k)) children += specs[i].num_caps << (mk[i].lg_w - k + 1);
-                if (!children) break;
-                l.narrow = (has_narrow_kernel((uint64_t)ht) || has_tile_top((uint64_t)ht)) && children <= kNarrowNodes;
-                for (size_t i = 0; i < n; i++) {
-                    if (!apart(i, k)) continue;
-                    MerkleArgs a;
-                    if (l.narrow) {
-                        l.first_ctr.push_back(total_ctr);
-                        const uint32_t written = mk[i].lg_w - k + 1;
-                        total_ctr += plan_merkle_narrow(specs[i], &written, a);
-                    } else {
-                        a = merkle_level_args(mk[i], mk[i].lg_w - k);  // the level written (0: the caps)
-                    }
-                    a.tile_begin = l.blocks;
-                    l.blocks += l.narrow ? a.count >> a.tile_log
-                                         : (a.count + kMerkleLevelLanes - 1) / kMerkleLevelLanes;
-                    l.list.push_back(a);
+    for (int ht : {kPoseidon, kKeccak, kPoseidonBN128, kPoseidon2, kMonolith}) {
+        // mk[i].lg_w is the log2 width of tree i's leaf level per subtree
+        // (0: caps == leaves, no levels)
+        auto apart = [&](size_t i, uint32_t k) {
+            return (int)jobs[i].hash_type == ht && by_level[i] && mk[i].lg_w >= k;
+        };
+        for (uint32_t k = 1;; k++) {
+            LevelLaunch l{ht, false, {}, {}};
+            uint64_t children = 0;
+            for (size_t i = 0; i < n; i++)
+                if (apart(i, k)) children += specs[i].num_caps << (mk[i].lg_w - k + 1);
+            if (!children) break;
+            l.narrow = (has_narrow_kernel((uint64_t)ht) || has_tile_top((uint64_t)ht)) && children <= kNarrowNodes;
+            for (size_t i = 0; i < n; i++) {
+                if (!apart(i, k)) continue;
+                MerkleArgs a;
+                if (l.narrow) {
+                    l.first_ctr.push_back(total_ctr);
+                    const uint32_t written = mk[i].lg_w - k + 1;
+                    total_ctr += plan_merkle_narrow(specs[i], &written, a);
+                } else {
+                    a = merkle_level_args(mk[i], mk[i].lg_w - k);  // the level written (0: the caps)
                 }
-                const bool last = l.narrow;
-                levels.push_back(std::move(l));
-                if (last) break;
+                a.tile_begin = l.blocks;
+                l.blocks += l.narrow ? a.count >> a.tile_log
+                                     : (a.count + kMerkleLevelLanes - 1) / kMerkleLevelLanes;
+                l.list.push_back(a);
             }
+            const bool last = l.narrow;
+            levels.push_back(std::move(l));
+            if (last) break;
         }
+    }
     // arrival counters of the fused upper Merkle passes: zero between launches
     if (ctr_.bytes < total_ctr * sizeof(uint32_t)) {
         sync();
@@ -297,11 +300,11 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
             std::vector<MerkleArgs> list;
             uint64_t blocks = 0;
             for (size_t i = 0; i < n; i++) {
-                if ((int)jobs[i].hash_type != ht || narrow != narrow_trees(jobs[i].hash_type)) continue;
+                if ((int)jobs[i].hash_type != ht || narrow != (narrow_tree[i] != 0)) continue;
                 if (!narrow && tun[i].merkle_tile_log != tl) continue;
                 MerkleArgs a = mk[i];
                 a.tile_begin = blocks;
-                a.ctr = by_level((uint64_t)ht) ? nullptr : ctr_.as<uint32_t>() + mk_ctr[i];
+                a.ctr = by_level[i] ? nullptr : ctr_.as<uint32_t>() + mk_ctr[i];
                 blocks += a.count >> a.tile_log;
                 list.push_back(a);
             }
@@ -394,7 +397,7 @@ void Engine::issue(hipStream_t s, const std::vector<Launch> &launches, const Lau
                                l.blocks, l.tile_log, pieces.merkle_groups);
         } else if (l.kind == 3) {
             launch_merkle_narrow(s, l.hash, reinterpret_cast<const MerkleArgs *>(base), l.count, MerkleArgs{}, l.blocks,
-                                 l.tile_log ? "merkle_leaves" : "merkle_levels", pieces.merkle_groups);
+                                 l.tile_log ? "merkle_narrow" : "merkle_levels", pieces.merkle_groups);
         } else {
             launch_merkle_level(s, l.hash, reinterpret_cast<const MerkleArgs *>(base), l.count, l.blocks,
                                 pieces.merkle_groups);

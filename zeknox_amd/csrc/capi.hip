@@ -407,6 +407,7 @@ RustError zkx_set_tuning(size_t device_id, const ZkxCommitJob *job, const ZkxTun
         v.merkle_tile_log = t->merkle_tile_log;
         v.merkle_valu = t->merkle_valu;
         if (!valid_tuning(v)) invalid("schedule parameters out of range");
+        v.by_caller = true;
         Device &d = device(device_id);
         std::lock_guard<std::mutex> g(d.tune_mu);
         if (job) {
@@ -521,13 +522,13 @@ RustError zkx_tuning_save(size_t device_id, const char *path)
         std::lock_guard<std::mutex> g(d.tune_mu);
         FILE *f = fopen(path, "w");
         if (!f) invalid(std::string("cannot open ") + path);
-        fprintf(f, "# cols lg_n rate hash leaves : ntt_strided_max ntt_even merkle_tile_log merkle_valu\n");
+        fprintf(f, "# cols lg_n rate hash leaves : ntt_strided_max ntt_even merkle_tile_log merkle_valu set\n");
         for (const auto &kv : d.tuned) {
             const TuneKey &k = kv.first;
             const Tuning &t = kv.second;
-            fprintf(f, "%u %u %u %u %d : %u %u %u %u\n", std::get<0>(k), std::get<1>(k), std::get<2>(k),
+            fprintf(f, "%u %u %u %u %d : %u %u %u %u %d\n", std::get<0>(k), std::get<1>(k), std::get<2>(k),
                     std::get<3>(k), (int)std::get<4>(k), t.ntt_strided_max, t.ntt_even, t.merkle_tile_log,
-                    t.merkle_valu);
+                    t.merkle_valu, (int)t.by_caller);
         }
         const bool ok = fclose(f) == 0;
         if (!ok) invalid(std::string("cannot write ") + path);
@@ -549,10 +550,11 @@ RustError zkx_tuning_load(size_t device_id, const char *path)
             lineno++;
             if (line[0] == '#' || line[0] == '\n') continue;
             unsigned c, n, r, h, s, e, t, mv = 0;
-            int lv;
-            // the merkle_valu column is optional (tables written before it existed)
-            const int got = sscanf(line, "%u %u %u %u %d : %u %u %u %u", &c, &n, &r, &h, &lv, &s, &e, &t, &mv);
-            if (got != 8 && got != 9) {
+            int lv, set = 0;
+            // the last two columns are optional (tables written before they existed)
+            const int got =
+                sscanf(line, "%u %u %u %u %d : %u %u %u %u %d", &c, &n, &r, &h, &lv, &s, &e, &t, &mv, &set);
+            if (got < 8) {
                 bad = true;
                 break;
             }
@@ -561,6 +563,7 @@ RustError zkx_tuning_load(size_t device_id, const char *path)
             v.ntt_even = e;
             v.merkle_tile_log = t;
             v.merkle_valu = mv;
+            v.by_caller = set != 0;
             if (!valid_tuning(v)) {
                 bad = true;
                 break;

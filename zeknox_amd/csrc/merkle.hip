@@ -212,7 +212,7 @@ void build_narrow(Device &d, const MerkleSpec &s, const uint32_t *written, const
         return;
     }
     launch_merkle_narrow(d.stream, (int)s.hash_type, nullptr, 0, f, f.count >> f.tile_log,
-                         f.leaves ? "merkle_leaves" : "merkle_levels");
+                         f.leaves ? "merkle_narrow" : "merkle_levels");
 }
 
 }  // namespace
@@ -229,7 +229,7 @@ void merkle_build(Device &d, const MerkleSpec &s, const MerkleScratch &scratch)
     MerkleArgs passes[kMerkleMaxPasses];
     const uint32_t np = plan_merkle(sv, passes, tl);
     const bool narrow = has_narrow_kernel(s.hash_type);
-    if (narrow && s.num_leaves <= kNarrowLeaves) {
+    if (narrow && !tun.by_caller && s.num_leaves <= kNarrowLeaves) {
         build_narrow(d, s, nullptr, scratch);
         return;
     }

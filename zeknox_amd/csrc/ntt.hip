@@ -199,7 +199,7 @@ uint64_t plan_dif(std::vector<NttPass> &out, uint64_t *buf, uint64_t nblk, uint3
     // 2.01 -> 1.86 ms against a strided and a contiguous pass.  At 2^14, one
     // work-group per CU, nothing overlaps its loads and the two passes are as
     // fast (3.70 against 3.72 ms).
-    const bool whole = mode0 == kSrcLde && !inverse && L == kNttTileLog + 1;
+    const bool whole = mode0 == kSrcLde && !inverse && L == kNttTileLog + 1 && !tun.by_caller;
     const uint32_t tile_log = whole ? L : (uint32_t)kNttTileLog;
     const uint64_t tiles = (total + (1ull << tile_log) - 1) >> tile_log;
     const std::vector<uint32_t> sizes = whole ? std::vector<uint32_t>{L} : ntt_pass_sizes(L, tun);
@@ -282,6 +282,10 @@ const uint64_t *lde_factor_table(Device &d, uint32_t lg_n, uint32_t rate, bool i
 }
 
 namespace {
+
+// Whether the caller's default schedule says how stages L are cut into passes
+// (up to 2^12 they are one pass under any).
+bool callers_passes(Device &d, uint32_t L) { return L > (uint32_t)kNttTileLog && d.tuning_default().by_caller; }
 
 // A whole transform into natural order in one launch, where there is one:
 // cols blocks-of-2^rate columns of 2^(L + rate), read through `mode`.
@@ -392,11 +396,12 @@ void lde(Device &d, uint64_t *out, const uint64_t *in, uint32_t lg_n, uint32_t r
     const uint32_t lg = lg_n + rate;
     if (with_coset && inverse && (!d.coset || d.coset_lg < lg))
         invalid("coset table not initialised for log size " + std::to_string(lg));
-    if (column_tile_log(lg_n, lg, cols) &&
+    const bool passes = callers_passes(d, lg_n);
+    if (!passes && column_tile_log(lg_n, lg, cols) &&
         columns(d, out, lg_n, rate, cols, inverse, kSrcLde, in, lde_factor_table(d, lg_n, rate, inverse, with_coset),
                 (inverse && with_coset) ? d.coset : nullptr))
         return;
-    if (two_launch_chunk(lg_n, lg, cols) &&
+    if (!passes && two_launch_chunk(lg_n, lg, cols) &&
         two_launches(d, out, lg_n, rate, cols, inverse, kSrcLde, in, lde_factor_table(d, lg_n, rate, inverse, with_coset),
                      (inverse && with_coset) ? d.coset : nullptr))
         return;
@@ -413,8 +418,10 @@ void ntt(Device &d, uint64_t *inout, uint32_t lg, uint32_t cols, bool inverse, b
         invalid("coset table not initialised for log size " + std::to_string(lg));
     const uint32_t mode = (with_coset && !inverse) ? kSrcCoset : kSrcInPlace;
     const uint64_t *after = (inverse && with_coset) ? d.coset : nullptr;
-    if (columns(d, inout, lg, 0, cols, inverse, mode, nullptr, d.coset, after)) return;
-    if (two_launches(d, inout, lg, 0, cols, inverse, mode, inout, d.coset, after)) return;
+    if (!callers_passes(d, lg)) {
+        if (columns(d, inout, lg, 0, cols, inverse, mode, nullptr, d.coset, after)) return;
+        if (two_launches(d, inout, lg, 0, cols, inverse, mode, inout, d.coset, after)) return;
+    }
     const uint64_t *tw = d.twiddle_table(lg);
     run_dif(d, inout, cols, lg, lg, tw, inverse, mode, nullptr, 0, false, d.coset);
     bitrev_columns(d, inout, lg, cols, inverse, inverse ? host_inv((1ull << lg) % 0xFFFFFFFF00000001ull) : 1,

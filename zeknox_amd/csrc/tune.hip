@@ -68,6 +68,7 @@ Tuning autotune(Engine &e, const CommitJob &job, int iters)
     const size_t copies = lg_rows >= 20 ? 1 : std::min<size_t>(64, (size_t)1 << (20 - lg_rows));
     const std::vector<CommitJob> batch(copies, job);
     Tuning best = d.tuning_default();
+    best.by_caller = false;
     // warm-up: builds the tables the shape needs and sizes the engine's scratch
     e.commit(batch.data(), batch.size(), nullptr, &best);
     double best_ms = time_commit(e, batch, best, iters, tm);

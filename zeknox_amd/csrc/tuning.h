@@ -21,6 +21,12 @@ struct Tuning {
     // Merkle, Poseidon leaves: 0 = the MDS layers of whole-wave leaf
     // permutations on the i8 matrix cores; 1 = every permutation on the VALU.
     uint32_t merkle_valu = 0;
+    // Set by the caller (zkx_set_tuning): the schedule runs as it stands.
+    // Otherwise (built-in default, autotuner) small Poseidon and Poseidon2
+    // forests are built by the 16-permutations-per-wave kernel and transforms
+    // of 2^13 to 2^20 in one or two launches where that is faster, and the
+    // schedule is that of what is left to passes and tiles.
+    bool by_caller = false;
 };
 
 // Work-group size (log2 lanes) of the C-ABI Merkle entry points for one tree
