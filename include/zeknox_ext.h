@@ -178,16 +178,17 @@ RustError zkx_set_commit_graphs(size_t device_id, int on);
  * Poseidon and Poseidon2 from an eighth of it) hashes the leaves in one launch
  * per hash kind and builds the levels above them in launches of their own over
  * every tree: one per level, Poseidon's and Poseidon2's narrow levels together
- * in one.  Smaller batches, and Poseidon and Poseidon2 forests of at most 2^15
- * leaves in any batch, finish every tree inside the leaf launch.  0: always
- * apart; UINT64_MAX: never.  No setting changes a result. */
+ * in one.  Smaller batches finish every tree inside the leaf launch, and so do
+ * in any batch the Poseidon forests, or the Poseidon2 forests, of together at
+ * most 2^15 leaves and fewer than min_leaves / 4.  0: always apart;
+ * UINT64_MAX: never.  No setting changes a result. */
 RustError zkx_set_level_launches(size_t device_id, uint64_t min_leaves);
 /* The same for one tree through fill_digests_buf_linear_gpu_with_gpu_ptr and
  * the other C-ABI Merkle entry points, the allocation-free one included:
- * Poseidon, Poseidon2 and Poseidon-BN128 trees of at least min_leaves / 32
- * leaves (default 2^20 / 32), Keccak-256 and Monolith trees of at least
- * min_leaves / 4.  0: always apart; UINT64_MAX: never.  No setting changes a
- * result. */
+ * Poseidon and Poseidon2 trees of at least min_leaves / 16 leaves (default
+ * 2^20 / 16), Poseidon-BN128 trees of at least min_leaves / 32, Keccak-256 and
+ * Monolith trees of at least min_leaves / 4.  0: always apart; UINT64_MAX:
+ * never.  No setting changes a result. */
 RustError zkx_set_lone_level_launches(size_t device_id, uint64_t min_leaves);
 /* Graphs the device's zkx_commit_batch engine holds (tests, benchmarks). */
 size_t zkx_commit_graphs_captured(size_t device_id);

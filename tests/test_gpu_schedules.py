@@ -96,6 +96,37 @@ def test_lone_tree_under_a_set_default(zk, ht, tile, valu):
             zk.set_tuning(zk.Tuning(merkle_tile_log=tile, merkle_valu=valu))
 
 
+@pytest.mark.parametrize("ht", [0, 3])
+@pytest.mark.parametrize("lg,cap", [(11, 2), (6, 6), (3, 0), (15, 4)])
+def test_zero_takes_small_levels_apart(zk, ht, lg, cap):
+    leaves = ob.canonical(7 << lg, 31 + lg)
+    want = ob.merkle(leaves, 7, cap, ht)
+    apart = {"merkle_leaves": 1, "merkle_levels": 1} if cap < lg else {"merkle_leaves": 1}
+    for least, seen in ((0, apart), (None, {"merkle_narrow": 1}), (zk.LONE_LEVEL_LAUNCHES_DEFAULT, {"merkle_narrow": 1})):
+        zk.set_lone_level_launches(least)
+        zk.set_level_launches(zk.LEVEL_LAUNCHES_DEFAULT if least else least)
+        out = []
+        assert launches(zk, lambda: out.extend(zk.merkle_tree(leaves, 7, cap, ht))) == seen
+        assert np.array_equal(out[0], want[0]) and np.array_equal(out[1], want[1])
+        j = Job(zk, 7, lg - 1, 1, cap, ht)
+        got = launches(zk, lambda: zk.commit_batch([j.commit]))
+        assert {k: v for k, v in got.items() if k.startswith("merkle")} == seen
+        j.check()
+
+
+@pytest.mark.parametrize("ht", [0, 3])
+def test_switch_of_a_lone_tree(zk, ht):
+    """2^16 leaves, the smallest whose levels are apart by default."""
+    leaves = ob.canonical(9 << 16, 16)
+    want = ob.merkle(leaves, 9, 4, ht)
+    for least, levels in ((zk.LONE_LEVEL_LAUNCHES_DEFAULT, 1), (None, 0), (0, 1)):
+        zk.set_lone_level_launches(least)
+        out = []
+        got = launches(zk, lambda: out.extend(zk.merkle_tree(leaves, 9, 4, ht)))
+        assert got["merkle_leaves"] == 1 and got.get("merkle_levels", 0) == levels
+        assert np.array_equal(out[0], want[0]) and np.array_equal(out[1], want[1])
+
+
 @pytest.mark.parametrize("strided,even", [(9, 0), (4, 1), (1, 0)])
 def test_transforms_under_a_set_schedule(zk, strided, even):
     t = zk.Tuning(strided, even)

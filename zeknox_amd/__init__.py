@@ -474,8 +474,9 @@ LEVEL_LAUNCHES_DEFAULT = 1 << 18
 
 def set_level_launches(min_leaves, device_id=0):
     """Batches whose trees hold at least min_leaves leaves (an eighth of it for
-    Poseidon and Poseidon2) build the tree levels in launches of their own
-    (0: always, None: never)."""
+    Poseidon and Poseidon2, but not for one's forests of together at most 2^15
+    leaves and fewer than min_leaves / 4) build the tree levels in launches of
+    their own (0: always, None: never)."""
     v = (1 << 64) - 1 if min_leaves is None else int(min_leaves)
     _check(lib.zkx_set_level_launches(device_id, v))
 
@@ -485,8 +486,9 @@ LONE_LEVEL_LAUNCHES_DEFAULT = 1 << 20
 
 def set_lone_level_launches(min_leaves, device_id=0):
     """One tree through the C-ABI Merkle entry points builds its levels in
-    launches of their own from min_leaves / 4 leaves for Keccak-256 and
-    Monolith, min_leaves / 32 for the others (0: always, None: never)."""
+    launches of their own from min_leaves / 16 leaves for Poseidon and
+    Poseidon2, min_leaves / 4 for Keccak-256 and Monolith, min_leaves / 32 for
+    Poseidon-BN128 (0: always, None: never)."""
     v = (1 << 64) - 1 if min_leaves is None else int(min_leaves)
     _check(lib.zkx_set_lone_level_launches(device_id, v))
 

@@ -157,7 +157,7 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
     std::vector<char> narrow_tree(n), by_level(n);
     for (size_t i = 0; i < n; i++) {
         const uint64_t ht = jobs[i].hash_type;
-        narrow_tree[i] = has_narrow_kernel(ht) && !tun[i].by_caller && hash_leaves[ht] <= kNarrowLeaves;
+        narrow_tree[i] = !tun[i].by_caller && batch_narrow(hash_leaves[ht], ht, apart_from);
         by_level[i] = !narrow_tree[i] && batch_levels_apart(tree_leaves, ht, apart_from);
     }
 

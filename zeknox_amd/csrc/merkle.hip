@@ -228,19 +228,19 @@ void merkle_build(Device &d, const MerkleSpec &s, const MerkleScratch &scratch)
     sv.leaf_valu = tun.merkle_valu;
     MerkleArgs passes[kMerkleMaxPasses];
     const uint32_t np = plan_merkle(sv, passes, tl);
-    const bool narrow = has_narrow_kernel(s.hash_type);
-    if (narrow && !tun.by_caller && s.num_leaves <= kNarrowLeaves) {
+    const uint64_t apart_from = d.lone_level_leaves.load();
+    if (!tun.by_caller && lone_tree_narrow(s.num_leaves, s.hash_type, apart_from)) {
         build_narrow(d, s, nullptr, scratch);
         return;
     }
-    if (s.num_caps < s.num_leaves && lone_tree_levels_apart(s.num_leaves, s.hash_type, d.lone_level_leaves.load())) {
+    if (s.num_caps < s.num_leaves && lone_tree_levels_apart(s.num_leaves, s.hash_type, apart_from)) {
         // a large tree: the leaf digests in one launch, then one launch per
         // level (k_merkle_level), each level's descriptor passed by value
         MerkleArgs leaf = passes[0];
         leaf.leaves_only = 1;
         launch_merkle_pass(d.stream, (int)s.hash_type, nullptr, 0, leaf, leaf.count >> leaf.tile_log, tl);
         for (uint32_t w = leaf.lg_w; w-- > 0;) {
-            if ((narrow || has_tile_top(s.hash_type)) && s.num_caps << (w + 1) <= kNarrowNodes) {
+            if ((has_narrow_kernel(s.hash_type) || has_tile_top(s.hash_type)) && s.num_caps << (w + 1) <= kNarrowNodes) {
                 const uint32_t written = w + 1;
                 build_narrow(d, s, &written, scratch);
                 break;

@@ -83,7 +83,7 @@ constexpr bool has_tile_top(uint64_t hash_type) { return hash_type == 1; }
 // with one launch per level (after a leaf-digests-only launch; Poseidon and
 // Poseidon2 finish with one launch of the 16-per-wave kernel) rather than
 // inside its leaf launch, given the device threshold `min_leaves` (default
-// 2^20): Poseidon and Poseidon2 trees switch at min_leaves / 32, Keccak-256
+// 2^20): Poseidon and Poseidon2 trees switch at min_leaves / 16, Keccak-256
 // and Monolith at min_leaves / 4, Poseidon-BN128 at min_leaves / 32 (0:
 // always).  Measured, fused against apart, 135-element leaves, cap 4, ms:
 //   leaves  Poseidon      Poseidon2     Keccak-256     Monolith       Poseidon-BN128
@@ -104,8 +104,15 @@ constexpr bool has_tile_top(uint64_t hash_type) { return hash_type == 1; }
 // pays at every size measured.
 inline bool lone_tree_levels_apart(uint64_t num_leaves, uint64_t hash_type, uint64_t min_leaves)
 {
-    const uint32_t shift = hash_type == 1 || hash_type == 4 ? 2 : 5;
+    const uint32_t shift = hash_type == 2 ? 5 : has_narrow_kernel(hash_type) ? 4 : 2;
     return num_leaves >= (min_leaves >> shift);
+}
+// Whether the 16-per-wave kernel builds it whole: up to kNarrowLeaves, and
+// below the line above.
+inline bool lone_tree_narrow(uint64_t num_leaves, uint64_t hash_type, uint64_t min_leaves)
+{
+    return has_narrow_kernel(hash_type) && num_leaves <= kNarrowLeaves &&
+           !lone_tree_levels_apart(num_leaves, hash_type, min_leaves);
 }
 // The same for the forests of one hash in a batch of `batch_leaves` leaves in
 // total (default threshold 2^18; Poseidon and Poseidon2 at an eighth).
@@ -115,6 +122,13 @@ inline bool lone_tree_levels_apart(uint64_t num_leaves, uint64_t hash_type, uint
 inline bool batch_levels_apart(uint64_t batch_leaves, uint64_t hash_type, uint64_t min_leaves)
 {
     return batch_leaves > 0 && batch_leaves >= (has_narrow_kernel(hash_type) ? min_leaves >> 3 : min_leaves);
+}
+// Whether the 16-per-wave kernel builds a hash's forests of a batch
+// (hash_leaves in all) whole: up to kNarrowLeaves, and below a quarter of
+// min_leaves, which is above them by default.
+inline bool batch_narrow(uint64_t hash_leaves, uint64_t hash_type, uint64_t min_leaves)
+{
+    return has_narrow_kernel(hash_type) && hash_leaves <= kNarrowLeaves && hash_leaves < (min_leaves >> 2);
 }
 
 }  // namespace zkx
