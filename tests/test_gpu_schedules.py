@@ -127,6 +127,20 @@ def test_switch_of_a_lone_tree(zk, ht):
         assert np.array_equal(out[0], want[0]) and np.array_equal(out[1], want[1])
 
 
+def test_keccak_tops_are_timed_as_levels(zk):
+    """2^18 and 2^17 children in a launch each, the rest on tiles of 256."""
+    leaves = ob.canonical(3 << 18, 18)
+    want = ob.merkle(leaves, 3, 1, zk.HASH_KECCAK)
+    out = []
+    got = launches(zk, lambda: out.extend(zk.merkle_tree(leaves, 3, 1, zk.HASH_KECCAK)))
+    assert got == {"merkle_leaves": 1, "merkle_levels": 3}
+    assert np.array_equal(out[0], want[0]) and np.array_equal(out[1], want[1])
+    j = Job(zk, 3, 17, 1, 1, zk.HASH_KECCAK)
+    got = launches(zk, lambda: zk.commit_batch([j.commit]))
+    assert (got["merkle_leaves"], got["merkle_levels"]) == (1, 3)
+    j.check()
+
+
 @pytest.mark.parametrize("strided,even", [(9, 0), (4, 1), (1, 0)])
 def test_transforms_under_a_set_schedule(zk, strided, even):
     t = zk.Tuning(strided, even)

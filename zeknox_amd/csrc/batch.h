@@ -98,6 +98,7 @@ private:
         int hash;           // NTT: contiguous; Merkle: hash type
         int kernel;         // NTT: ntt_kernel_kind of the list
         uint32_t tile_log;  // Merkle work-group size (log2 lanes)
+        bool top = false;   // Merkle: what lies above a written level
     };
     void issue(hipStream_t s, const std::vector<Launch> &launches, const LaunchPieces &pieces);
     void drop_graphs();

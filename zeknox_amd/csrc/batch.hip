@@ -318,7 +318,7 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
         const size_t off = push(l.list.data(), l.list.size() * sizeof(MerkleArgs));
         const bool tiles = l.narrow && has_tile_top((uint64_t)l.hash);
         launches.push_back({off, (uint32_t)l.list.size(), l.blocks, tiles ? 1 : l.narrow ? 3 : 2, l.hash, 0,
-                            tiles ? (uint32_t)kMerkleMinTileLog : 0});
+                            tiles ? (uint32_t)kMerkleMinTileLog : 0, tiles});
         host.resize(align_up(host.size()));
     }
     size_t off0 = 0;
@@ -394,7 +394,8 @@ void Engine::issue(hipStream_t s, const std::vector<Launch> &launches, const Lau
                             "batch_ntt", pieces.ntt_tiles);
         } else if (l.kind == 1) {
             launch_merkle_pass(s, l.hash, reinterpret_cast<const MerkleArgs *>(base), l.count, MerkleArgs{},
-                               l.blocks, l.tile_log, pieces.merkle_groups);
+                               l.blocks, l.tile_log, pieces.merkle_groups,
+                               l.top ? "merkle_levels" : "merkle_leaves");
         } else if (l.kind == 3) {
             launch_merkle_narrow(s, l.hash, reinterpret_cast<const MerkleArgs *>(base), l.count, MerkleArgs{}, l.blocks,
                                  l.tile_log ? "merkle_narrow" : "merkle_levels", pieces.merkle_groups);

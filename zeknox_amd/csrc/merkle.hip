@@ -116,13 +116,14 @@ uint64_t fuse_merkle_passes(const std::vector<MerkleArgs> &passes, MerkleArgs &o
 }
 
 void launch_merkle_pass(hipStream_t stream, int hash_type, const MerkleArgs *dev_list,
-                        uint32_t n, const MerkleArgs &one, uint64_t blocks, uint32_t tile_log_max, uint64_t chunk)
+                        uint32_t n, const MerkleArgs &one, uint64_t blocks, uint32_t tile_log_max, uint64_t chunk,
+                        const char *name)
 {
     if (blocks == 0) return;
     if (blocks > 0x7FFFFFFFull) invalid("tree too large for one launch");
     if (tile_log_max < (uint32_t)kMerkleMinTileLog || tile_log_max > (uint32_t)kMerkleMaxTileLog)
         invalid("Merkle tile size out of range");
-    ProfScope ps("merkle_leaves", stream);
+    ProfScope ps(name, stream);
     const uint64_t step = (chunk && n > 0) ? chunk : blocks;
     for (uint64_t b0 = 0; b0 < blocks; b0 += step) {
         const uint64_t nb = std::min(step, blocks - b0);
@@ -208,7 +209,8 @@ void build_narrow(Device &d, const MerkleSpec &s, const uint32_t *written, const
     if (nctr) f.ctr = scratch.counters(d, nctr);
     if (has_tile_top(s.hash_type)) {
         const MerkleArgs *dj = scratch.descriptor(d, f);
-        launch_merkle_pass(d.stream, (int)s.hash_type, dj, 1, MerkleArgs{}, f.count >> f.tile_log, kMerkleMinTileLog);
+        launch_merkle_pass(d.stream, (int)s.hash_type, dj, 1, MerkleArgs{}, f.count >> f.tile_log, kMerkleMinTileLog, 0,
+                           "merkle_levels");
         return;
     }
     launch_merkle_narrow(d.stream, (int)s.hash_type, nullptr, 0, f, f.count >> f.tile_log,
