@@ -159,6 +159,27 @@ def test_transforms_under_a_set_schedule(zk, strided, even):
         assert np.array_equal(out, ob.ntt(x, lg_n, B, False, True) if rate == 0 else ob.lde(x, lg_n, rate, B))
 
 
+@pytest.mark.parametrize("lg_n,rate,ht,candidates", [(13, 1, 1, 2),   # one pass split, two more work-group sizes
+                                                     (6, 2, 0, 0),    # and no Merkle schedule
+                                                     (8, 1, 3, 0),
+                                                     (8, 2, 0, 3),    # 64 copies are above 2^15 leaves
+                                                     (14, 1, 1, None)])
+def test_the_tuner_times_each_plan_once(zk, lg_n, rate, ht, candidates):
+    j = Job(zk, 5, lg_n, rate, 1, ht)
+    if candidates is None:  # every split that differs, and the work-group sizes
+        plans = {tuple(zk.ntt_pass_sizes(lg_n, zk.Tuning(s, e))) for s in range(4, 10) for e in (0, 1)}
+        candidates = len(plans) - 1 + 2
+    got = launches(zk, lambda: zk.autotune([j.commit], iters=2))
+    # the warm-up, then two runs of the default and of each candidate
+    assert sum(v for k, v in got.items() if k in ("merkle_leaves", "merkle_narrow")) == 1 + 2 * (1 + candidates)
+    t = zk.get_tuning(j.commit).astuple()
+    if lg_n == 13:
+        assert t[:2] == (9, 0)
+    if not candidates:
+        assert t[2:] == (8, 0)
+    j.check()
+
+
 def test_a_set_schedule_is_saved_as_one(zk, tmp_path):
     j = Job(zk, 4, 8, 2, 1, zk.HASH_POSEIDON)
     zk.set_tuning(zk.Tuning(merkle_tile_log=9), j.commit)

@@ -40,6 +40,9 @@ uint64_t plan_dif(std::vector<NttPass> &out, uint64_t *buf, uint64_t nblk, uint3
 // Stage counts of the DIF passes over blocks of 2^L under `tun`, top
 // stages first (the last pass contiguous).
 std::vector<uint32_t> ntt_pass_sizes(uint32_t L, const Tuning &tun);
+// The same for the forward LDE from coefficients (plan_dif with kSrcLde),
+// which has one-launch blocks of 2^13 unless the caller set the schedule.
+std::vector<uint32_t> lde_pass_sizes(uint32_t L, const Tuning &tun);
 
 // Which register-round kernel a launch over these passes can use (each runs
 // one tile per work-group): 0 none (k_ntt_tiles); 1 contiguous (every pass

@@ -188,21 +188,26 @@ std::vector<uint32_t> ntt_pass_sizes(uint32_t L, const Tuning &tun)
     return sizes;
 }
 
+// An LDE of 2^13-word blocks fits the one-launch kernel (ntt_columns.h) with
+// two work-groups per CU: 8 commits of 135 x 2^13 rate 3, Keccak-256, 2.01 ->
+// 1.86 ms against a strided and a contiguous pass.  At 2^14, one work-group per
+// CU, nothing overlaps its loads and the two passes are as fast (3.70 against
+// 3.72 ms).
+std::vector<uint32_t> lde_pass_sizes(uint32_t L, const Tuning &tun)
+{
+    if (L == (uint32_t)kNttTileLog + 1 && !tun.by_caller) return {L};
+    return ntt_pass_sizes(L, tun);
+}
+
 uint64_t plan_dif(std::vector<NttPass> &out, uint64_t *buf, uint64_t nblk, uint32_t L, uint32_t lg_tw,
                   const uint64_t *tw, const uint64_t *tw12, const uint64_t *const *tw_lg, bool inverse,
                   uint32_t mode0, const uint64_t *src, uint32_t rate, bool with_coset, const uint64_t *coset,
                   const Tuning &tun)
 {
     const uint64_t total = nblk << L;
-    // an LDE of 2^13-word blocks fits the one-launch kernel (ntt_columns.h)
-    // with two work-groups per CU: 8 commits of 135 x 2^13 rate 3, Keccak-256,
-    // 2.01 -> 1.86 ms against a strided and a contiguous pass.  At 2^14, one
-    // work-group per CU, nothing overlaps its loads and the two passes are as
-    // fast (3.70 against 3.72 ms).
-    const bool whole = mode0 == kSrcLde && !inverse && L == kNttTileLog + 1 && !tun.by_caller;
-    const uint32_t tile_log = whole ? L : (uint32_t)kNttTileLog;
+    const std::vector<uint32_t> sizes = mode0 == kSrcLde && !inverse ? lde_pass_sizes(L, tun) : ntt_pass_sizes(L, tun);
+    const uint32_t tile_log = std::max<uint32_t>(sizes.back(), kNttTileLog);
     const uint64_t tiles = (total + (1ull << tile_log) - 1) >> tile_log;
-    const std::vector<uint32_t> sizes = whole ? std::vector<uint32_t>{L} : ntt_pass_sizes(L, tun);
     uint32_t hi = L;  // stages [0, hi) not yet planned
     for (size_t k = 0; k < sizes.size(); k++) {
         NttPass a{};

@@ -74,13 +74,13 @@ Tuning autotune(Engine &e, const CommitJob &job, int iters)
     double best_ms = time_commit(e, batch, best, iters, tm);
 
     // NTT pass split over the coefficient blocks (2^lg_n points)
-    std::vector<std::vector<uint32_t>> seen{ntt_pass_sizes(job.lg_n, best)};
+    std::vector<std::vector<uint32_t>> seen{lde_pass_sizes(job.lg_n, best)};
     for (uint32_t even = 0; even <= 1; even++)
         for (uint32_t smax = 9; smax >= 4; smax--) {
             Tuning c = best;
             c.ntt_strided_max = smax;
             c.ntt_even = even;
-            const std::vector<uint32_t> plan = ntt_pass_sizes(job.lg_n, c);
+            const std::vector<uint32_t> plan = lde_pass_sizes(job.lg_n, c);
             if (std::find(seen.begin(), seen.end(), plan) != seen.end()) continue;
             seen.push_back(plan);
             const double ms = time_commit(e, batch, c, iters, tm);
@@ -90,10 +90,13 @@ Tuning autotune(Engine &e, const CommitJob &job, int iters)
             }
         }
 
-    // Merkle work-group size (all sizes give one tile when the tree is small)
+    // Merkle work-group size (all sizes give one tile when the tree is small).
+    // Forests that the 16-per-wave kernel builds whole have no Merkle schedule,
+    // and 64 copies of the smallest shapes are such a forest: the default stays.
     const uint32_t lg_leaves = job.lg_n + job.rate;
+    const bool tiles = !batch_narrow(copies << lg_leaves, job.hash_type, d.level_launch_leaves.load());
     const Tuning ntt_best = best;
-    for (uint32_t tl = kMerkleMinTileLog; tl <= (uint32_t)kMerkleMaxTileLog; tl++) {
+    for (uint32_t tl = kMerkleMinTileLog; tiles && tl <= (uint32_t)kMerkleMaxTileLog; tl++) {
         if (tl == ntt_best.merkle_tile_log || (tl > lg_leaves && ntt_best.merkle_tile_log >= lg_leaves)) continue;
         Tuning c = ntt_best;
         c.merkle_tile_log = tl;
@@ -105,7 +108,7 @@ Tuning autotune(Engine &e, const CommitJob &job, int iters)
     }
 
     // Poseidon leaves: MDS layers on the matrix cores or all-VALU permutations
-    if (job.hash_type == kPoseidon && job.cols > 4) {
+    if (tiles && job.hash_type == kPoseidon && job.cols > 4) {
         Tuning c = best;
         c.merkle_valu = 1 - best.merkle_valu;
         const double ms = time_commit(e, batch, c, iters, tm);
