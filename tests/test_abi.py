@@ -123,3 +123,15 @@ def test_init_cuda_degree_reports_bad_degree():
     with pytest.raises(zk.ZeknoxError):
         zk.init_cuda_degree_rs(40)
     assert "max_degree" in zk.last_error()
+
+
+@pytest.mark.parametrize("ht", [0, 2, 3, 4])
+def test_leaf_sizes_whose_block_count_would_wrap_are_refused(ht):
+    """Sponges of eight elements a block step by eight in 32 bits; nothing is
+    read (the check is on the host, before any device)."""
+    import zeknox_amd as zk
+    buf = (ctypes.c_uint64 * 4)()
+    p = ctypes.addressof(buf)
+    for size in (2**32 - 7, 2**32 - 1, 2**32, 0):
+        with pytest.raises(zk.ZeknoxError, match="leaf size out of range"):
+            zk.fill_digests_buf_linear_gpu_with_gpu_ptr(p, p, p, 0, 1, 1, size, 0, ht, 0)

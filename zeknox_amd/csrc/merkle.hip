@@ -25,7 +25,10 @@ void check_merkle(const MerkleSpec &s)
     if (!s.caps || !s.leaves) invalid("null cap or leaf buffer");
     if (!is_pow2(s.num_leaves) || !is_pow2(s.num_caps) || s.num_caps > s.num_leaves)
         invalid("leaves and caps must be powers of two with caps <= leaves");
-    if (s.leaf_size == 0 || s.leaf_size > 0xFFFFFFFFull) invalid("leaf size out of range");
+    // (the sponges of eight elements a block count them in steps of eight in 32
+    // bits: beyond 2^32 - 8 the count would wrap and never end)
+    if (s.leaf_size == 0 || s.leaf_size > (s.hash_type == kKeccak ? 0xFFFFFFFFull : 0xFFFFFFF8ull))
+        invalid("leaf size out of range");
     if (s.num_caps == s.num_leaves) return;
     if ((1ull << s.cap_height) != s.num_caps) invalid("cap_buf_size must be 2^cap_height");
     if (s.num_digests != 2 * (s.num_leaves - s.num_caps))
