@@ -76,8 +76,6 @@ __device__ __forceinline__ uint64_t sub(uint64_t a, uint64_t b)
     return b2 ? pack(tlo, thi) : pack(dlo, dhi);
 }
 
-__device__ __forceinline__ uint64_t neg(uint64_t a) { return sub(0, a); }
-
 // h * EPS = h * 2^32 - h for h < 2^32 (exact, <= 2^64 - 2^33 + 1).
 __device__ __forceinline__ uint64_t mul_eps(uint32_t h)
 {
@@ -138,26 +136,13 @@ __device__ __forceinline__ uint64_t reduce96_lazy(uint64_t lo, uint32_t top)
     return r;
 }
 
-// 64x64 -> 128 product from five 32x32+64 multiply-adds (any a, b < 2^64).
-// The last one adds hi(t2) to t3 (t3 + hi(t2) <= 2^64 - 1), which keeps the
-// high word off the slow 64-bit adder.
-__device__ __forceinline__ void mul128(uint64_t a, uint64_t b, uint64_t &lo, uint64_t &hi)
-{
-    const uint32_t a0 = lo32(a), a1 = hi32(a), b0 = lo32(b), b1 = hi32(b);
-    const uint64_t t0 = (uint64_t)a0 * b0;
-    const uint64_t t1 = (uint64_t)a1 * b0 + hi32(t0);
-    const uint64_t t2 = (uint64_t)a0 * b1 + lo32(t1);
-    const uint64_t t3 = (uint64_t)a1 * b1 + hi32(t1);  // <= 2^64 - 2^32
-    hi = add_small(t3, hi32(t2));
-    lo = pack(lo32(t0), lo32(t2));
-}
-
 // 64x64 -> 128 product from four multiply-adds, the carry of the middle sum
 // left in a lane mask: a * b = lo + (hi + c * 2^32) * 2^64, c in {0, 1}
 // (any a, b < 2^64).  u = a0 b0; v = a0 b1 + hi(u) (< 2^64); w = a1 b0 + v,
 // whose bit 64 is c; hi = a1 b1 + hi(w) <= 2^64 - 2^32 (no carry).  Two
-// instructions fewer than mul128 (one multiply-add and one register-pair
-// copy): the carry goes into the reduction as a borrow (reduce128c_lazy).
+// instructions fewer than with the middle sum kept below 2^64 (a fifth
+// multiply-add and a register-pair copy): the carry goes into the reduction as
+// a borrow (reduce128c_lazy).
 __device__ __forceinline__ void mul128c(uint64_t a, uint64_t b, uint64_t &lo, uint64_t &hi, uint64_t &c)
 {
     const uint32_t a0 = lo32(a), a1 = hi32(a), b0 = lo32(b), b1 = hi32(b);
@@ -244,50 +229,10 @@ __device__ __forceinline__ uint64_t reduce128c_lazy(uint64_t lo, uint64_t hi, ui
     return pack(lo32(t), rhi);
 }
 
-// Two independent reduce128_lazy at once: the same instructions with the two
+// Two independent reduce128c_lazy at once: the same instructions with the two
 // reductions interleaved, so every lane-mask read already sits two
 // instructions after its write (one s_nop 0 per pair of steps instead of an
 // s_nop 1 per step).
-__device__ __forceinline__ void reduce128_lazy2(uint64_t lo0, uint64_t hi0, uint64_t lo1, uint64_t hi1, uint64_t &r0,
-                                                uint64_t &r1)
-{
-    uint64_t u0, u1, sc0, sc1;
-    uint32_t cv0, cv1;
-    asm("v_mad_u64_u32 %[u0], %[sc0], %[a0], -1, %[l0]\n\t"
-        "v_mad_u64_u32 %[u1], %[sc1], %[a1], -1, %[l1]\n\t"
-        "s_nop 0\n\t"
-        "v_cndmask_b32_e64 %[cv0], 0, 1, %[sc0]\n\t"
-        "v_cndmask_b32_e64 %[cv1], 0, 1, %[sc1]"
-        : [u0] "=&v"(u0), [u1] "=&v"(u1), [sc0] "=&s"(sc0), [sc1] "=&s"(sc1), [cv0] "=&v"(cv0), [cv1] "=&v"(cv1)
-        : [a0] "v"(lo32(hi0)), [l0] "v"(lo0), [a1] "v"(lo32(hi1)), [l1] "v"(lo1));
-    uint32_t zl0, zh0, cb0, zl1, zh1, cb1;
-    uint64_t b10, b0, j0, b11, b1, j1;
-    asm("v_sub_co_u32_e64 %[zl0], %[b10], %[ul0], %[h10]\n\t"
-        "v_sub_co_u32_e64 %[zl1], %[b11], %[ul1], %[h11]\n\t"
-        "s_nop 0\n\t"
-        "v_subb_co_u32_e64 %[zh0], %[b0], %[uh0], 0, %[b10]\n\t"
-        "v_subb_co_u32_e64 %[zh1], %[b1], %[uh1], 0, %[b11]\n\t"
-        "s_nop 0\n\t"
-        "v_subb_co_u32_e64 %[cb0], %[j0], %[cv0], 0, %[b0]\n\t"
-        "v_subb_co_u32_e64 %[cb1], %[j1], %[cv1], 0, %[b1]"
-        : [zl0] "=&v"(zl0), [zh0] "=&v"(zh0), [cb0] "=&v"(cb0), [zl1] "=&v"(zl1), [zh1] "=&v"(zh1),
-          [cb1] "=&v"(cb1), [b10] "=&s"(b10), [b0] "=&s"(b0), [j0] "=&s"(j0), [b11] "=&s"(b11), [b1] "=&s"(b1),
-          [j1] "=&s"(j1)
-        : [ul0] "v"(lo32(u0)), [uh0] "v"(hi32(u0)), [h10] "v"(hi32(hi0)), [cv0] "v"(cv0), [ul1] "v"(lo32(u1)),
-          [uh1] "v"(hi32(u1)), [h11] "v"(hi32(hi1)), [cv1] "v"(cv1));
-    uint64_t t0, t1, tj0, tj1;
-    asm("v_mad_i64_i32 %[t0], %[tj0], %[cb0], -1, %[z0]\n\t"
-        "v_mad_i64_i32 %[t1], %[tj1], %[cb1], -1, %[z1]"
-        : [t0] "=&v"(t0), [t1] "=&v"(t1), [tj0] "=&s"(tj0), [tj1] "=&s"(tj1)
-        : [cb0] "v"(cb0), [z0] "v"(pack(zl0, zh0)), [cb1] "v"(cb1), [z1] "v"(pack(zl1, zh1)));
-    uint32_t rh0, rh1;  // high-word adds kept in asm (see reduce128_lazy)
-    asm("v_add_u32 %[r], %[a], %[b]" : [r] "=v"(rh0) : [a] "v"(hi32(t0)), [b] "v"(cb0));
-    asm("v_add_u32 %[r], %[a], %[b]" : [r] "=v"(rh1) : [a] "v"(hi32(t1)), [b] "v"(cb1));
-    r0 = pack(lo32(t0), rh0);
-    r1 = pack(lo32(t1), rh1);
-}
-
-// reduce128_lazy2 with the borrows cin0, cin1 (reduce128c_lazy).
 __device__ __forceinline__ void reduce128c_lazy2(uint64_t lo0, uint64_t hi0, uint64_t cin0, uint64_t lo1, uint64_t hi1,
                                                  uint64_t cin1, uint64_t &r0, uint64_t &r1)
 {
@@ -345,16 +290,6 @@ __device__ __forceinline__ uint64_t mul_lazy(uint64_t a, uint64_t b)
     return reduce128c_lazy(lo, hi, c);
 }
 
-// mul_lazy through mul128 and reduce128_lazy: two instructions more, for
-// kernels where the carry form's schedule spills (its products' operands
-// and partial sums live longer).
-__device__ __forceinline__ uint64_t mul_lazy_nc(uint64_t a, uint64_t b)
-{
-    uint64_t lo, hi;
-    mul128(a, b, lo, hi);
-    return reduce128_lazy(lo, hi);
-}
-
 // Two independent lazy products (their multiply-add chains and reductions
 // interleave).
 __device__ __forceinline__ void mul_lazy2(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_t &r0,
@@ -369,9 +304,6 @@ __device__ __forceinline__ void mul_lazy2(uint64_t a0, uint64_t b0, uint64_t a1,
 // a * b, canonical (the lazy product's 7-instruction reduction plus the
 // 4-instruction canonical fold is shorter than reduce128's chains).
 __device__ __forceinline__ uint64_t mul(uint64_t a, uint64_t b) { return canon(mul_lazy(a, b)); }
-__device__ __forceinline__ uint64_t mul_nc(uint64_t a, uint64_t b) { return canon(mul_lazy_nc(a, b)); }
-
-__device__ __forceinline__ uint64_t sqr(uint64_t a) { return mul(a, a); }
 
 // ---- multiplication by a power of two known at compile time
 //
@@ -398,32 +330,8 @@ constexpr int clog2(uint64_t w)
     return -1;
 }
 
-// x * 2^T, lazy, for 0 <= T < 32 and any x < 2^64: the 96-bit value
-// (x << T) + (x >> (64 - T)) * 2^64.
-template <int T>
-__device__ __forceinline__ uint64_t shl_lazy(uint64_t x)
-{
-    static_assert(T >= 0 && T < 32, "shift below 32");
-    if constexpr (T == 0) return x;
-    else return reduce96_lazy(x << T, (uint32_t)(x >> (64 - T)));
-}
-
 // x * 2^32, lazy: lo(x) * 2^32 + hi(x) * 2^64 = pack(0, lo(x)) + hi(x) * EPS.
 __device__ __forceinline__ uint64_t shl32_lazy(uint64_t x) { return reduce96_lazy(pack(0u, lo32(x)), hi32(x)); }
-
-// x * 2^E mod p, canonical, for 0 <= E < 192 and any x < 2^64.
-template <int E>
-__device__ __forceinline__ uint64_t mul_pow2(uint64_t x)
-{
-    static_assert(E >= 0 && E < 192, "exponent below the order of 2");
-    constexpr int t = E % 96;
-    uint64_t r = shl_lazy<t % 32>(x);
-    if constexpr (t >= 32) r = shl32_lazy(r);
-    if constexpr (t >= 64) r = shl32_lazy(r);
-    r = canon(r);
-    if constexpr (E >= 96) r = neg(r);
-    return r;
-}
 
 // x^7 with the addition chain x2 = x^2, x3 = x*x2, x4 = x2^2, x7 = x3*x4;
 // lazy in and out (any x < 2^64; result below 2^64, congruent mod p).  x3

@@ -8,7 +8,6 @@ namespace zkx {
 constexpr int kNttTileLog = 12;  // 4096 u64 = 32 KB of LDS per work-group
 constexpr int kNttThreads = 256;
 constexpr int kNttPerThread = (1 << kNttTileLog) / kNttThreads;  // 16 elements per lane
-constexpr int kNttRadixLog = 4;                                 // stages per register round
 constexpr uint32_t kMaxRateBits = 5;                             // LDE blowup up to 32
 
 enum SrcMode : uint32_t {
