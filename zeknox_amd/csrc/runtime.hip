@@ -148,7 +148,7 @@ Tuning Device::cabi_merkle_tuning(uint64_t num_leaves, uint64_t hash_type)
 {
     std::lock_guard<std::mutex> g(tune_mu);
     Tuning t = tune_default;
-    if (!tune_default_set) t.merkle_tile_log = lone_tree_tile_log(num_leaves, hash_type);
+    if (!tune_default_set) t.merkle_tile_log = lone_tree_tile_log(num_leaves, hash_type, lone_level_leaves.load());
     return t;
 }
 

@@ -29,31 +29,6 @@ struct Tuning {
     bool by_caller = false;
 };
 
-// Work-group size (log2 lanes) of the C-ABI Merkle entry points for one tree
-// of num_leaves leaves while the caller has not set a default schedule.  A
-// tree alone has no other tree's leaves to hide the upper levels, which run
-// at low occupancy at the end of the launch, so the largest tile that still
-// gives every CU a work-group (2^lg / 2^tile >= 256) wins up to 2^18 leaves;
-// above, leaves take several rounds of work-groups and 2^9 lanes win for
-// Poseidon and Poseidon2, 2^8 for Keccak-256 and Monolith, 2^10 for Poseidon
-// over BN254 (as measured; the cause is not analysed).  Measured on one
-// MI355X, leaf launch of 135-element leaves, cap 4, tiles 2^8 / 2^9 / 2^10:
-//   Poseidon  2^16 1.07 / 1.31 / 2.09 ms, 2^17 1.51 / 1.38 / 2.12,
-//             2^18 2.65 / 2.52 / 2.41, 2^20 9.32 / 9.08 / 9.61;
-//   Keccak    2^17 0.39 / 0.33 / 0.45, 2^18 0.57 / 0.58 / 0.50,
-//             2^20 1.82 / 1.97 / 1.98 (Poseidon2, Monolith alike);
-//   BN254     2^19 178 / 181 / 145, 2^20 324 / 359 / 281.
-// In a batch other trees' leaves hide that tail and the batch default or
-// the autotuned schedule applies.  hash_type: merkle/merkle.h numbering.
-inline uint32_t lone_tree_tile_log(uint64_t num_leaves, uint64_t hash_type)
-{
-    const uint32_t lg = num_leaves ? 63u - (uint32_t)__builtin_clzll(num_leaves) : 0u;
-    if (lg <= 16) return 8;
-    if (lg <= 18) return lg - 8;
-    if (hash_type == 2) return 10;                   // Poseidon over BN254
-    return hash_type == 0 || hash_type == 3 ? 9 : 8;  // Poseidon, Poseidon2
-}
-
 // A commit shape: (columns, log2 degree, rate bits, hash type, leaf rows kept).
 using TuneKey = std::tuple<uint32_t, uint32_t, uint32_t, uint32_t, bool>;
 
@@ -114,8 +89,47 @@ inline bool lone_tree_narrow(uint64_t num_leaves, uint64_t hash_type, uint64_t m
     return has_narrow_kernel(hash_type) && num_leaves <= kNarrowLeaves &&
            !lone_tree_levels_apart(num_leaves, hash_type, min_leaves);
 }
-// The same for the forests of one hash in a batch of `batch_leaves` leaves in
-// total (default threshold 2^18; Poseidon and Poseidon2 at an eighth).
+
+// Work-group size (log2 lanes) of the C-ABI Merkle entry points for one tree of
+// num_leaves leaves while the caller has not set a default schedule.
+//
+// Levels apart: the launch hashes leaves alone, and 2^8 lanes are as fast as any
+// (135-element leaves, cap 4, one MI355X, ms, tiles 2^8 / 2^9 / 2^10: Poseidon
+// 2^17 0.883 / 0.882 / 1.305, 2^20 5.28 / 5.30 / 5.36, Poseidon2 2^20 5.65 /
+// 5.69 / 5.84, Keccak-256 2^20 1.180 / 1.198 / 1.284, Monolith 2^20 3.13 / 3.15 /
+// 3.43).  Poseidon over BN254, either side of that by size (2^17 46.1 / 46.2 /
+// 68.3, 2^18 73.8 / 76.1 / 72.5, 2^19 128 / 136 / 129, 2^20 234 / 256 / 241),
+// keeps the sizes below.
+//
+// Levels inside the launch: a tree alone has no other tree's leaves to hide
+// them, and they run at low occupancy at its end, so the largest tile that
+// still gives every CU a work-group (2^lg / 2^tile >= 256) wins up to 2^18
+// leaves.  Above, which takes a caller's threshold, leaves take several rounds
+// of work-groups and 2^9 lanes win for Poseidon and Poseidon2, 2^8 for
+// Keccak-256 and Monolith, 2^10 for Poseidon over BN254 (as measured; the
+// cause is not analysed).  The same trees, fused:
+//   Poseidon    2^16 0.79 / 0.91 / 1.39, 2^17 1.01 / 0.96 / 1.44,
+//               2^18 1.74 / 1.66 / 1.63, 2^20 6.17 / 6.07 / 6.31;
+//   Keccak-256  2^16 0.194 / 0.247 / 0.366, 2^17 0.293 / 0.269 / 0.388,
+//               2^18 0.474 / 0.474 / 0.428, 2^20 1.72 / 1.75 / 1.71
+//               (Poseidon2, Monolith alike);
+//   BN254       2^14 35.3 / 42.5 / 66.4, 2^17 55 / 49 / 72, 2^18 100 / 92 / 76,
+//               2^19 180 / 182 / 146.
+// In a batch other trees' leaves hide that tail and the batch default or
+// the autotuned schedule applies.  hash_type: merkle/merkle.h numbering.
+inline uint32_t lone_tree_tile_log(uint64_t num_leaves, uint64_t hash_type, uint64_t min_leaves)
+{
+    const uint32_t lg = num_leaves ? 63u - (uint32_t)__builtin_clzll(num_leaves) : 0u;
+    const bool bn254 = hash_type == 2;
+    if (lg <= 16 || (!bn254 && lone_tree_levels_apart(num_leaves, hash_type, min_leaves))) return 8;
+    if (lg <= 18) return lg - 8;
+    if (bn254) return 10;
+    return has_narrow_kernel(hash_type) ? 9 : 8;
+}
+
+// lone_tree_levels_apart for the forests of one hash in a batch of
+// `batch_leaves` leaves in total (default threshold 2^18; Poseidon and
+// Poseidon2 at an eighth).
 // Commits of 135 x 2^n rate 3, Poseidon, fused against apart, ms: 2^16 leaves
 // 0.93 / 0.85, 2^17 1.23 / 1.12, 2^18 2.28 / 2.00; 8 of 20 x 2^12 rate 3
 // (2^18 leaves) 0.71 / 0.55.
