@@ -55,25 +55,25 @@ MFMA_WAVE_INSTS_PER_PERM = {(8, 0): 4.3125, (9, 0): 4.3125, (10, 0): 4.3125, (9,
 #   SHA-256 (first 16 hex digits) of the leaf kernel's sources those counts
 #   were measured on (leaf_kernel_digest()); a build whose sources differ is
 #   flagged in the JSON ("counters_match_build": false)
-LEAF_COUNTERS_SOURCES = "e57c836782a8f862"
+LEAF_COUNTERS_SOURCES = "e9db8bec14b07845"
 #   issue slots (one per 4 cycles) that one such MFMA takes from the vector
 #   issue of its SIMD beside full-rate VALU work: measured live by the
 #   "issue" leg (zkx_issue_probe); this value only when that leg is skipped
-MFMA_ISSUE_SLOTS = 3.25
+MFMA_ISSUE_SLOTS = 0.3
 #   HBM bytes per commit: FETCH_SIZE x 2 (the counter reads half the bytes of
 #   a plain 1 GiB copy) + WRITE_SIZE x 1, KiB x 1024, by work-group size
-LEAF_TRAFFIC_BYTES_PER_COMMIT = {(8, 0): 7.642e8, (9, 0): 7.697e8, (10, 0): 7.779e8, (9, 1): 7.901e8}
+LEAF_TRAFFIC_BYTES_PER_COMMIT = {(8, 0): 7.625e8, (9, 0): 7.694e8, (10, 0): 7.785e8, (9, 1): 7.878e8}
 # Sources of the leaf-hash launch (zeknox_amd/csrc)
 LEAF_KERNEL_SOURCES = ("gl64.h", "gl_constants.h", "gmem.h", "hash.h", "mfma_tables.h", "poseidon_mfma.h", "merkle_kernels.h",
                        "merkle_launch.h", "merkle_launch_impl.h", "merkle_types.h", "merkle_poseidon.hip")
 #   NTT passes (both), same scaling
-NTT_TRAFFIC_BYTES_PER_COMMIT = 8.855e8
+NTT_TRAFFIC_BYTES_PER_COMMIT = 8.984e8
 #   VALU wave-instructions of the NTT launches per commit (both passes,
 #   SQ_INSTS_VALU), keyed by the LDE's pass split (stages per pass), measured
 #   on the sources NTT_COUNTERS_SOURCES
-NTT_VALU_WAVE_INSTS_PER_COMMIT = {(3, 12): 1.069e8, (4, 11): 1.065e8, (5, 10): 1.113e8, (6, 9): 1.119e8,
-                                  (7, 8): 1.131e8, (8, 7): 1.184e8}
-NTT_COUNTERS_SOURCES = "e7fd9ac3372ff032"
+NTT_VALU_WAVE_INSTS_PER_COMMIT = {(3, 12): 1.069e8, (4, 11): 1.065e8, (5, 10): 1.125e8, (6, 9): 1.130e8,
+                                  (7, 8): 1.140e8, (8, 7): 1.194e8}
+NTT_COUNTERS_SOURCES = "f609912ad21d6e5c"
 # 32-bit VALU issue peak: 256 CUs x 4 SIMDs x one wave64 instruction per 4
 # cycles x 2.4 GHz = 39.3 T lane-ops/s (MI355X's published 78.6 TFLOP/s
 # vector FP64 counts an FMA as 2 flops on the same issue rate)
@@ -688,10 +688,10 @@ def main():
     # stream); peak = VALU_PEAK_TOPS (one wave-instruction per 4 cycles).
     dom = max(batch_kernels, key=lambda k: batch_kernels[k]["ms_per_step"])
     leaf = batch_kernels.get("merkle_leaves")
-    # the batch builds its tree levels in launches of their own (the
-    # library's default for batches of >= LEVEL_LAUNCHES_DEFAULT leaves)
+    # the batch builds its tree levels in launches of their own (the library's
+    # default for Poseidon batches of >= LEVEL_LAUNCHES_DEFAULT / 8 leaves)
     levels_apart = args.merkle_schedule == "by_level" or (args.merkle_schedule == "auto"
-                                                          and args.jobs * N >= zk.LEVEL_LAUNCHES_DEFAULT)
+                                                          and args.jobs * N >= zk.LEVEL_LAUNCHES_DEFAULT >> 3)
     roofline = None
     if leaf and levels_apart and (schedule["merkle_tile_log"], schedule["merkle_valu"]) in VALU_WAVE_INSTS_PER_PERM:
         tl = (schedule["merkle_tile_log"], schedule["merkle_valu"])
@@ -719,16 +719,16 @@ def main():
                     "mfma_issue_slots_source": "measured (zkx_issue_probe)" if issue else "constant",
                     "leaf_kernel_sources": digest, "counters_match_build": digest == LEAF_COUNTERS_SOURCES}
 
-    # the tree levels: one launch per level over every tree (internal nodes
-    # and caps: N - caps permutations per commit)
+    # the tree levels in launches of their own (internal nodes and caps: N -
+    # caps permutations per commit)
     lv = batch_kernels.get("merkle_levels")
     merkle_levels = None
     if lv:
         lperms = args.jobs * (N - nc)
         merkle_levels = {"launches_per_step": lv["launches_per_step"], "ms_per_step": round(lv["ms_per_step"], 4),
                          "perms_per_step": lperms, "perms_per_s": round(lperms / (lv["ms_per_step"] * 1e-3)),
-                         "note": "one launch per level over all trees; the narrowest levels are bound by one "
-                                 "permutation's latency"}
+                         "note": "one launch per level over all trees, the narrow ones (at most 2^16 children) "
+                                 "together in one, bound by one permutation's latency each"}
 
     # LDE passes against HBM: algorithmic bytes of the LDE (read n, write N
     # per column) over the batch's NTT launches
@@ -741,12 +741,13 @@ def main():
                         "frac": round(gbs / HBM_PEAK_GBS, 3), "traffic": round(NTT_TRAFFIC_BYTES_PER_COMMIT * args.jobs),
                         "traffic_gbs": round(NTT_TRAFFIC_BYTES_PER_COMMIT * args.jobs / (ntt["ms_per_step"] * 1e-3) / 1e9, 1),
                         "kernel": "batch_ntt (all passes)",
-                        "note": "VALU-bound (64-bit modular butterflies), not HBM-bound"}
+                        "note": "bound by the memory passes: their loads and stores alone take most of the time, "
+                                "and the VALU issue of the same launches (valu_issue) is below its peak"}
         split = tuple(zk.ntt_pass_sizes(LG_N, zk.get_tuning(commits[0])))
         ntt_valu = NTT_VALU_WAVE_INSTS_PER_COMMIT.get(split)
         ntt_roofline["pass_split"] = list(split)
         if ntt_valu:
-            # the bound that holds: VALU issue of the same launches
+            # VALU issue of the same launches
             valu = ntt_valu * args.jobs * 64 / (ntt["ms_per_step"] * 1e-3) / 1e12
             digest = leaf_kernel_digest(NTT_KERNEL_SOURCES)
             ntt_roofline["valu_issue"] = {"achieved": round(valu, 2), "peak": round(VALU_PEAK_TOPS, 2),

@@ -141,9 +141,9 @@ void Engine::commit(const CommitJob *jobs, size_t n, void *scratch, const Tuning
     }
 
     // ---- Merkle schedule: batches whose trees hold many leaves build the
-    // levels above the leaves with one launch per level over every tree
-    // (after a leaf launch that writes the leaf digests only); smaller ones
-    // finish every tree inside its hash kind's leaf launch
+    // levels above the leaves in launches of their own over every tree (after
+    // a leaf launch that writes the leaf digests only); smaller ones finish
+    // every tree inside its hash kind's leaf launch
     uint64_t tree_leaves = 0;
     for (size_t i = 0; i < n; i++)
         if (jobs[i].cap_height < jobs[i].lg_n + jobs[i].rate) tree_leaves += 1ull << (jobs[i].lg_n + jobs[i].rate);

@@ -9,8 +9,8 @@
 //
 // Schedule.  A work-group of TPB (256..1024) lanes owns a tile of consecutive
 // leaves.  Each lane hashes its leaf, then the tile is reduced level by level
-// in LDS (Poseidon and Poseidon2 on lane pairs, two lanes per node, since a
-// level is one permutation deep and runs at low occupancy): every level's
+// in LDS (Poseidon, Poseidon2 and Keccak-256 on lane pairs, two lanes per node,
+// since a level is one permutation deep and runs at low occupancy): every level's
 // digests are written to HBM on the way up, and a tile
 // that reaches the width-2 top level of its subtree also writes the cap.  A
 // tile that stops below the top leaves its root for an upper pass (a tile of
@@ -341,9 +341,9 @@ k_merkle_tile(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs on
 // the OUTPUT level here (width 2^lg_w per subtree; 0: the caps), count its
 // nodes over all subtrees, tile_begin its first work-group; node g =
 // hash_two of the 8 consecutive words of its two children at level lg_w + 1.
-// Poseidon hashes 64 nodes per wave on the matrix cores (the state [l, r, 0]
-// laid out as leaf_hash_mfma lays out a leaf's first chunk), the other hashes
-// one node per lane.  njobs == 0: the single descriptor `one` (a lone tree).
+// Poseidon and Poseidon2 hash 64 nodes per wave on the matrix cores (the state
+// [l, r, 0] laid out as leaf_hash_mfma lays out a leaf's first chunk), the other
+// hashes one node per lane.  njobs == 0: the single descriptor `one` (a lone tree).
 template <int HT>
 __global__ void __launch_bounds__(kMerkleLevelLanes) __attribute__((amdgpu_waves_per_eu(merkle_waves_per_eu(HT))))
 k_merkle_level(const MerkleArgs *__restrict__ jobs, uint32_t njobs, MerkleArgs one, uint32_t block0)

@@ -344,7 +344,8 @@ k_ntt_tiles(const NttPass *__restrict__ passes, uint32_t npasses, NttPass one, u
 // w_4096^(that << (3 - dd)) from the global table (16 KB of it in use).  So
 // those stages run on the loaded registers and only the stages below 8 go
 // through LDS (two register rounds, the last with its small roots as
-// shifts).  Four work-groups per CU.  This replaced a
+// shifts).  Four work-groups per CU: at 128 VGPRs the rounds spill 20 of them
+// (48 bytes a lane).  This replaced a
 // persistent kernel that prefetched the next tile and staged the stage
 // twiddles in LDS (three waves per SIMD, 164-168 VGPRs): batched LDE NTT
 // 5.13 -> 4.75 ms per 16 commits, the plain 12-stage pass 0.216 -> 0.198 ms,

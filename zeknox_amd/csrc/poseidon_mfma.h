@@ -45,9 +45,10 @@
 // limb_combine(L, H) (0 <= L, H < 2^47).  The chains run in signed 32x32+64
 // multiply-adds.
 //
-// (Accumulator chains stay within one opcode, in place: a 16x16x64 result
-// taken as the accumulator of a 16x16x32 product, issued with no wait states
-// between them, came out wrong.)
+// (Accumulator chains stay within one opcode, in place.  Observed: a 16x16x64
+// result taken as the accumulator of a 16x16x32 product, issued with no wait
+// states between them, came out wrong; why is not established, and no kernel
+// does it.)
 #pragma once
 #include "hash.h"
 #include "mfma_tables.h"
@@ -130,11 +131,13 @@ __device__ __forceinline__ mf_v4i mfma_pair(uint64_t x0, uint64_t x1)
 __device__ __forceinline__ uint32_t digit_pair(int d0, int d1) { return (uint32_t)d0 + ((uint32_t)d1 << 8); }
 
 // Keeps the operands of an MFMA chain in their registers until p, computed
-// from the chain's result, is there.  A register of a chain's A operand
-// overwritten by a v_mov right after the MFMA that reads it gave wrong sums
-// whenever another wave held the SIMD's matrix pipe (the second group of a
-// wave, at two or more waves per SIMD): the compiler lets go of the operands
-// as soon as the instruction is issued, and it reads them later than that.
+// from the chain's result, is there.  Observed: without it, where the compiler
+// put a v_mov over a register of a chain's A operand right after the MFMA that
+// reads it, the sums came out wrong with two or more waves on the SIMD (in the
+// second group of a wave), and right with it.  The cause is not established:
+// the documented waits after an MFMA cover its accumulator, not A and B, and
+// the compiler counts none for them.  Every chain holds its operands, so no
+// kernel depends on the answer.
 template <int NK>
 __device__ __forceinline__ void hold_operands(const mf_v4i (&a)[NK], const mf_v4i (&b)[NK], uint32_t p)
 {
@@ -142,7 +145,9 @@ __device__ __forceinline__ void hold_operands(const mf_v4i (&a)[NK], const mf_v4
     for (int kappa = 0; kappa < NK; kappa++) asm volatile("; hold %0 %1 %2" ::"v"(p), "v"(a[kappa]), "v"(b[kappa]));
 }
 
-// limb_combine for B < 2^48, less the EPS of the lanes of `carry`.
+// limb_combine (any A and B with B + hi(A) below 2^64; the sums here are below
+// 2^63), less the EPS of the lanes of `carry`, which are the rarer the smaller
+// B is: about one value in 2^64 / B.
 __device__ __forceinline__ uint64_t limb_combine_rare(uint64_t A, uint64_t B, uint64_t &carry)
 {
     const uint64_t T = gl::add_small(B, gl::hi32(A));

@@ -129,9 +129,9 @@ struct Device {
     std::atomic<bool> commit_graphs{true};
     // Batches whose trees hold at least this many leaves in total build the
     // levels above the leaves in launches of their own over all trees
-    // (zkx_set_level_launches, batch_levels_apart); smaller ones, one fused
-    // launch per hash kind.  Keccak-256 and Monolith, 1-16 commits: by level
-    // 0.93-0.99 of the fused time from 2^18 leaves up, 1.14-1.16 below.
+    // (zkx_set_level_launches; the rules by hash and their measurements:
+    // batch_levels_apart and batch_narrow); smaller ones, one fused launch per
+    // hash kind.
     std::atomic<uint64_t> level_launch_leaves{1ull << 18};
     // The same for one tree through the C-ABI Merkle entry points
     // (zkx_set_lone_level_launches, lone_tree_levels_apart).

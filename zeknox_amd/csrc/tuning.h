@@ -62,21 +62,21 @@ constexpr bool has_tile_top(uint64_t hash_type) { return hash_type == 1; }
 // and Monolith at min_leaves / 4, Poseidon-BN128 at min_leaves / 32 (0:
 // always).  Measured, fused against apart, 135-element leaves, cap 4, ms:
 //   leaves  Poseidon      Poseidon2     Keccak-256     Monolith       Poseidon-BN128
-//   2^15                                0.215 / 0.219  0.540 / 0.533  36.2 / 33.5
-//   2^16                  0.92 / 0.76   0.225 / 0.234
-//   2^17                  1.11 / 0.96   0.299 / 0.295  0.695 / 0.697  48.5 / 46.2
-//   2^18    1.74 / 1.53   1.86 / 1.65         / 0.423  1.078 / 1.056  75.3 / 72.8
-//   2^19                  3.66 / 3.25         / 0.688  2.069 / 1.760
-//   2^20    6.36 / 5.67   7.01 / 6.02         / 1.179  3.639 / 3.143
-// (Keccak-256 above 2^17 before its lane pairs and top of tiles: 0.503 / 0.485,
-// 1.095 / 0.779, 1.928 / 1.344.)
+//   2^13    0.324 / 0.639 0.362 / 0.679 0.164 / 0.166  0.490 / 0.479  33.6 / 31.1
+//   2^15    0.449 / 0.679 0.498 / 0.725 0.185 / 0.189  0.540 / 0.534  36.6 / 33.6
+//   2^16    0.792 / 0.717 0.917 / 0.767 0.194 / 0.200  0.556 / 0.555  38.4 / 35.3
+//   2^17    0.957 / 0.882 1.083 / 0.941 0.270 / 0.265  0.698 / 0.699  49.4 / 46.5
+//   2^18    1.62 / 1.48   1.77 / 1.58   0.429 / 0.394  1.078 / 1.060  75.9 / 72.6
+//   2^19    3.13 / 2.84   3.50 / 3.00   0.931 / 0.661  2.071 / 1.763  146 / 129
+//   2^20    6.13 / 5.32   6.74 / 5.70   1.720 / 1.160  3.645 / 3.148
+// (Poseidon and Poseidon2 up to 2^15 against the 16-per-wave kernel.)
 // Poseidon's and Poseidon2's narrow levels cost 12 us each in the 16-per-wave
 // kernel against 25-36 us on lane pairs and rows inside the leaf launch, so
 // every tree that is not built whole by that kernel gains.  Keccak's and
 // Monolith's permutations are short, so what their fused trees' lower levels
-// lose on ever fewer lanes weighs more;
-// Poseidon-BN128's levels are slow enough that a full-GPU launch per level
-// pays at every size measured.
+// lose on ever fewer lanes weighs more (their line is left where both sides
+// are within 2%).  Poseidon-BN128's levels are slow enough that a full-GPU
+// launch per level pays at every size measured.
 inline bool lone_tree_levels_apart(uint64_t num_leaves, uint64_t hash_type, uint64_t min_leaves)
 {
     const uint32_t shift = hash_type == 2 ? 5 : has_narrow_kernel(hash_type) ? 4 : 2;
@@ -130,9 +130,12 @@ inline uint32_t lone_tree_tile_log(uint64_t num_leaves, uint64_t hash_type, uint
 // lone_tree_levels_apart for the forests of one hash in a batch of
 // `batch_leaves` leaves in total (default threshold 2^18; Poseidon and
 // Poseidon2 at an eighth).
-// Commits of 135 x 2^n rate 3, Poseidon, fused against apart, ms: 2^16 leaves
-// 0.93 / 0.85, 2^17 1.23 / 1.12, 2^18 2.28 / 2.00; 8 of 20 x 2^12 rate 3
-// (2^18 leaves) 0.71 / 0.55.
+// One commit of 135 x 2^13 / 2^14 / 2^15 rate 3 (2^16, 2^17, 2^18 leaves), and
+// eight of 20 x 2^12 rate 3 (2^18 leaves), fused against apart, ms:
+//   Poseidon    0.877 / 0.808   1.174 / 1.054   2.08 / 1.82   0.703 / 0.524
+//   Poseidon2   1.004 / 0.858   1.347 / 1.120   2.38 / 2.00   0.806 / 0.572
+//   Keccak-256  0.298 / 0.302   0.470 / 0.470   1.15 / 1.06   0.326 / 0.293
+//   Monolith    0.658 / 0.660   0.940 / 0.892   1.61 / 1.44   0.523 / 0.472
 inline bool batch_levels_apart(uint64_t batch_leaves, uint64_t hash_type, uint64_t min_leaves)
 {
     return batch_leaves > 0 && batch_leaves >= (has_narrow_kernel(hash_type) ? min_leaves >> 3 : min_leaves);
