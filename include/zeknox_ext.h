@@ -209,8 +209,8 @@ int zkx_merkle_plan(uint64_t nl, uint64_t nc, uint32_t tile_log, uint64_t *count
                     uint32_t *tile_logs, uint32_t *first_ctr, int cap, uint64_t *counters);
 /* Forget every shape entry and restore the built-in default. */
 RustError zkx_tuning_clear(size_t device_id);
-/* The shape table as text, one shape per line (with a mark on those that
- * zkx_set_tuning set). */
+/* The shape table as text, one shape per line, with a mark on those that
+ * zkx_set_tuning set (lines without it load as autotuned ones). */
 RustError zkx_tuning_save(size_t device_id, const char *path);
 RustError zkx_tuning_load(size_t device_id, const char *path);
 

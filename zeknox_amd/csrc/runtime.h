@@ -82,7 +82,7 @@ struct Device {
     // A transform holds spare_mu until its launches on `stream` are queued;
     // given back by zkx_commit_trim and by an allocation that finds no memory
     // left, which both wait for the device.  Taken last: whoever holds it
-    // allocates nothing else and takes no other lock.
+    // allocates nothing else and takes no other lock of a device or engine.
     std::mutex spare_mu;
     SpareMemory ntt_scratch{device_alloc_spare, device_free};
     bool drop_spare();
